@@ -2,7 +2,8 @@
 // kernels/whisper.cu:168-299 (enc_flash). softmax(Q K^T / 8) V with fp32 scores and online softmax, P rounded to
 // fp16 for the P.V product, O / l rounded to fp16 (the SDPA arithmetic the reference follows, whisper.cu:3-4).
 //
-// Work: one block per (256 queries, head, clip) = 4 waves x 2 sets of 32 queries. K and V^T tiles of 64 keys are
+// Work: one block per (256 queries, head, clip) = 4 waves x 2 sets of 32 queries, or per 128 queries with one set per
+// wave where that spreads few (clip, head) pairs better over the CUs (mz_enc_attention_launch). K and V^T tiles of 64 keys are
 // staged in LDS (double buffered, register prefetch) and shared by the 4 waves. Scores are computed transposed,
 // S^T = K Q^T (32x32x16 MFMA), so each lane owns one query column: the running max and the rescale of O are per
 // lane, and the only cross-lane step is one swap with lane l ^ 32. K rows are stored in LDS with bits 2 and 3 of the
@@ -24,7 +25,6 @@
 namespace {
 
 constexpr int KP = 72;  // LDS row pitch in halves (144 B): conflict-free 16-byte fragment reads
-constexpr int QB = 256; // queries per block
 constexpr int NT = MZ_TPAD / 64;  // key tiles (the last one holds keys 1472..1535, valid < 1500)
 
 __device__ __forceinline__ int swap23(int x) { return (x & ~12) | ((x & 4) << 1) | ((x & 8) >> 1); }
@@ -54,14 +54,18 @@ __device__ __forceinline__ float probs(const f32x16& sc, unsigned (&pw)[2][4]) {
     return lb;
 }
 
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) enc_attn_kernel(const f16* __restrict__ qkvh, f16* __restrict__ out, int nh, int G) {
+// NS query sets of 32 per wave, NW waves: 32 NS NW queries per block
+template <int NS, int NW>
+__global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
+enc_attn_kernel(const f16* __restrict__ qkvh, f16* __restrict__ out, int nh, int G) {
     __shared__ __attribute__((aligned(16))) f16 sK[2][64 * KP];
     __shared__ __attribute__((aligned(16))) f16 sV[2][64 * KP];
 
-    // workgroup i runs on XCD i % 8: XCD x takes (clip, head) pairs x, x + 8, ... and all six query blocks of a pair,
-    // so a pair's K and V tiles are fetched into one L2 only
-    const int xcd = blockIdx.x & 7, li = blockIdx.x >> 3, npq = (MZ_TENC + QB - 1) / QB;
-    const int pair = (li / npq) * 8 + xcd, qb = li % npq;
+    // workgroup i runs on XCD i % 8: XCD x takes the x-th eighth of the query blocks in (clip, head) order, so that a
+    // pair's K and V tiles are fetched into one L2 (two for the pairs at a border) and no XCD holds more blocks than
+    // another
+    constexpr int QB = 32 * NS * NW, npq = (MZ_TENC + QB - 1) / QB;
+    const int idx = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3), pair = idx / npq, qb = idx % npq;
     if (pair >= nh * G) return;
     const int head = pair % nh, g = pair / nh;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, lr = lane & 31, lh = lane >> 5;
@@ -73,43 +77,48 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 
     // query fragments (B operand of S^T): query row, dims 16c + 8 lh .. + 8; the QKV product stores q multiplied by
     // log2(e) / 8, so the products are the scores in log2 units
-    const int q0 = qb * QB + wave * 64;
-    f16x8 qf[2][4];
+    const int q0 = qb * QB + wave * (32 * NS);
+    f16x8 qf[NS][4];
 #pragma unroll
-    for (int s = 0; s < 2; s++)
+    for (int s = 0; s < NS; s++)
 #pragma unroll
         for (int c = 0; c < 4; c++) qf[s][c] = ld8(Q + (long)(q0 + s * 32 + lr) * MZ_HD + 16 * c + 8 * lh);
 
-    // this thread's two K chunks and two V^T chunks of a tile: buffer loads with a fixed per-lane offset and the tile
-    // step in the scalar offset (no address arithmetic per tile; every offset lies within the padded head block)
-    const int c0 = tid, c1 = tid + 256;
-    const int kr0 = c0 >> 3, kr1 = c1 >> 3, cc = (tid & 7) * 8;
+    // this thread's NCH K chunks and V^T chunks of a tile (chunk tid + 64 NW i: row i (8 NW) + tid / 8): buffer loads
+    // with a fixed per-lane offset and the tile step in the scalar offset (no address arithmetic per tile; every
+    // offset lies within the padded head block)
+    constexpr int NCH = 8 / NW, RS = 8 * NW;
+    const int kr = tid >> 3, cc = (tid & 7) * 8;
     const __amdgpu_buffer_rsrc_t rK = rsrc(K, MZ_TPAD * MZ_HD * 2), rV = rsrc(Vt, MZ_HD * MZ_TPAD * 2);
-    const unsigned ok0 = (kr0 * MZ_HD + cc) * 2, ok1 = (kr1 * MZ_HD + cc) * 2;
-    const unsigned ov0 = (kr0 * MZ_TPAD + cc) * 2, ov1 = (kr1 * MZ_TPAD + cc) * 2;
-    f16x8 pk0, pk1, pv0, pv1;
+    f16x8 pk[NCH], pv[NCH];
     auto gload = [&](int kt) {
         const int sk = kt * 64 * MZ_HD * 2, sv = kt * 64 * 2;
-        pk0 = __builtin_bit_cast(f16x8, __builtin_amdgcn_raw_buffer_load_b128(rK, ok0, sk, 0));
-        pk1 = __builtin_bit_cast(f16x8, __builtin_amdgcn_raw_buffer_load_b128(rK, ok1, sk, 0));
-        pv0 = __builtin_bit_cast(f16x8, __builtin_amdgcn_raw_buffer_load_b128(rV, ov0, sv, 0));
-        pv1 = __builtin_bit_cast(f16x8, __builtin_amdgcn_raw_buffer_load_b128(rV, ov1, sv, 0));
+#pragma unroll
+        for (int i = 0; i < NCH; i++)
+            pk[i] = __builtin_bit_cast(
+                f16x8, __builtin_amdgcn_raw_buffer_load_b128(rK, (unsigned)(((kr + RS * i) * MZ_HD + cc) * 2), sk, 0));
+#pragma unroll
+        for (int i = 0; i < NCH; i++)
+            pv[i] = __builtin_bit_cast(
+                f16x8, __builtin_amdgcn_raw_buffer_load_b128(rV, (unsigned)(((kr + RS * i) * MZ_TPAD + cc) * 2), sv, 0));
     };
     auto lstore = [&](int buf) {
-        *(f16x8*)&sK[buf][swap23(kr0) * KP + cc] = pk0;
-        *(f16x8*)&sK[buf][swap23(kr1) * KP + cc] = pk1;
-        *(f16x8*)&sV[buf][kr0 * KP + cc] = pv0;
-        *(f16x8*)&sV[buf][kr1 * KP + cc] = pv1;
+#pragma unroll
+        for (int i = 0; i < NCH; i++) {
+            *(f16x8*)&sK[buf][swap23(kr + RS * i) * KP + cc] = pk[i];
+            *(f16x8*)&sV[buf][(kr + RS * i) * KP + cc] = pv[i];
+        }
     };
 
     // running max of the scores (per query column), set by the first block, kept as -m in all 16 elements of the C
     // input of each block's first product: the scores come out of the matrix core relative to it
-    float m[2] = {0.f, 0.f};
-    f32x16 cm[2] = {f32x16{}, f32x16{}};
-    float l[2] = {0.f, 0.f};
-    f32x16 o[2][2];
+    float m[NS], l[NS];
+    f32x16 cm[NS], o[NS][2];
 #pragma unroll
-    for (int s = 0; s < 2; s++) o[s][0] = o[s][1] = f32x16{};
+    for (int s = 0; s < NS; s++) {
+        m[s] = l[s] = 0.f;
+        cm[s] = o[s][0] = o[s][1] = f32x16{};
+    }
 
     gload(0);
     lstore(0);
@@ -130,7 +139,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
                 for (int c = 0; c < 2; c++)
                     vf[t][c] = *(const f16x8*)&sV[buf][(32 * t + lr) * KP + 32 * ss + 16 * c + 8 * lh];
 #pragma unroll
-            for (int qs = 0; qs < 2; qs++) {
+            for (int qs = 0; qs < NS; qs++) {
                 f32x16 sc = mfma32(kf[0], qf[qs][0], cm[qs]);
 #pragma unroll
                 for (int c = 1; c < 4; c++) sc = mfma32(kf[c], qf[qs][c], sc);
@@ -189,7 +198,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
     tile(NT - 1, std::true_type{});
 
 #pragma unroll
-    for (int qs = 0; qs < 2; qs++) {
+    for (int qs = 0; qs < NS; qs++) {
         const float lt = pair32_sum(l[qs]);
         const float inv = 1.f / lt;
         const int q = q0 + qs * 32 + lr;
@@ -206,12 +215,24 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
     }
 }
 
+template <int NS, int NW>
+hipError_t launch(hipStream_t s, const f16* qkvh, f16* out, int G, int nh) {
+    // 1-D grid: 8 XCDs x an eighth of the query blocks, rounded up
+    constexpr int QB = 32 * NS * NW, npq = (MZ_TENC + QB - 1) / QB;
+    hipLaunchKernelGGL((enc_attn_kernel<NS, NW>), dim3(8 * ((G * nh * npq + 7) / 8)), dim3(64 * NW), 0, s, qkvh, out, nh, G);
+    return hipGetLastError();
+}
+
 }  // namespace
 
 hipError_t mz_enc_attention_launch(hipStream_t s, const f16* qkvh, f16* out, int G, int nh) {
     if (G <= 0 || nh <= 0) return hipErrorInvalidValue;
-    // 1-D grid: 8 XCDs x ceil(pairs / 8) pairs x 6 query blocks
-    const int npq = (MZ_TENC + QB - 1) / QB, pairs = G * nh;
-    hipLaunchKernelGGL(enc_attn_kernel, dim3(8 * ((pairs + 7) / 8) * npq), dim3(256), 0, s, qkvh, out, nh, G);
-    return hipGetLastError();
+    // The time goes by the blocks that the fullest CU holds. Blocks of 128 queries (one set per wave), k per CU: 20, 31,
+    // 48, 63, 78, 93, 108, 126 us for k = 1 .. 8; blocks of 256 (two sets, fewer fragment reads per product): 32, 56,
+    // 84, 111 us for 1 .. 4 (1 to 160 pairs). So the small blocks are taken where they fill a CU to an odd count, which
+    // the large ones would round up (1 x 20 heads 31.6 -> 20.4 us, 3 x 20 56.4 -> 50.4), and for two per CU (35.6 ->
+    // 33.4); beyond 7 the large ones win either way (16 x 20 220 vs 231). Both give the same bits.
+    const int k = (G * nh * ((MZ_TENC + 127) / 128) + mz_cu_count() - 1) / mz_cu_count();
+    if (k == 2 || (k <= 7 && k % 2 == 1)) return launch<1, 4>(s, qkvh, out, G, nh);
+    return launch<2, 4>(s, qkvh, out, G, nh);
 }

@@ -400,24 +400,11 @@ __global__ void __launch_bounds__(NW * 64) gemm_kernel(const MzGemm p) {
 #endif
 }
 
-// compute units of the current device (workgroups of a persistent grid: one per CU), a multiple of 8
-int cu_groups() {
-    static int cached[64] = {};
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-    if (!cached[dev]) {
-        int n = 0;
-        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n < 8) n = 256;
-        cached[dev] = n / 8 * 8;
-    }
-    return cached[dev];
-}
-
 template <int BM, int BN, int ALOAD, int EPI>
 hipError_t launch(hipStream_t s, const MzGemm& g) {
     const int nbm = (g.M + BM - 1) / BM, nbn = (g.N + BN - 1) / BN;
     const int nvirt = 8 * ((nbm + 7) / 8) * nbn;
-    const int cus = cu_groups(), grid = ALOAD == ALOAD_PLAIN && nvirt > cus ? cus : nvirt;
+    const int cus = mz_cu_count(), grid = ALOAD == ALOAD_PLAIN && nvirt > cus ? cus : nvirt;
     hipLaunchKernelGGL((gemm_kernel<BM, BN, ALOAD, EPI>), dim3(grid), dim3(NW * 64), 0, s, g);
     return hipGetLastError();
 }
@@ -433,6 +420,19 @@ hipError_t pick(hipStream_t s, const MzGemm& g) {
 }
 
 }  // namespace
+
+// compute units of the current device rounded down to a multiple of 8 (workgroups of a persistent grid: one per CU)
+int mz_cu_count() {
+    static int cached[64] = {};
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+    if (!cached[dev]) {
+        int n = 0;
+        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n < 8) n = 256;
+        cached[dev] = n / 8 * 8;
+    }
+    return cached[dev];
+}
 
 hipError_t mz_gemm_launch(hipStream_t s, int aload, int epi, const MzGemm& g) {
     if (g.K % 64 != 0 || g.M <= 0 || g.N <= 0 || g.K <= 0 || g.N % 4 != 0) return hipErrorInvalidValue;

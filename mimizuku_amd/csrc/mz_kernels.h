@@ -38,6 +38,8 @@ struct MzGemm {
     int blocks_per_clip, nh, kind, slot0;
 };
 hipError_t mz_gemm_launch(hipStream_t s, int aload, int epi, const MzGemm& g);
+// compute units of the current device, rounded down to a multiple of 8
+int mz_cu_count();
 
 // ---------------------------------------------------------------- encoder attention
 // qkvh: [G][3][nh] tiles of 1536 x 64 halves (q, k row-major [t][64]; v transposed [64][t]; t >= 1500 zero);

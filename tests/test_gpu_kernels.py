@@ -146,6 +146,23 @@ def test_enc_attention_late_peak(ctx):
     assert rel_err(out, np.broadcast_to(v[:, :, 1490:1491].astype(np.float64), out.shape)) < 0.05
 
 
+@pytest.mark.parametrize("shape", [(1, 21), (2, 11), (3, 14), (7, 10), (5, 18), (6, 20)])
+def test_enc_attention_block_sizes(ctx, shape):
+    """Pair counts on both sides of every border between blocks of 128 and of 256 queries (one block per CU and more):
+    the same bits as each pair alone, peaks past the running max among them (so the recomputed blocks too), and the
+    float64 attention on some rows."""
+    rng = np.random.default_rng(sum(shape))
+    q, k, v = (f16(rng, (*shape, 1500, 64), s) for s in (2.0, 2.0, 1.0))
+    qs, q = prescaled(q)
+    out = run_attention(ctx, qs, k, v)
+    rows = np.r_[np.arange(0, 1500, 131), 1408, 1499]
+    for g, h in ((0, 0), (shape[0] // 2, shape[1] // 3), (shape[0] - 1, shape[1] - 1)):
+        one = np.s_[g:g + 1, h:h + 1]
+        np.testing.assert_array_equal(run_attention(ctx, qs[one], k[one], v[one]), out[one])
+        ref = attention64(q[one][:, :, rows], k[one], v[one])
+        assert rel_err(out[one][:, :, rows], ref) < attention_bar(q[one][:, :, rows], k[one], v[one], ref)
+
+
 def test_enc_attention_large_v3_shape(ctx):
     """8 clips x 20 heads x 1500 x 1500, head 64 (the encoder group's attention); every (clip, head) checked on 48
     query rows spread over the window, including the last ones of the padded tile."""
