@@ -29,8 +29,17 @@ constexpr unsigned OOB = 0x80000000u;  // a buffer offset past every operand: th
 // Workgroup i runs on XCD i % 8, and each XCD has its own L2. XCD x owns a band of rows = ceil(nbm / 8) block rows
 // and visits its tiles with the block row fastest: the band's activation panels stay in its L2 while each weight
 // panel is read once per XCD and shared by the band's tiles that run at the same time. The grid is 8 * rows * nbn.
-__device__ __forceinline__ bool xcd_tile(int bid, int nbm, int nbn, int* bm, int* bn) {
+// With share > 0 (launch() says when) XCD x takes tiles x * share .. of the same order instead, an eighth of them, and
+// the grid is 8 * share.
+__device__ __forceinline__ bool xcd_tile(int bid, int nbm, int nbn, int share, int* bm, int* bn) {
     const int rows = (nbm + 7) >> 3, li = bid >> 3;
+    if (share > 0) {
+        const int idx = (bid & 7) * share + li, band = idx / (rows * nbn), r = idx - band * rows * nbn;
+        const int rb = max(min(rows, nbm - band * rows), 1);  // rows of this band (the last one may be short)
+        *bm = band * rows + r % rb;
+        *bn = r / rb;
+        return idx < nbm * nbn;
+    }
     *bm = (bid & 7) * rows + li % rows;
     *bn = li / rows;
     return *bm < nbm && *bn < nbn;
@@ -53,9 +62,9 @@ __global__ void __launch_bounds__(NW * 64) gemm_kernel(const MzGemm p) {
     // and the next tile's first K tile is requested before this tile's epilogue runs, so its round trip and the
     // workgroup's dispatch are not paid once per tile. The convolution takes one tile per workgroup.
     constexpr bool PERSIST = ALOAD == ALOAD_PLAIN;
-    const int nvirt = 8 * ((nbm + 7) >> 3) * nbn, vstep = PERSIST ? (int)gridDim.x : nvirt;
+    const int nvirt = 8 * (p.share > 0 ? p.share : ((nbm + 7) >> 3) * nbn), vstep = PERSIST ? (int)gridDim.x : nvirt;
     int v = blockIdx.x, bm = 0, bn = 0;
-    while (v < nvirt && !xcd_tile(v, nbm, nbn, &bm, &bn)) v += vstep;
+    while (v < nvirt && !xcd_tile(v, nbm, nbn, p.share, &bm, &bn)) v += vstep;
     if (v >= nvirt) return;
     // the wave index through readfirstlane: wave-uniform values (tile origins, store descriptors) stay scalar
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -367,7 +376,7 @@ __global__ void __launch_bounds__(NW * 64) gemm_kernel(const MzGemm p) {
         if (kt < nk) tile(kt, sA0, sW0, sA1, sW1);
         const int m0 = bm * BM + wm * WM, n0c = n0;
         int vn = v + vstep, bmn = 0, bnn = 0;
-        while (vn < nvirt && !xcd_tile(vn, nbm, nbn, &bmn, &bnn)) vn += vstep;
+        while (vn < nvirt && !xcd_tile(vn, nbm, nbn, p.share, &bmn, &bnn)) vn += vstep;
         const bool more = PERSIST && vn < nvirt;
         f16 bias_n[TN];
         if (more) {  // the next tile's biases and first K tile, in flight during this epilogue
@@ -402,10 +411,16 @@ __global__ void __launch_bounds__(NW * 64) gemm_kernel(const MzGemm p) {
 
 template <int BM, int BN, int ALOAD, int EPI>
 hipError_t launch(hipStream_t s, const MzGemm& g) {
-    const int nbm = (g.M + BM - 1) / BM, nbn = (g.N + BN - 1) / BN;
-    const int nvirt = 8 * ((nbm + 7) / 8) * nbn;
-    const int cus = mz_cu_count(), grid = ALOAD == ALOAD_PLAIN && nvirt > cus ? cus : nvirt;
-    hipLaunchKernelGGL((gemm_kernel<BM, BN, ALOAD, EPI>), dim3(grid), dim3(NW * 64), 0, s, g);
+    const int nbm = (g.M + BM - 1) / BM, nbn = (g.N + BN - 1) / BN, cus = mz_cu_count();
+    // An XCD takes whole bands unless equal shares of the tiles save it a round of its CUs: 12 or 18 block rows (one
+    // clip in 128-row, three in 256-row blocks) are six bands, which left two XCDs without work (encoder pass of one
+    // clip, width 1280: 611 -> 530 us; three clips, width 768: 520 -> 460). Where the rounds are the same, the bands
+    // keep an XCD's panels together (8 clips, width 1280: 1562 us, against 1594 with equal shares).
+    const int band = ((nbm + 7) / 8) * nbn, even = (nbm * nbn + 7) / 8, per = cus / 8;
+    MzGemm p = g;
+    p.share = (even + per - 1) / per < (band + per - 1) / per ? even : 0;
+    const int nvirt = 8 * (p.share ? even : band), grid = ALOAD == ALOAD_PLAIN && nvirt > cus ? cus : nvirt;
+    hipLaunchKernelGGL((gemm_kernel<BM, BN, ALOAD, EPI>), dim3(grid), dim3(NW * 64), 0, s, p);
     return hipGetLastError();
 }
 

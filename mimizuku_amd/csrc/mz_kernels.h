@@ -36,6 +36,7 @@ struct MzGemm {
     // every tile row-major [1536][64]).
     f16* heads;
     int blocks_per_clip, nh, kind, slot0;
+    int share;  // set by the launcher: tiles of one XCD when all take equal shares, else 0
 };
 hipError_t mz_gemm_launch(hipStream_t s, int aload, int epi, const MzGemm& g);
 // compute units of the current device, rounded down to a multiple of 8
