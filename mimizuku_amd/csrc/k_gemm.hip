@@ -3,7 +3,8 @@
 // implicit GEMM (no im2col buffer), and the cross-attention K/V of every decoder layer. Replaces the reference's
 // cuBLAS calls with a bias prefill (src/gpu.rs:208-236, 254-286; kernels/whisper.cu:92-104, 106-139).
 //
-// Block tile BM x BN x 64 with 8 waves in a 2 x 4 grid (two waves per SIMD, so one wave's LDS reads overlap the
+// Two kernels, chosen by how many tiles a product has (pick): gemm_ring_kernel for few, described there, and for the rest
+// gemm_kernel: block tile BM x BN x 64 with 8 waves in a 2 x 4 grid (two waves per SIMD, so one wave's LDS reads overlap the
 // other's products); each wave owns a (BM/2) x (BN/4) tile of 32x32x16 MFMA products. Both operands are
 // K-contiguous and go from global memory straight into LDS (buffer_load ... lds, 16 bytes per lane, no register
 // staging), double buffered: the loads of K tile k + 1 are in flight while tile k is multiplied, with one barrier per
@@ -26,6 +27,9 @@ typedef __attribute__((address_space(3))) void lds_void;
 #define LDSP(p) ((lds_void*)(p))
 constexpr unsigned OOB = 0x80000000u;  // a buffer offset past every operand: the load returns zeros
 
+// s_waitcnt operand: at most n vector memory operations of this wave outstanding (n < 64) and no LDS operation
+constexpr int vm_lgkm_wait(int n) { return (n & 15) | ((n >> 4) << 14) | (7 << 4); }
+
 // Workgroup i runs on XCD i % 8, and each XCD has its own L2. XCD x owns a band of rows = ceil(nbm / 8) block rows
 // and visits its tiles with the block row fastest: the band's activation panels stay in its L2 while each weight
 // panel is read once per XCD and shared by the band's tiles that run at the same time. The grid is 8 * rows * nbn.
@@ -45,175 +49,57 @@ __device__ __forceinline__ bool xcd_tile(int bid, int nbm, int nbn, int share, i
     return *bm < nbm && *bn < nbn;
 }
 
-template <int BM, int BN, int ALOAD, int EPI>
-__global__ void __launch_bounds__(NW * 64) gemm_kernel(const MzGemm p) {
-#if defined(__HIP_DEVICE_COMPILE__)  // the buffer-resource type exists only in the device pass
-    constexpr int WM = BM / 2, WN = BN / 4, TM = WM / 32, TN = WN / 32;
-    constexpr int AR = BM / (8 * NW), WR = BN / (8 * NW);  // 8-row slices each wave loads per K tile
-    static_assert(AR >= 1 && WR >= 1 && TN >= 1, "tile too small for 8 waves");
-    __shared__ __attribute__((aligned(16))) f16 sA0[BM * 64];
-    __shared__ __attribute__((aligned(16))) f16 sA1[BM * 64];
-    __shared__ __attribute__((aligned(16))) f16 sW0[BN * 64];
-    __shared__ __attribute__((aligned(16))) f16 sW1[BN * 64];
-
-    const int nbn = (p.N + BN - 1) / BN, nbm = (p.M + BM - 1) / BM;
-    // Plain products run a persistent grid (one workgroup per CU) over xcd_tile's virtual tile order: workgroup w
-    // takes virtual tiles w, w + G, w + 2 G, ... (G a multiple of 8, so all of a workgroup's tiles lie on its XCD),
-    // and the next tile's first K tile is requested before this tile's epilogue runs, so its round trip and the
-    // workgroup's dispatch are not paid once per tile. The convolution takes one tile per workgroup.
-    constexpr bool PERSIST = ALOAD == ALOAD_PLAIN;
-    const int nvirt = 8 * (p.share > 0 ? p.share : ((nbm + 7) >> 3) * nbn), vstep = PERSIST ? (int)gridDim.x : nvirt;
-    int v = blockIdx.x, bm = 0, bn = 0;
-    while (v < nvirt && !xcd_tile(v, nbm, nbn, p.share, &bm, &bn)) v += vstep;
-    if (v >= nvirt) return;
-    // the wave index through readfirstlane: wave-uniform values (tile origins, store descriptors) stay scalar
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm = wave >> 2, wn = wave & 3, lr = lane & 31, lh = lane >> 5;
-    // the epilogue's bias values are requested here, ahead of the operand loads, so that their round trip is hidden
-    // behind the K loop instead of stalling the products' end. One unconditional buffer load per column block (a
-    // missing bias is a descriptor of no bytes, which reads zeros): a branch would make the compiler wait for the
-    // load at once. Kept as fp16 until used.
-    int n0 = bn * BN + wn * WN;
-    const __amdgpu_buffer_rsrc_t rB = rsrc(p.bias, p.bias ? (unsigned)p.N * 2 : 0u);
-    f16 bias_h[TN];
-#pragma unroll
-    for (int j = 0; j < TN; j++)
-        bias_h[j] = __builtin_bit_cast(f16, __builtin_amdgcn_raw_buffer_load_b16(rB, (unsigned)(n0 + j * 32 + lr) * 2, 0, 0));
-    const int nk = p.K >> 6;
-    // this lane's slot in a direct load: row lrow of an 8-row slice, 16-byte chunk lc of the row
-    // (slice r of a wave starts at a multiple of 8 rows whose bit 3 is r's bit 0)
-    const int lrow = lane >> 3, lc = (lane & 7) ^ lrow;
-    static_assert((BM / NW) % 16 == 0 && (BN / NW) % 16 == 0, "a wave's slices must start on a 16-row boundary");
-
-    const __amdgpu_buffer_rsrc_t rW = rsrc(p.W, (unsigned)p.N * p.K * 2);
-    unsigned voW[WR];
-    auto set_w = [&](int bn_) {
-#pragma unroll
-        for (int r = 0; r < WR; r++)
-            voW[r] = (unsigned)(bn_ * BN + wave * (BN / NW) + 8 * r + lrow) * p.K * 2 + (lc ^ (r & 1)) * 16;
-    };
-    set_w(bn);
-    __amdgpu_buffer_rsrc_t rA;
-    unsigned voA[AR];
-    int srow[AR], stime[AR];  // conv: source row of tap 0 and its time index (-1 .. tin - 1), or a row past M
-    auto set_a = [&](int bm_) {
-#pragma unroll
-        for (int r = 0; r < AR; r++)
-            voA[r] = (unsigned)(bm_ * BM + wave * (BM / NW) + 8 * r + lrow) * p.lda * 2 + (lc ^ (r & 1)) * 16;
-    };
-    if (ALOAD == ALOAD_PLAIN) {
-        rA = rsrc(p.A, (unsigned)p.M * p.lda * 2);
-        set_a(bm);
-    } else {
-        const int clips = p.M / p.conv_tout;
-        rA = rsrc(p.A, (unsigned)clips * p.conv_tin * p.conv_cin * 2);
-#pragma unroll
-        for (int r = 0; r < AR; r++) {
-            const int m = bm * BM + wave * (BM / NW) + 8 * r + lrow;
-            const int g = m / p.conv_tout, t = m - g * p.conv_tout;
-            stime[r] = m < p.M ? p.conv_stride * t - 1 : -(1 << 20);
-            srow[r] = g * p.conv_tin + p.conv_stride * t - 1;
+// One lane's direct loads of an A row: byte offset of its 16-byte chunk (column c of the K tile) in K tile kt. Plain
+// rows take the K tile through the load's scalar offset. A convolution row is a contiguous run of the source, because
+// the taps are adjacent source rows: column k = tap * cin + ci of (clip g, time t) is element
+// (g * tin + stride * t - 1) * cin + k. Outside [lo, lo + span) lie the zero padding (tap 0 at t = 0, tap 2 past the
+// last source row) and K's own padding past 3 cin: read past the descriptor, so zeros.
+template <int ALOAD>
+struct ALane {
+    unsigned vo;
+    int off;
+    unsigned span;
+    __device__ __forceinline__ void set(const MzGemm& p, int m, int c) {
+        if (ALOAD == ALOAD_PLAIN) {
+            vo = (unsigned)m * p.lda * 2 + c * 2;
+        } else {
+            const int g = m / p.conv_tout, s = p.conv_stride * (m - g * p.conv_tout) - 1;
+            const int lo = s < 0 ? p.conv_cin : 0, hi = min(3, p.conv_tin - s) * p.conv_cin;
+            vo = (unsigned)((g * p.conv_tin + s) * p.conv_cin + c) * 2u;
+            off = c - lo;
+            span = m < p.M ? max(hi - lo, 0) : 0;
         }
     }
+    __device__ __forceinline__ unsigned voff(int kt) const {
+        if (ALOAD == ALOAD_PLAIN) return vo;
+        return (unsigned)(kt * 64 + off) < span ? vo + kt * 128 : OOB;
+    }
+};
+// bytes of the A operand (the descriptor's range)
+template <int ALOAD>
+__device__ __forceinline__ unsigned a_bytes(const MzGemm& p) {
+    return ALOAD == ALOAD_PLAIN ? (unsigned)p.M * p.lda * 2
+                                : (unsigned)(p.M / p.conv_tout) * p.conv_tin * p.conv_cin * 2;
+}
 
-    auto issue = [&](int kt, f16* a, f16* w) {
-        if (ALOAD == ALOAD_PLAIN) {
-#pragma unroll
-            for (int r = 0; r < AR; r++)
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(rA, LDSP(a + (wave * (BM / NW) + 8 * r) * 64), 16, voA[r],
-                                                         kt * 128, 0, 0);
-        } else {
-            // implicit im2col: column k = tap * cin + ci of a row reads source time stride * t + tap - 1
-            int tap2[2], ci2[2];
-#pragma unroll
-            for (int h = 0; h < 2; h++) {
-                const int k0 = kt * 64 + (lc ^ h) * 8;
-                tap2[h] = k0 / p.conv_cin;
-                ci2[h] = k0 - tap2[h] * p.conv_cin;
-            }
-#pragma unroll
-            for (int r = 0; r < AR; r++) {
-                const int tap = tap2[r & 1], ci = ci2[r & 1];
-                const int tt = stime[r] + tap;
-                const bool ok = tap < 3 && tt >= 0 && tt < p.conv_tin;
-                const unsigned vo = ok ? (unsigned)((srow[r] + tap) * p.conv_cin + ci) * 2 : OOB;
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(rA, LDSP(a + (wave * (BM / NW) + 8 * r) * 64), 16, vo, 0, 0,
-                                                         0);
-            }
-        }
-#pragma unroll
-        for (int r = 0; r < WR; r++)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(rW, LDSP(w + (wave * (BN / NW) + 8 * r) * 64), 16, voW[r],
-                                                     kt * 128, 0, 0);
-    };
-
-    f32x16 acc[TM][TN];
-#pragma unroll
-    for (int i = 0; i < TM; i++)
-#pragma unroll
-        for (int j = 0; j < TN; j++) acc[i][j] = f32x16{};
-    // Fragments of K step kk (16 wide) of a tile: TM A and TN W fragments. They are double buffered across steps:
-    // step kk + 1's reads go out while step kk's products issue, one read between two products (explicit scheduling
-    // groups; the hardware interleaves the two waves of a SIMD on top). The last step's products are split around
-    // the tile's wait and barrier, so that the next tile's first fragments are read under the second half.
-    f16x8 fa0[TM], fw0[TN], fa1[TM], fw1[TN];
-    auto frags = [&](const f16* a, const f16* w, int kk, f16x8(&fa)[TM], f16x8(&fw)[TN]) {
-        const int sw = (((2 * kk + lh) ^ (lr & 7) ^ ((lr >> 3) & 1)) << 3);
-#pragma unroll
-        for (int i = 0; i < TM; i++) fa[i] = *(const f16x8*)&a[(wm * WM + i * 32 + lr) * 64 + sw];
-#pragma unroll
-        for (int j = 0; j < TN; j++) fw[j] = *(const f16x8*)&w[(wn * WN + j * 32 + lr) * 64 + sw];
-    };
-    auto mma = [&](const f16x8(&fa)[TM], const f16x8(&fw)[TN], int i0, int i1) {
-#pragma unroll
-        for (int i = i0; i < i1; i++)
-#pragma unroll
-            for (int j = 0; j < TN; j++) acc[i][j] = mfma32(fa[i], fw[j], acc[i][j]);
-    };
-    constexpr int NM = TM * TN, NR = TM + TN, NI = NM < NR ? NM : NR;  // products, reads, interleaved pairs
-    auto interleave = [&]() {
-#pragma unroll
-        for (int g = 0; g < NI; g++) {
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // one MFMA
-            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // one LDS read
-        }
-        if (NM > NI) __builtin_amdgcn_sched_group_barrier(0x008, NM - NI, 0);
-        if (NR > NI) __builtin_amdgcn_sched_group_barrier(0x100, NR - NI, 0);
-    };
-    // tile kt from (a, w), its step-0 fragments already in (fa0, fw0); the loads of tile kt + 1 go to (an, wn_)
-    auto tile = [&](int kt, const f16* a, const f16* w, f16* an, f16* wn_) {
-        if (kt + 1 < nk) issue(kt + 1, an, wn_);
-        frags(a, w, 1, fa1, fw1);
-        mma(fa0, fw0, 0, TM);
-        __builtin_amdgcn_sched_group_barrier(0x020, AR + WR, 0);  // the next tile's loads first
-        interleave();
-        frags(a, w, 2, fa0, fw0);
-        mma(fa1, fw1, 0, TM);
-        interleave();
-        frags(a, w, 3, fa1, fw1);
-        mma(fa0, fw0, 0, TM);
-        interleave();
-        mma(fa1, fw1, 0, TM / 2);
-        __builtin_amdgcn_sched_barrier(0);
-        __builtin_amdgcn_s_waitcnt(0);  // tile kt + 1 has landed (vmcnt) and every wave is done with tile kt
-        __syncthreads();
-        if (kt + 1 < nk) frags(an, wn_, 0, fa0, fw0);
-        mma(fa1, fw1, TM / 2, TM);
-        __builtin_amdgcn_sched_barrier(0);
-    };
-
-    // epilogue: acc[i][j] element r is row m0 + i * 32 + 8 (r / 4) + 4 lh + r % 4, column n0 + j * 32 + lr
-    auto epilogue = [&](const int m0, const int n0) {
+// Epilogue of a wave's (BM / NWM) x (BN / NWN) tile at (m0, n0): acc[i][j] element r is row m0 + i * 32 + 8 (r / 4) + 4 lh
+// + r % 4, column n0 + j * 32 + lr. stage: LDS for the transposes of the encoder's v (32 x WN halves per wave), free once
+// every wave of the workgroup has passed its last operand read.
+template <int BM, int BN, int NWM, int NWN, int EPI>
+__device__ __forceinline__ void gemm_epilogue(const MzGemm& p, const f32x16 (&acc)[BM / NWM / 32][BN / NWN / 32],
+                                              const f16 (&bias_h)[BN / NWN / 32], f16* stage, const int m0, const int n0) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    constexpr int WN = BN / NWN, TM = BM / NWM / 32, TN = WN / 32;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lr = lane & 31, lh = lane >> 5;
     if (EPI == EPI_HEADS) {
         if (p.kind == 3) lds_barrier();  // every wave is done reading operands: LDS is free for the v transposes
         const int blk = n0 >> 6;           // a wave's columns lie in one 64-wide head block (WN <= 64)
         const bool vt = p.kind == 3 && blk / p.nh == 2;
         if (vt) {
             // encoder v: stage each 32-row slice of the wave's tile in LDS as [column][row] (the wave's own 32 x WN
-            // halves of sW1, which the next tile's first loads leave alone: 8 waves x 32 x WN <= BN x 64) and write
-            // runs of 4 token positions
-            static_assert(NW * 32 * WN <= BN * 64, "staging slice exceeds sW1");
-            f16* st = sW1 + wave * (32 * WN);
+            // halves of the stage) and write runs of 4 token positions
+            static_assert(EPI != EPI_HEADS || NWM * 32 * WN * NWN <= BN * 64, "the staging slices exceed one W tile");
+            f16* st = stage + wave * (32 * WN);
 #pragma unroll
             for (int i = 0; i < TM; i++) {
 #pragma unroll
@@ -358,6 +244,129 @@ __global__ void __launch_bounds__(NW * 64) gemm_kernel(const MzGemm p) {
                 ((float*)p.out)[(long)m * p.ldo + n] = gelu_erf(v) + (float)p.pos[(long)(m % MZ_TENC) * p.N + n];
             }
     }
+#endif
+}
+
+template <int BM, int BN, int ALOAD, int EPI>
+__global__ void __launch_bounds__(NW * 64) gemm_kernel(const MzGemm p) {
+#if defined(__HIP_DEVICE_COMPILE__)  // the buffer-resource type exists only in the device pass
+    constexpr int WM = BM / 2, WN = BN / 4, TM = WM / 32, TN = WN / 32;
+    constexpr int AR = BM / (8 * NW), WR = BN / (8 * NW);  // 8-row slices each wave loads per K tile
+    static_assert(AR >= 1 && WR >= 1 && TN >= 1, "tile too small for 8 waves");
+    __shared__ __attribute__((aligned(16))) f16 sA0[BM * 64];
+    __shared__ __attribute__((aligned(16))) f16 sA1[BM * 64];
+    __shared__ __attribute__((aligned(16))) f16 sW0[BN * 64];
+    __shared__ __attribute__((aligned(16))) f16 sW1[BN * 64];
+
+    const int nbn = (p.N + BN - 1) / BN, nbm = (p.M + BM - 1) / BM;
+    // Plain products run a persistent grid (one workgroup per CU) over xcd_tile's virtual tile order: workgroup w
+    // takes virtual tiles w, w + G, w + 2 G, ... (G a multiple of 8, so all of a workgroup's tiles lie on its XCD),
+    // and the next tile's first K tile is requested before this tile's epilogue runs, so its round trip and the
+    // workgroup's dispatch are not paid once per tile. The convolution takes one tile per workgroup.
+    constexpr bool PERSIST = ALOAD == ALOAD_PLAIN;
+    const int nvirt = 8 * (p.share > 0 ? p.share : ((nbm + 7) >> 3) * nbn), vstep = PERSIST ? (int)gridDim.x : nvirt;
+    int v = blockIdx.x, bm = 0, bn = 0;
+    while (v < nvirt && !xcd_tile(v, nbm, nbn, p.share, &bm, &bn)) v += vstep;
+    if (v >= nvirt) return;
+    // the wave index through readfirstlane: wave-uniform values (tile origins, store descriptors) stay scalar
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave >> 2, wn = wave & 3, lr = lane & 31, lh = lane >> 5;
+    // the epilogue's bias values are requested here, ahead of the operand loads, so that their round trip is hidden
+    // behind the K loop instead of stalling the products' end. One unconditional buffer load per column block (a
+    // missing bias is a descriptor of no bytes, which reads zeros): a branch would make the compiler wait for the
+    // load at once. Kept as fp16 until used.
+    int n0 = bn * BN + wn * WN;
+    const __amdgpu_buffer_rsrc_t rB = rsrc(p.bias, p.bias ? (unsigned)p.N * 2 : 0u);
+    f16 bias_h[TN];
+#pragma unroll
+    for (int j = 0; j < TN; j++)
+        bias_h[j] = __builtin_bit_cast(f16, __builtin_amdgcn_raw_buffer_load_b16(rB, (unsigned)(n0 + j * 32 + lr) * 2, 0, 0));
+    const int nk = p.K >> 6;
+    // this lane's slot in a direct load: row lrow of an 8-row slice, 16-byte chunk lc of the row
+    // (slice r of a wave starts at a multiple of 8 rows whose bit 3 is r's bit 0)
+    const int lrow = lane >> 3, lc = (lane & 7) ^ lrow;
+    static_assert((BM / NW) % 16 == 0 && (BN / NW) % 16 == 0, "a wave's slices must start on a 16-row boundary");
+
+    const __amdgpu_buffer_rsrc_t rW = rsrc(p.W, (unsigned)p.N * p.K * 2);
+    unsigned voW[WR];
+    auto set_w = [&](int bn_) {
+#pragma unroll
+        for (int r = 0; r < WR; r++)
+            voW[r] = (unsigned)(bn_ * BN + wave * (BN / NW) + 8 * r + lrow) * p.K * 2 + (lc ^ (r & 1)) * 16;
+    };
+    set_w(bn);
+    const __amdgpu_buffer_rsrc_t rA = rsrc(p.A, a_bytes<ALOAD>(p));
+    ALane<ALOAD> la[AR];
+    auto set_a = [&](int bm_) {
+#pragma unroll
+        for (int r = 0; r < AR; r++) la[r].set(p, bm_ * BM + wave * (BM / NW) + 8 * r + lrow, (lc ^ (r & 1)) * 8);
+    };
+    set_a(bm);
+
+    auto issue = [&](int kt, f16* a, f16* w) {
+#pragma unroll
+        for (int r = 0; r < AR; r++)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rA, LDSP(a + (wave * (BM / NW) + 8 * r) * 64), 16, la[r].voff(kt),
+                                                     ALOAD == ALOAD_PLAIN ? kt * 128 : 0, 0, 0);
+#pragma unroll
+        for (int r = 0; r < WR; r++)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rW, LDSP(w + (wave * (BN / NW) + 8 * r) * 64), 16, voW[r],
+                                                     kt * 128, 0, 0);
+    };
+
+    f32x16 acc[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++) acc[i][j] = f32x16{};
+    // Fragments of K step kk (16 wide) of a tile: TM A and TN W fragments. They are double buffered across steps:
+    // step kk + 1's reads go out while step kk's products issue, one read between two products (explicit scheduling
+    // groups; the hardware interleaves the two waves of a SIMD on top). The last step's products are split around
+    // the tile's wait and barrier, so that the next tile's first fragments are read under the second half.
+    f16x8 fa0[TM], fw0[TN], fa1[TM], fw1[TN];
+    auto frags = [&](const f16* a, const f16* w, int kk, f16x8(&fa)[TM], f16x8(&fw)[TN]) {
+        const int sw = (((2 * kk + lh) ^ (lr & 7) ^ ((lr >> 3) & 1)) << 3);
+#pragma unroll
+        for (int i = 0; i < TM; i++) fa[i] = *(const f16x8*)&a[(wm * WM + i * 32 + lr) * 64 + sw];
+#pragma unroll
+        for (int j = 0; j < TN; j++) fw[j] = *(const f16x8*)&w[(wn * WN + j * 32 + lr) * 64 + sw];
+    };
+    auto mma = [&](const f16x8(&fa)[TM], const f16x8(&fw)[TN], int i0, int i1) {
+#pragma unroll
+        for (int i = i0; i < i1; i++)
+#pragma unroll
+            for (int j = 0; j < TN; j++) acc[i][j] = mfma32(fa[i], fw[j], acc[i][j]);
+    };
+    constexpr int NM = TM * TN, NR = TM + TN, NI = NM < NR ? NM : NR;  // products, reads, interleaved pairs
+    auto interleave = [&]() {
+#pragma unroll
+        for (int g = 0; g < NI; g++) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // one MFMA
+            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // one LDS read
+        }
+        if (NM > NI) __builtin_amdgcn_sched_group_barrier(0x008, NM - NI, 0);
+        if (NR > NI) __builtin_amdgcn_sched_group_barrier(0x100, NR - NI, 0);
+    };
+    // tile kt from (a, w), its step-0 fragments already in (fa0, fw0); the loads of tile kt + 1 go to (an, wn_)
+    auto tile = [&](int kt, const f16* a, const f16* w, f16* an, f16* wn_) {
+        if (kt + 1 < nk) issue(kt + 1, an, wn_);
+        frags(a, w, 1, fa1, fw1);
+        mma(fa0, fw0, 0, TM);
+        __builtin_amdgcn_sched_group_barrier(0x020, AR + WR, 0);  // the next tile's loads first
+        interleave();
+        frags(a, w, 2, fa0, fw0);
+        mma(fa1, fw1, 0, TM);
+        interleave();
+        frags(a, w, 3, fa1, fw1);
+        mma(fa0, fw0, 0, TM);
+        interleave();
+        mma(fa1, fw1, 0, TM / 2);
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_waitcnt(0);  // tile kt + 1 has landed (vmcnt) and every wave is done with tile kt
+        __syncthreads();
+        if (kt + 1 < nk) frags(an, wn_, 0, fa0, fw0);
+        mma(fa1, fw1, TM / 2, TM);
+        __builtin_amdgcn_sched_barrier(0);
     };
 
     // two K tiles per iteration, one per LDS buffer (distinct arrays, so the compiler sees that the loads in flight
@@ -391,7 +400,8 @@ __global__ void __launch_bounds__(NW * 64) gemm_kernel(const MzGemm p) {
             set_w(bnn);
             issue(0, sA0, sW0);
         }
-        epilogue(m0, n0c);
+        // (the v transposes go to sW1, which the next tile's first loads leave alone)
+        gemm_epilogue<BM, BN, 2, 4, EPI>(p, acc, bias_h, sW1, m0, n0c);
         if (!more) break;
         v = vn;
         bm = bmn;
@@ -409,29 +419,172 @@ __global__ void __launch_bounds__(NW * 64) gemm_kernel(const MzGemm p) {
 #endif
 }
 
-template <int BM, int BN, int ALOAD, int EPI>
-hipError_t launch(hipStream_t s, const MzGemm& g) {
-    const int nbm = (g.M + BM - 1) / BM, nbn = (g.N + BN - 1) / BN, cus = mz_cu_count();
+// The same product for grids that leave most CUs with one small tile. There a K tile does not take its products' time: with
+// two buffers in turn it takes its loads' round trip, and with the fragments read a 16-wide K step ahead the LDS reads'
+// latency four times (one wave per SIMD has nothing else to run). So NWM x NWN waves keep a ring of four K tiles in LDS,
+// three or four in flight, and hold all fragments of a K tile in registers: tile k + 1's are read while tile k is
+// multiplied, and a slot is refilled as soon as every wave has read it. Same products in the same order as
+// gemm_kernel, so the same bits. One tile per workgroup.
+template <int BM, int BN, int NWM, int NWN, int ALOAD, int EPI>
+__global__ void __launch_bounds__(NWM * NWN * 64) gemm_ring_kernel(const MzGemm p) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    constexpr int NWV = NWM * NWN, WM = BM / NWM, WN = BN / NWN, TM = WM / 32, TN = WN / 32;
+    constexpr int AR = BM / (8 * NWV), WR = BN / (8 * NWV), LPT = AR + WR;  // loads per wave and K tile
+    static_assert(3 * LPT < 64, "the wait's count");
+    static_assert((BM / NWV) % 16 == 0 && (BN / NWV) % 16 == 0, "a wave's slices must start on a 16-row boundary");
+    // one array per slot (the A tile, then the W tile), so that the compiler sees that the loads in flight never alias
+    // the tile being read (it tells few arrays apart: with A and W in arrays of their own it waits for the loads)
+    __shared__ __attribute__((aligned(16))) f16 s0[(BM + BN) * 64], s1[(BM + BN) * 64], s2[(BM + BN) * 64], s3[(BM + BN) * 64];
+
+    const int nbn = (p.N + BN - 1) / BN, nbm = (p.M + BM - 1) / BM, nk = p.K >> 6;
+    int bm, bn;
+    if (!xcd_tile(blockIdx.x, nbm, nbn, p.share, &bm, &bn)) return;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave / NWN, wn = wave % NWN, lr = lane & 31, lh = lane >> 5;
+    const int m0 = bm * BM + wm * WM, n0 = bn * BN + wn * WN;
+    const __amdgpu_buffer_rsrc_t rB = rsrc(p.bias, p.bias ? (unsigned)p.N * 2 : 0u);
+    f16 bias_h[TN];
+#pragma unroll
+    for (int j = 0; j < TN; j++)
+        bias_h[j] = __builtin_bit_cast(f16, __builtin_amdgcn_raw_buffer_load_b16(rB, (unsigned)(n0 + j * 32 + lr) * 2, 0, 0));
+
+    const int lrow = lane >> 3, lc = (lane & 7) ^ lrow;
+    const __amdgpu_buffer_rsrc_t rA = rsrc(p.A, a_bytes<ALOAD>(p)), rW = rsrc(p.W, (unsigned)p.N * p.K * 2);
+    ALane<ALOAD> la[AR];
+    unsigned voW[WR];
+#pragma unroll
+    for (int r = 0; r < AR; r++) la[r].set(p, bm * BM + wave * (BM / NWV) + 8 * r + lrow, (lc ^ (r & 1)) * 8);
+#pragma unroll
+    for (int r = 0; r < WR; r++)
+        voW[r] = (unsigned)(bn * BN + wave * (BN / NWV) + 8 * r + lrow) * p.K * 2 + (lc ^ (r & 1)) * 16;
+    // K tile kt into slot a; past the last one the loads go past the descriptors (zeros, no memory read), so that every
+    // tile's count of loads in flight is the same
+    auto issue = [&](int kt, f16* a) {
+        f16* w = a + BM * 64;
+        const bool on = kt < nk;
+        const int so = on ? kt * 128 : 0;
+#pragma unroll
+        for (int r = 0; r < AR; r++)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rA, LDSP(a + (wave * (BM / NWV) + 8 * r) * 64), 16,
+                                                     on ? la[r].voff(kt) : OOB, ALOAD == ALOAD_PLAIN ? so : 0, 0, 0);
+#pragma unroll
+        for (int r = 0; r < WR; r++)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rW, LDSP(w + (wave * (BN / NWV) + 8 * r) * 64), 16,
+                                                     on ? voW[r] : OOB, so, 0, 0);
+    };
+
+    f32x16 acc[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++) acc[i][j] = f32x16{};
+    struct Frags {
+        f16x8 a[4][TM], w[4][TN];
+    } f0, f1;
+    auto frags = [&](const f16* a, Frags& f) {
+        const f16* w = a + BM * 64;
+#pragma unroll
+        for (int kk = 0; kk < 4; kk++) {
+            const int sw = (((2 * kk + lh) ^ (lr & 7) ^ ((lr >> 3) & 1)) << 3);
+#pragma unroll
+            for (int i = 0; i < TM; i++) f.a[kk][i] = *(const f16x8*)&a[(wm * WM + i * 32 + lr) * 64 + sw];
+#pragma unroll
+            for (int j = 0; j < TN; j++) f.w[kk][j] = *(const f16x8*)&w[(wn * WN + j * 32 + lr) * 64 + sw];
+        }
+    };
+    // K tile kt, whose fragments are in f and which every wave has read once this wave is past the barrier: its slot a
+    // takes tile kt + 4, tile kt + 1's fragments are read from an into g
+    auto tile = [&](int kt, f16* a, const f16* an, const Frags& f, Frags& g) {
+        __builtin_amdgcn_s_waitcnt(vm_lgkm_wait(2 * LPT));  // tile kt + 1 has landed; kt + 2 and kt + 3 in flight
+        asm volatile("s_barrier" ::: "memory");
+        issue(kt + 4, a);
+        frags(an, g);
+#pragma unroll
+        for (int kk = 0; kk < 4; kk++)
+#pragma unroll
+            for (int i = 0; i < TM; i++)
+#pragma unroll
+                for (int j = 0; j < TN; j++) acc[i][j] = mfma32(f.a[kk][i], f.w[kk][j], acc[i][j]);
+        __builtin_amdgcn_sched_group_barrier(0x020, LPT, 0);  // the loads first, then reads between products
+        constexpr int NM = 4 * TM * TN, NR = 4 * (TM + TN), Q = (NR + NM - 1) / NM;
+#pragma unroll
+        for (int i = 0; i < NM; i++) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x100, Q, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    issue(0, s0);
+    __builtin_amdgcn_sched_barrier(0);  // in this order: the waits count on it
+    issue(1, s1);
+    __builtin_amdgcn_sched_barrier(0);
+    issue(2, s2);
+    __builtin_amdgcn_sched_barrier(0);
+    issue(3, s3);
+    __builtin_amdgcn_s_waitcnt(vm_lgkm_wait(3 * LPT));
+    asm volatile("s_barrier" ::: "memory");
+    frags(s0, f0);
+    // whole rounds of the ring without a branch inside (a way out of each tile makes the compiler wait for loads in
+    // flight at the loop's head), then the K tiles left over
+    int kt = 0;
+    for (; kt + 4 <= nk; kt += 4) {
+        tile(kt, s0, s1, f0, f1);
+        tile(kt + 1, s1, s2, f1, f0);
+        tile(kt + 2, s2, s3, f0, f1);
+        tile(kt + 3, s3, s0, f1, f0);
+    }
+    if (kt < nk) tile(kt, s0, s1, f0, f1);
+    if (kt + 1 < nk) tile(kt + 1, s1, s2, f1, f0);
+    if (kt + 2 < nk) tile(kt + 2, s2, s3, f0, f1);
+    // no load may still be on its way into LDS when the workgroup ends, or when the v transposes are staged there
+    __builtin_amdgcn_s_waitcnt(vm_lgkm_wait(0));
+    if (EPI == EPI_HEADS) asm volatile("s_barrier" ::: "memory");
+    gemm_epilogue<BM, BN, NWM, NWN, EPI>(p, acc, bias_h, s0, m0, n0);
+#endif
+}
+
+// virtual tiles of the grid, and how the XCDs share them
+int share_tiles(int nbm, int nbn, int cus, MzGemm* p) {
     // An XCD takes whole bands unless equal shares of the tiles save it a round of its CUs: 12 or 18 block rows (one
     // clip in 128-row, three in 256-row blocks) are six bands, which left two XCDs without work (encoder pass of one
     // clip, width 1280: 611 -> 530 us; three clips, width 768: 520 -> 460). Where the rounds are the same, the bands
     // keep an XCD's panels together (8 clips, width 1280: 1562 us, against 1594 with equal shares).
     const int band = ((nbm + 7) / 8) * nbn, even = (nbm * nbn + 7) / 8, per = cus / 8;
+    p->share = (even + per - 1) / per < (band + per - 1) / per ? even : 0;
+    return 8 * (p->share ? even : band);
+}
+
+template <int BM, int BN, int ALOAD, int EPI>
+hipError_t launch(hipStream_t s, const MzGemm& g) {
+    const int nbm = (g.M + BM - 1) / BM, nbn = (g.N + BN - 1) / BN, cus = mz_cu_count();
     MzGemm p = g;
-    p.share = (even + per - 1) / per < (band + per - 1) / per ? even : 0;
-    const int nvirt = 8 * (p.share ? even : band), grid = ALOAD == ALOAD_PLAIN && nvirt > cus ? cus : nvirt;
+    const int nvirt = share_tiles(nbm, nbn, cus, &p), grid = ALOAD == ALOAD_PLAIN && nvirt > cus ? cus : nvirt;
     hipLaunchKernelGGL((gemm_kernel<BM, BN, ALOAD, EPI>), dim3(grid), dim3(NW * 64), 0, s, p);
+    return hipGetLastError();
+}
+
+template <int BM, int BN, int NWM, int NWN, int ALOAD, int EPI>
+hipError_t launch_ring(hipStream_t s, const MzGemm& g) {
+    MzGemm p = g;
+    const int nvirt = share_tiles((g.M + BM - 1) / BM, (g.N + BN - 1) / BN, mz_cu_count(), &p);
+    hipLaunchKernelGGL((gemm_ring_kernel<BM, BN, NWM, NWN, ALOAD, EPI>), dim3(nvirt), dim3(NWM * NWN * 64), 0, s, p);
     return hipGetLastError();
 }
 
 template <int ALOAD, int EPI>
 hipError_t pick(hipStream_t s, const MzGemm& g) {
-    // 256 x 256 tiles once they cover most of the 256 CUs; 256 x 128, then 128 x 128 below that
-    const long t256 = (long)((g.M + 255) / 256) * ((g.N + 255) / 256);
-    if (t256 >= 200) return launch<256, 256, ALOAD, EPI>(s, g);
-    const long t128 = (long)((g.M + 255) / 256) * ((g.N + 127) / 128);
-    if (t128 >= 200) return launch<256, 128, ALOAD, EPI>(s, g);
-    return launch<128, 128, ALOAD, EPI>(s, g);
+    // The largest tile that still gives half of the CUs one each: below that, more CUs at work gain more than the
+    // larger tile's fewer operand bytes per product. Over M = 1500 c (c = 1 .. 8) and the N, K of widths 384 to 1280 the
+    // choice is within 4% of the fastest of the five shapes (11% at one: M 4500, N 5120, K 1280). M = 1500, K = 1280 / 5120,
+    // N = 1280: 128 x 64 ring 9.4 / 28.4 us, 64 x 64 ring 10.2 / 34.9, 128 x 128 ring 11.0 / 34.0, a 128 x 128 tile with
+    // two buffers (the rule before) 13.5 / 52.9. N = 384, K = 1536: 64 x 64 ring 6.5 us, before 11.9.
+    auto tiles = [&](int bm, int bn) { return (long)((g.M + bm - 1) / bm) * ((g.N + bn - 1) / bn); };
+    const long half = mz_cu_count() / 2 + 2;
+    if (tiles(256, 256) >= half) return launch<256, 256, ALOAD, EPI>(s, g);
+    if (tiles(256, 128) >= half) return launch<256, 128, ALOAD, EPI>(s, g);
+    if (tiles(128, 128) >= half) return launch_ring<128, 128, 2, 4, ALOAD, EPI>(s, g);
+    if (tiles(128, 64) >= half) return launch_ring<128, 64, 2, 2, ALOAD, EPI>(s, g);
+    return launch_ring<64, 64, 2, 2, ALOAD, EPI>(s, g);
 }
 
 }  // namespace

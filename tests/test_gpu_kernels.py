@@ -350,6 +350,51 @@ def test_gemm_persistent_shapes(ctx, m, n, k):
         ctx.free(p)
 
 
+@pytest.mark.parametrize("m,n,k", [(33, 4, 64), (64, 64, 256), (65, 132, 128), (1500, 384, 192), (1500, 516, 1280),
+                                   (1500, 1284, 320), (1500, 1280, 5120), (1499, 2308, 448), (3000, 768, 384)])
+def test_gemm_small_grids(ctx, m, n, k):
+    """Products of few tiles: 64 x 64, 128 x 64 and 128 x 128 tiles with partial last rows and columns, and K tile counts
+    on both sides of the ring's four slots (1, 2, 3, 4, 5, 7 and whole rounds). The same bits as the same rows within a
+    product large enough for 256 x 256 tiles, and the float64 product."""
+    rng = np.random.default_rng(m + 3 * n + k)
+    big = 256 * (132 // ((n + 255) // 256) + 1)
+    x, w, b = f16(rng, (max(m, big), k)), f16(rng, (n, k), 0.05), f16(rng, (n,), 0.1)
+    dx, dw, db = (ctx.upload_new(a) for a in (x, w, b))
+    dy = ctx.alloc(x.shape[0] * n * 2)
+    out = []
+    for rows in (m, x.shape[0]):
+        L.check(L.lib().mz_gemm(ctx.h, dx, k, dw, dy, n, rows, n, k, db))
+        out.append(ctx.download(dy, (rows, n), np.float16))
+    np.testing.assert_array_equal(out[0], out[1][:m])
+    assert_f16(out[0], x[:m].astype(np.float64) @ w.astype(np.float64).T + b)
+    for p in (dx, dw, db, dy):
+        ctx.free(p)
+
+
+@pytest.mark.parametrize("clips,cin,n,stride", [(1, 80, 384, 1), (1, 384, 384, 2), (3, 128, 512, 1), (1, 512, 1280, 2)])
+def test_conv_small_grids(ctx, clips, cin, n, stride):
+    """The convolution's padding (both ends of each clip, K past the taps) in the tiles of few clips: the same bits as
+    the plain product of the unrolled rows."""
+    rng = np.random.default_rng(clips + cin + n)
+    src, b = f16(rng, (clips, 3000, cin)), f16(rng, (n,), 0.1)
+    k, t = (3 * cin + 63) // 64 * 64, 3000 // stride
+    w = f16(rng, (n, k), 0.05)  # non-zero past the taps too: those columns of the rows read as zero
+    rows = np.zeros((clips, t, k), np.float16)
+    pad = np.pad(src, ((0, 0), (1, 1), (0, 0)))
+    for tap in range(3):
+        rows[:, :, tap * cin:(tap + 1) * cin] = pad[:, tap:tap + stride * (t - 1) + 1:stride]
+    ds, dr, dw, db = (ctx.upload_new(a) for a in (src, rows, w, b))
+    dy = ctx.alloc(clips * t * n * 2)
+    out = []
+    for conv in (dict(a=ds, conv_cin=cin, conv_tin=3000, conv_tout=t, conv_stride=stride), dict(a=dr, lda=k)):
+        L.check(L.lib().mz_linear(ctx.h, linear_args(epilogue=L.EPI_GELU_F16, w=dw, bias=db, m=clips * t, n=n, k=k,
+                                                     out=dy, ldo=n, **conv)))
+        out.append(ctx.download(dy, (clips * t, n), np.float16))
+    np.testing.assert_array_equal(out[0], out[1])
+    for p in (ds, dr, dw, db, dy):
+        ctx.free(p)
+
+
 def test_conv_stem_implicit_gemm(ctx):
     """mel transpose + conv1 (k 3, pad 1) + GELU, conv2 (stride 2) + GELU + positions, against the oracle's conv1d."""
     rng = np.random.default_rng(6)
