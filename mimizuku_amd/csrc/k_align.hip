@@ -12,8 +12,8 @@
 //   ts_cost_kernel   one workgroup per 32 x 64 tile of (row, column): median of the width-w reflect-padded window
 //                    of z-scores, summed over heads; the cells are stored in anti-diagonal-major order
 //                    [d = i + j][i], so that the DTW reads each diagonal with consecutive addresses
-//   ts_dtw_wave_kernel  tables of at most 256 rows: one wave per clip, four rows per lane, the previous two
-//                    anti-diagonals in registers and the moves packed in LDS, where one lane walks the path back
+//   ts_dtw_wave_kernel  tables of at most 256 rows: one row per lane of one to four waves per clip, the previous two
+//                    anti-diagonals in registers and the moves in LDS, where one lane walks the path back
 //   ts_dtw_kernel    larger tables: one workgroup per clip; the DTW table is filled one anti-diagonal per step (every
 //                    cell of a diagonal depends only on the two previous diagonals, kept in LDS), the move taken into
 //                    each cell goes to a trace in the same diagonal-major order, and one lane walks the path back.
@@ -237,10 +237,10 @@ __global__ void __launch_bounds__(256) ts_cost_kernel(const MzTs p) {
 }
 
 // One workgroup per clip. Row i of the table (0..R) is handled by threads i, i + blockDim, ... The costs are staged
-// in LDS DTW_CH diagonals at a time (diagonal-major, so a chunk is one contiguous run, copied with direct-to-LDS
+// in LDS DTW_STAGE diagonals at a time (diagonal-major, so a chunk is one contiguous run, copied with direct-to-LDS
 // loads) while the previous chunk is being used; within a chunk a diagonal waits only for the LDS traffic of the
 // one before (lds_barrier), so the trace stores and the next chunk's loads stay in flight.
-constexpr int DTW_CH = 12;
+constexpr int DTW_STAGE = 12;
 
 __global__ void __launch_bounds__(1024) ts_dtw_kernel(const MzTs p) {
 #if defined(__HIP_DEVICE_COMPILE__)  // the buffer-resource type exists only in the device pass
@@ -255,27 +255,27 @@ __global__ void __launch_bounds__(1024) ts_dtw_kernel(const MzTs p) {
     const int ld = p.ldd;
     float* diag = lds;                       // 3 x (R + 1): diagonals d, d - 1, d - 2 in rotation
     int* first = (int*)(lds + 3 * ld);       // per row: the column of the path's first cell in that row
-    float* chunk = lds + 4 * ld;             // 2 x DTW_CH diagonals of costs
+    float* chunk = lds + 4 * ld;             // 2 x DTW_STAGE diagonals of costs
     const float* cost = p.cost + c * p.diag_stride;
     signed char* tr = p.trace + c * p.diag_stride;
     // reads past the clip's cost table return zeros (the descriptor's range check)
     const __amdgpu_buffer_rsrc_t rc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(cost), (short)0,
                                                                          (int)(p.diag_stride * 4), 0x00020000);
     // a chunk buffer holds a whole number of 64-float wave copies (the last one may read past the chunk)
-    const int lane = tid & 63, wave = tid >> 6, per = (DTW_CH * ld + 63) & ~63;
+    const int lane = tid & 63, wave = tid >> 6, per = (DTW_STAGE * ld + 63) & ~63;
     auto stage = [&](int d0, float* dst) {
-        // wave w's lanes copy floats w * 64 + lane, + nt, ... of diagonals d0 .. d0 + DTW_CH - 1
+        // wave w's lanes copy floats w * 64 + lane, + nt, ... of diagonals d0 .. d0 + DTW_STAGE - 1
         for (int k = wave * 64; k < per; k += nt)
             __builtin_amdgcn_raw_ptr_buffer_load_lds(rc, (__attribute__((address_space(3))) void*)(dst + k), 4,
                                                      (unsigned)((d0 * ld + k + lane) * 4), 0, 0, 0);
     };
     stage(0, chunk);
-    for (int d0 = 0; d0 <= R + C; d0 += DTW_CH) {
-        float* cb = chunk + ((d0 / DTW_CH) & 1) * per;
+    for (int d0 = 0; d0 <= R + C; d0 += DTW_STAGE) {
+        float* cb = chunk + ((d0 / DTW_STAGE) & 1) * per;
         __builtin_amdgcn_s_waitcnt(0);  // this chunk's copies (and the trace stores so far) are done
         __syncthreads();                // ... in every wave, and the other buffer's last chunk is no longer read
-        if (d0 + DTW_CH <= R + C) stage(d0 + DTW_CH, chunk + (((d0 / DTW_CH) + 1) & 1) * per);
-        const int dend = min(d0 + DTW_CH, R + C + 1);
+        if (d0 + DTW_STAGE <= R + C) stage(d0 + DTW_STAGE, chunk + (((d0 / DTW_STAGE) + 1) & 1) * per);
+        const int dend = min(d0 + DTW_STAGE, R + C + 1);
         for (int d = d0; d < dend; d++) {
             float* cur = diag + (d % 3) * ld;
             const float* p1 = diag + ((d + 2) % 3) * ld;
@@ -340,133 +340,142 @@ __global__ void __launch_bounds__(1024) ts_dtw_kernel(const MzTs p) {
 #endif
 }
 
-// Tables of at most 256 rows (R <= 255): one wave per clip. Lane l holds table rows 4l .. 4l + 3 of the two
-// previous anti-diagonals in registers and takes row 4l - 1 from lane l - 1 through cross-lane moves, so a diagonal
-// needs no barrier and no LDS round trip; its costs arrive four per lane, one 16-byte load per lane for the whole
-// diagonal, DTW_PF diagonals ahead. The move into each cell (2 bits) is packed into LDS ([diagonal][lane], a byte
-// per lane), where the path is walked back. Same comparisons and results as ts_dtw_kernel, so the same bits.
-constexpr int DTW_PF = 16;
-constexpr int DTW_WAVE_ND = 256 + 1500;  // diagonals of a table: rows 0 .. 255, columns 0 .. 1500
+// Tables of at most 64 NW token rows: NW waves per clip, one table row per lane, a diagonal per step. A cell needs its
+// left neighbour (this lane, one diagonal back) and the row above at the two diagonals before, which is the lane before
+// one and two steps ago: one cross-lane move (DPP wave_shr) per step and no LDS round trip. Row 64 w (the last of the
+// wave before) reaches wave w in chunks of 64 diagonals through LDS: wave w works one chunk behind wave w - 1, with one
+// barrier per chunk, and takes the chunk's values out of a register that shifts by a lane per step. The moves (a bit per
+// lane and kind) collect in two registers per 32 diagonals and go to LDS, where the path is walked back a run of equal
+// moves at a time. The time is the serial chain of about 20 instructions per diagonal: 32 clips of 220 rows and 1500
+// columns 466 -> 147 us, one of 41 rows 415 -> 93 (four rows per lane in one wave and a walk of one cell at a time before).
+// Same comparisons and results as ts_dtw_kernel, so the same bits.
+constexpr int DTW_CH = 64;   // diagonals per chunk
+constexpr int DTW_NCH = 28;  // chunks of a table: its diagonals 2 .. R + C are at most 1792 (256 rows x 1500 columns: 1755)
 
-// lane l gets lane l - 1's v (lane 0: 0): a row shift within each 16-lane row (DPP row_shr:1), and the first lane of
-// rows 1 .. 3 takes the last lane of the row before through lane reads merged in with per-lane bit masks (made once
-// by the caller). Bitwise merges, not selects: the compiler turns a select between lane reads into branches.
-struct LaneMasks {
-    int keep, m16, m32, m48;  // all ones where the lane keeps the row shift / is lane 16, 32, 48
-};
-__device__ __forceinline__ float lane_prev(float v, const LaneMasks& k) {
-    const int x = __builtin_bit_cast(int, v);
-    int y = __builtin_amdgcn_update_dpp(0, x, 0x111, 0xF, 0xF, false) & k.keep;
-    y |= __builtin_amdgcn_readlane(x, 15) & k.m16;
-    y |= __builtin_amdgcn_readlane(x, 31) & k.m32;
-    y |= __builtin_amdgcn_readlane(x, 47) & k.m48;
-    return __builtin_bit_cast(float, y);
+// lane l gets lane l - 1's v, lane 0 first; lane l gets lane l + 1's v, lane 63 last (DPP wave_shr:1, wave_shl:1)
+__device__ __forceinline__ float lane_prev(float v, float first) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, first), __builtin_bit_cast(int, v),
+                                                                 0x138, 0xF, 0xF, false));
+}
+__device__ __forceinline__ float lane_next(float v, float last) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, last), __builtin_bit_cast(int, v),
+                                                                 0x130, 0xF, 0xF, false));
 }
 
-__global__ void __launch_bounds__(64) ts_dtw_wave_kernel(const MzTs p) {
+template <int NW>
+__global__ void __launch_bounds__(64 * NW, 1) ts_dtw_wave_kernel(const MzTs p) {
 #if defined(__HIP_DEVICE_COMPILE__)
-    __shared__ unsigned char moves[(DTW_WAVE_ND + DTW_PF) * 64];  // [diagonal][lane], whole rounds of DTW_PF
-    __shared__ int first[257];                         // per row; [R + 1]: the first token row's offset
-    typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
-    const int c = blockIdx.x, R = p.rc[c].x, C = p.rc[c].y, lane = threadIdx.x;
+    // moves of 32 diagonals of a row: diagonal 2 + 32 g + k at bit 31 - k of x (diagonal move) and y (up); none: left
+    __shared__ uint2 moves[2 * DTW_NCH][64 * NW];
+    __shared__ float edge[NW][4 * DTW_CH];  // the last row of each wave, by diagonal modulo 256
+    __shared__ int first[64 * NW + 2];      // per row; [R + 1]: the first token row's offset
+    const int c = blockIdx.x, R = p.rc[c].x, C = p.rc[c].y, tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     float* out = p.out + (long)c * p.out_stride;
     if (R <= 0) return;
     if (C <= 0) {
-        for (int k = lane; k < R; k += 64) out[k] = 0.f;
+        for (int k = tid; k < R; k += 64 * NW) out[k] = 0.f;
         return;
     }
-    const int ld = p.ldd, nd = R + C + 1;
-    // reads past the clip's cost table return zeros (the descriptor's range check); rows past R are never used
+    const int row = tid + 1, nch = (R + C - 1 + DTW_CH - 1) / DTW_CH;
     const __amdgpu_buffer_rsrc_t rc = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<float*>(p.cost + c * p.diag_stride), (short)0, (int)(p.diag_stride * 4), 0x00020000);
-    auto load = [&](int d) {
-        return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rc, (unsigned)((d * ld + 4 * lane) * 4),
-                                                                                0, 0));
+    // the chunk's costs of this row, one register per diagonal: the diagonal (none past the table's last) in the
+    // scalar offset; rows past R, and the cells left of the table (column <= 0: only in the wave's first chunk), read
+    // zero through the range check
+    float cost[2][DTW_CH];
+    auto load = [&](int ch, float(&x)[DTW_CH]) {
+        const int d0 = 2 + ch * DTW_CH;
+        const bool edge_cells = ch <= wave;
+#pragma unroll
+        for (int k = 0; k < DTW_CH; k++) {
+            const int d = min(d0 + k, R + C);
+            const bool on = row <= R && !(edge_cells && d0 + k <= row);
+            x[k] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rc, on ? (unsigned)row * 4u : 0x80000000u,
+                                                                                  d * p.ldd * 4, 0));
+        }
     };
-    u32x4 ring[DTW_PF];
+    // Every cell of a diagonal is computed, in or out of the table: a cell outside (row past R, column past C) feeds only
+    // cells outside, and cells left of column 1 stay +inf, as column 0 and row 0 are (but for the 0 at (0, 0), the
+    // value up and left of the first cell).
+    float left = INFINITY, up2 = tid == 0 ? 0.f : INFINITY;
+    auto chunk = [&](int ch, const float(&x)[DTW_CH]) {
+        const int d0 = 2 + ch * DTW_CH;
+        float in = wave ? edge[wave ? wave - 1 : 0][(d0 - 1 + lane) & (4 * DTW_CH - 1)] : INFINITY, sent = 0.f;
 #pragma unroll
-    for (int k = 0; k < DTW_PF; k++) ring[k] = load(k);
-    float D1[4], D2[4];  // diagonals d - 1 and d - 2 of rows 4 lane + r
+        for (int h = 0; h < 2; h++) {
+            unsigned m0 = 0, m1 = 0;
 #pragma unroll
-    for (int r = 0; r < 4; r++) D1[r] = D2[r] = INFINITY;
-    // Every cell of a diagonal is computed, in or out of the table: a cell outside (row past R, column past C or
-    // below 0) feeds only cells outside, and the walk back reads moves of cells inside only, forcing the edges' moves
-    // itself, so no cell needs a range test and the choice is branch free. Row 0 is 0 at (0, 0) and +inf after;
-    // column 0 (i == d) is +inf. The moves of rows 4 lane .. 4 lane + 3 pack into one byte.
-    float up2 = INFINITY;  // lane_prev of diagonal d - 2's row 4 lane + 3, carried from the diagonal before
-    const bool lane0 = lane == 0;
-    const int m16 = -(lane == 16), m32 = -(lane == 32), m48 = -(lane == 48);
-    const LaneMasks lm{~(m16 | m32 | m48), m16, m32, m48};
-    // whole rounds of DTW_PF diagonals: the ones past the table are outside cells too
-    const int ndr = (nd + DTW_PF - 1) / DTW_PF * DTW_PF;
-    for (int d0 = 0; d0 < ndr; d0 += DTW_PF) {
-#pragma unroll
-        for (int k = 0; k < DTW_PF; k++) {
-            const int d = d0 + k;
-            const u32x4 cw = ring[k];
-            ring[k] = load(d + DTW_PF);
-            const float up1 = lane_prev(D1[3], lm);  // row 4 lane - 1 at d - 1 (lane 0: unused)
-            float nv[4];
-            unsigned bits = 0;
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const float c0 = r ? D2[r - 1] : up2, c1 = r ? D1[r - 1] : up1, c2 = D1[r];
-                // the reference's comparisons as written (align.rs:77-83), so a NaN cost (a NaN or infinite
-                // z-score in half mode) picks the same move as the host routine and ts_dtw_kernel: fminf would
-                // drop the NaN operand
-                const bool t0 = (c0 < c1) & (c0 < c2), t1 = (c1 < c0) & (c1 < c2);
-                const float m = t0 ? c0 : t1 ? c1 : c2;
+            for (int k = 0; k < 32; k++) {
+                const float up1 = lane_prev(left, in);
+                in = lane_next(in, in);
+                // the reference's comparisons as written (align.rs:77-83), so a NaN cost (a NaN or infinite z-score in
+                // half mode) picks the same move as the host routine and ts_dtw_kernel: fminf would drop the NaN
+                const bool t0 = (up2 < up1) & (up2 < left), t1 = (up1 < up2) & (up1 < left);
+                const float m = t0 ? up2 : t1 ? up1 : left;
                 // ts_dtw_kernel's fp64 -x + m rounded to fp32 equals the fp32 m - x: a sum rounded first to 53 bits
                 // and then to 24 rounds as if once, since 53 >= 2 x 24 + 2 (Figueroa, 1995)
-                float v = m - __uint_as_float(cw[r]);
-                v = 4 * lane + r == d ? INFINITY : v;
-                if (r == 0) v = lane0 ? (d == 0 ? 0.f : INFINITY) : v;
-                nv[r] = v;
-                bits |= (t0 ? 0u : t1 ? 1u : 2u) << (2 * r);
+                left = m - x[32 * h + k];
+                up2 = up1;
+                m0 = 2 * m0 + (t0 ? 1u : 0u);
+                m1 = 2 * m1 + (t1 ? 1u : 0u);
+                sent = lane_next(sent, left);
             }
-            up2 = up1;
+            moves[2 * ch + h][tid] = make_uint2(m0, m1);
+        }
+        edge[wave][(d0 + lane) & (4 * DTW_CH - 1)] = sent;
+    };
+    // wave w's chunk s - w at step s; its chunks before w hold no cell of the table
+    const bool live = 64 * wave < R;
+    if (live) load(wave, cost[0]);
+    for (int s = 0; s < nch + NW - 1; s += 2) {
 #pragma unroll
-            for (int r = 0; r < 4; r++) {
-                D2[r] = D1[r];
-                D1[r] = nv[r];
+        for (int b = 0; b < 2; b++) {
+            const int ch = s + b - wave;
+            if (live && ch >= wave && ch < nch) {
+                // (the chunk parity of a wave is that of s - 2 wave: buffer b)
+                if (ch + 1 < nch) load(ch + 1, cost[(b + 1) & 1]);
+                chunk(ch, cost[b]);
             }
-            moves[d * 64 + lane] = (unsigned char)bits;
+            lds_barrier();
         }
     }
     __syncthreads();
-    if (lane == 0) {
-        // at most R + C moves from (R, C) to (0, 0); row 0 moves left and column 0 up, as the table's edges do
+    if (tid == 0) {
+        // back from (R, C): in row i the path runs left to the last cell at or before this one whose move is another
+        // (column 0 if there is none), which is the row's first cell, then up or diagonally
         int i = R, j = C;
-        bool row0 = false;
-        for (int n = 0; n < R + C && (i > 0 || j > 0); n++) {
+        while (i > 0 && j > 0) {
+            int q = i + j - 2, d = -1;  // diagonal - 2
+            uint2 w;
+            do {
+                w = moves[q >> 5][i - 1];
+                const unsigned any = (w.x | w.y) >> (31 - (q & 31)) << (31 - (q & 31));
+                d = any ? (q | 31) - (__ffs(any) - 1) : -1;
+                q = (q & ~31) - 1;
+            } while (d < 0 && q >= i - 1);
+            j = d < 0 ? 0 : d + 2 - i;
+            if (j < 1) j = 0;
             first[i] = j - 1;
-            row0 |= i == 0;
-            unsigned t = (moves[(i + j) * 64 + (i >> 2)] >> (2 * (i & 3))) & 3u;
-            if (i == 0) t = 2;
-            else if (j == 0) t = 1;
-            if (t == 0) {
-                i--;
-                j--;
-            } else if (t == 1) {
-                i--;
-            } else {
-                j--;
-            }
+            if (j > 0 && (w.x >> (31 - (d & 31)) & 1)) j--;
+            i--;
         }
+        for (; i > 0; i--) first[i] = -1;  // column 0: up
+        first[0] = 0;
         // the token rows start at text index -1 when the path ran along row 0, else at 0
-        first[R + 1] = row0 ? 0 : 1;
+        first[R + 1] = j > 0 ? 0 : 1;
     }
     __syncthreads();
     const int r0 = first[R + 1];  // one start per row
 #pragma unroll 1
-    for (int n = lane; n < R; n += 64) out[n] = (float)((double)first[r0 + n] * 0.02);
+    for (int n = tid; n < R; n += 64 * NW) out[n] = (float)((double)first[r0 + n] * 0.02);
 #endif
 }
 
 }  // namespace
 
-// 3 diagonals, the first-column table and 2 chunks of DTW_CH diagonals of costs, ld = rmax + 1 floats each
-size_t mz_ts_lds_bytes(int rmax) { return ((size_t)(rmax + 1) * 4 + 2 * (((size_t)DTW_CH * (rmax + 1) + 63) & ~(size_t)63)) * 4; }
+// 3 diagonals, the first-column table and 2 chunks of DTW_STAGE diagonals of costs, ld = rmax + 1 floats each
+size_t mz_ts_lds_bytes(int rmax) { return ((size_t)(rmax + 1) * 4 + 2 * (((size_t)DTW_STAGE * (rmax + 1) + 63) & ~(size_t)63)) * 4; }
 
 hipError_t mz_ts_launch(hipStream_t s, const MzTs& p, int n) {
     if (n <= 0) return hipSuccess;
@@ -487,9 +496,11 @@ hipError_t mz_ts_launch(hipStream_t s, const MzTs& p, int n) {
         else
             hipLaunchKernelGGL(ts_cost_kernel<0>, gc, dim3(256), 0, s, p);
     }
-    // the wave kernel loads rows 4 lane .. 4 lane + 3 of a diagonal as one aligned 16-byte group: ldd % 4 == 0
-    if (p.rmax <= 255 && p.ldd % 4 == 0 && p.rmax + p.cols_full + 1 <= DTW_WAVE_ND && p.diag_stride * 4 < (1L << 31)) {
-        hipLaunchKernelGGL(ts_dtw_wave_kernel, dim3(n), dim3(64), 0, s, p);
+    // the wave kernel: at most 256 rows, and the moves of every diagonal in LDS
+    if (p.rmax <= 256 && p.rmax + p.cols_full - 1 <= DTW_NCH * DTW_CH && p.diag_stride * 4 < (1L << 31)) {
+        if (p.rmax <= 64) hipLaunchKernelGGL(ts_dtw_wave_kernel<1>, dim3(n), dim3(64), 0, s, p);
+        else if (p.rmax <= 128) hipLaunchKernelGGL(ts_dtw_wave_kernel<2>, dim3(n), dim3(128), 0, s, p);
+        else hipLaunchKernelGGL(ts_dtw_wave_kernel<4>, dim3(n), dim3(256), 0, s, p);
         return hipGetLastError();
     }
     int nt = ((p.rmax + 1 + 63) / 64) * 64;

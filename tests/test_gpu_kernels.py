@@ -505,6 +505,27 @@ def test_timestamps_device_row_limits(ctx, rows, cols):
                                       err_msg=f"clip {c}")
 
 
+@pytest.mark.parametrize("rows,cols,heads", [([64, 63, 1], [1500, 1, 130], 1), ([65, 64, 2], [1500, 63, 65], 3),
+                                             ([129, 128, 65], [1500, 1500, 1499], 2), ([256, 193, 192], [1500, 64, 1500], 2)])
+def test_timestamps_device_wave_borders(ctx, rows, cols, heads):
+    """Rows at the borders of the DTW's waves (64 rows each, one to four of them), tables of less than one chunk of
+    diagonals and of a whole number of them, a NaN in one column of one clip: identical floats to the host routine."""
+    from mimizuku_amd import transcribe
+    rng = np.random.default_rng(sum(rows) + sum(cols))
+    full, rmax = 1500, max(rows)
+    for half in (True, False):
+        w = softmax_rows(rng, (len(rows), rmax, heads, full))
+        if half:
+            w[2, 0::2, :, 40] = 0.0
+            w[2, 1::2, :, 40] = 2e5
+        dw = ctx.upload_new(w)
+        got = transcribe.jump_times_device(ctx, dw, rmax * heads * full, rows, cols, heads, full, 7, half)
+        for c in range(len(rows)):
+            np.testing.assert_array_equal(got[c], transcribe.jump_times(w[c, :rows[c]], cols[c], 7, half),
+                                          err_msg=f"clip {c} ({rows[c]} x {cols[c]}, half {half})")
+        ctx.free(dw)
+
+
 def test_timestamps_device_nan_costs(ctx):
     """A column whose values overflow fp16 (0 and 2e5 alternating: mean and deviation round to inf, z = inf / inf)
     gives NaN DTW costs in half mode. The DTW must then choose its moves with the reference's comparisons as written
