@@ -155,84 +155,158 @@ __global__ void __launch_bounds__(256) ts_stats4_kernel(const MzTs p) {
 }
 
 // One workgroup per tile of COST_RT rows x COST_CT columns of a clip. Per head, the tile's z-scores (with the window's
-// reflect-padded halo) are computed once into LDS; each cell takes the median of its window from there, summed over
-// heads in head order. The tile's cells then leave diagonal by diagonal: the cells of one anti-diagonal within the
-// tile are consecutive rows, so each diagonal's run is one contiguous store. W = 7: the window unrolled into registers
-// (a sorting network); W = 0: any odd width up to MZ_TS_MAX_WIDTH (insertion sort).
+// reflect-padded halo) are computed once into LDS, the next head's weights already requested; each thread then takes the
+// medians of eight adjacent cells, summed over heads in head order. The tile's cells leave diagonal by diagonal: the
+// cells of one anti-diagonal within the tile are consecutive rows, so each diagonal's run is one contiguous store.
+// W = 7: median of the two outer triples and the middle value. With both triples sorted, it is the middle one of the larger
+// low, the middle of the three middles and the smaller high (the 3 x 3 rule for the median of nine, the third triple being
+// -inf, the middle value, +inf), and a triple serves two windows: 8.5 min / med3 / max per cell where a sorting network
+// took 48 compares and selects. W = 0: any odd width up to MZ_TS_MAX_WIDTH (insertion sort). 32 clips x 220 rows x 1500
+// columns x 10 heads: 285 -> 109 us, one clip of 41 rows x 6 heads 40 -> 13.
 constexpr int COST_RT = 32, COST_CT = 64, COST_HALO = MZ_TS_MAX_WIDTH - 1;
 
 template <int W>
 __global__ void __launch_bounds__(256) ts_cost_kernel(const MzTs p) {
+    // row strides: 79 floats puts the eight cells of 8 x 8 threads in 64 banks, 66 a diagonal's 32 rows in 32
     __shared__ float zt[COST_RT][COST_CT + COST_HALO + 1];
-    __shared__ float val[COST_RT][COST_CT + 2];  // row stride 66: a diagonal's 32 rows fall in 32 different banks
+    __shared__ float val[COST_RT][COST_CT + 2];
+    __shared__ int nan_seen[2];
     const int c = blockIdx.z, i0 = blockIdx.y * COST_RT, j0 = blockIdx.x * COST_CT, tid = threadIdx.x;
     const int R = p.rc[c].x, C = p.rc[c].y;
     if (i0 >= R || j0 >= C) return;
-    const int width = W ? W : p.width, pad = width >> 1, span = COST_CT + 2 * pad;
-    // the median phase: column jl = tid % 64 of rows il = tid / 64 + 4 k
-    const int jl = tid & 63, ib = tid >> 6;
-    float acc[COST_RT / 4];
+    const int width = W ? W : p.width, pad = width >> 1, halo = 2 * pad;
+    if (tid < 2) nan_seen[tid] = 0;
+    lds_barrier();
+    // the z phase: tile column cl = tid % 64 of rows tid / 64 + 4 k, then the halo columns 64 .. 64 + halo - 1, NH of them
+    // per thread. Tile column cl stands for time j0 + cl - pad, reflected into 0 .. C - 1 as the window reads it
+    // (columns of cells past C, whose values are never stored, are clamped into range instead).
+    constexpr int NM = COST_RT / 4, NH = W ? 1 : (COST_RT * COST_HALO + 255) / 256;
+    static_assert(COST_RT * 6 <= 256, "one halo element per thread at width 7");
+    auto time_of = [&](int cl) {
+        int t = j0 + cl - pad;
+        if (t < 0) t = -t;
+        if (t >= C) t = 2 * (C - 1) - t;
+        return t < 0 ? 0 : t > C - 1 ? C - 1 : t;
+    };
+    const int zl = tid & 63, zi = tid >> 6, zt0 = time_of(zl);
+    int hi[NH], hc[NH], ht[NH];
 #pragma unroll
-    for (int k = 0; k < COST_RT / 4; k++) acc[k] = 0.f;
-    for (int a = 0; a < p.heads; a++) {
-        const float* mu = p.mean + ((long)c * p.heads + a) * p.cols_full;
-        const float* sd = p.sd + ((long)c * p.heads + a) * p.cols_full;
-        // z of tile column cl - pad (reflected into 0 .. C - 1 as the window reads it; columns of cells past C,
-        // whose values are never stored, are clamped into range instead)
-        for (int e = tid; e < COST_RT * span; e += 256) {
-            const int il = e / span, cl = e - il * span, i = i0 + il;
-            int t = j0 + cl - pad;
-            if (t < 0) t = -t;
-            if (t >= C) t = 2 * (C - 1) - t;
-            t = t < 0 ? 0 : t > C - 1 ? C - 1 : t;
-            float z = 0.f;
-            if (i < R) {
-                const float x = p.w[c * p.clip_stride + ((long)i * p.heads + a) * p.cols_full + t];
-                const float sv = sd[t];
-                if (sv > 0.f) z = p.half ? rh(rh(x - mu[t]) / sv) : (x - mu[t]) / sv;
-            }
-            zt[il][cl] = z;
+    for (int k = 0; k < NH; k++) {
+        const int e = tid + 256 * k;
+        hi[k] = halo ? e / max(halo, 1) : COST_RT;
+        hc[k] = COST_CT + e - hi[k] * halo;
+        ht[k] = time_of(hc[k]);
+    }
+    const float* wc = p.w + c * p.clip_stride;
+    const float *mu = p.mean + (long)c * p.heads * p.cols_full, *sd = p.sd + (long)c * p.heads * p.cols_full;
+    float xm[NM], xh[NH], mm, sm, mh[NH], sh[NH];
+    auto fetch = [&](int a) {
+        const long o = (long)a * p.cols_full;
+        mm = mu[o + zt0];
+        sm = sd[o + zt0];
+#pragma unroll
+        for (int k = 0; k < NM; k++) {
+            const int i = i0 + zi + 4 * k;
+            xm[k] = i < R ? wc[((long)i * p.heads + a) * p.cols_full + zt0] : 0.f;
         }
-        __syncthreads();
 #pragma unroll
-        for (int k = 0; k < COST_RT / 4; k++) {
-            const float* zr = &zt[ib + 4 * k][jl];
-            if (C <= pad) {
-                acc[k] += zr[pad];  // fewer columns than the half width: no filter
-            } else if (W == 7) {
+        for (int k = 0; k < NH; k++) {
+            const int i = i0 + hi[k];
+            const bool on = hi[k] < COST_RT && i < R;
+            mh[k] = on ? mu[o + ht[k]] : 0.f;
+            sh[k] = on ? sd[o + ht[k]] : 0.f;
+            xh[k] = on ? wc[((long)i * p.heads + a) * p.cols_full + ht[k]] : 0.f;
+        }
+    };
+    auto zscore = [&](float x, float m, float s) { return s > 0.f ? (p.half ? rh(rh(x - m) / s) : (x - m) / s) : 0.f; };
+    // the median phase: columns 8 jl .. 8 jl + 7 of row il
+    const int il = tid >> 3, jl = (tid & 7) * 8;
+    float acc[8];
+#pragma unroll
+    for (int q = 0; q < 8; q++) acc[q] = 0.f;
+    fetch(0);
+    for (int a = 0; a < p.heads; a++) {
+        bool nan = false;
+#pragma unroll
+        for (int k = 0; k < NM; k++) {
+            const float z = i0 + zi + 4 * k < R ? zscore(xm[k], mm, sm) : 0.f;
+            nan |= z != z;
+            zt[zi + 4 * k][zl] = z;
+        }
+#pragma unroll
+        for (int k = 0; k < NH; k++)
+            if (hi[k] < COST_RT) {
+                const float z = zscore(xh[k], mh[k], sh[k]);
+                nan |= z != z;
+                zt[hi[k]][hc[k]] = z;
+            }
+        if (__ballot(nan) && (tid & 63) == 0) nan_seen[a & 1] = 1;
+        if (a + 1 < p.heads) fetch(a + 1);
+        lds_barrier();  // (the weights of the next head stay in flight)
+        const bool slow = nan_seen[a & 1] != 0;
+        const float* zr = &zt[il][jl];
+        if (C <= pad) {
+#pragma unroll
+            for (int q = 0; q < 8; q++) acc[q] += zr[q + pad];  // fewer columns than the half width: no filter
+        } else if (W == 7 && !slow) {
+            float z[14], lo[12], md[12], up[12];
+#pragma unroll
+            for (int q = 0; q < 14; q++) z[q] = zr[q];
+#pragma unroll
+            for (int q = 0; q < 12; q++) {
+                lo[q] = fminf(fminf(z[q], z[q + 1]), z[q + 2]);
+                md[q] = __builtin_amdgcn_fmed3f(z[q], z[q + 1], z[q + 2]);
+                up[q] = fmaxf(fmaxf(z[q], z[q + 1]), z[q + 2]);
+            }
+#pragma unroll
+            for (int q = 0; q < 8; q++)
+                acc[q] += __builtin_amdgcn_fmed3f(fmaxf(lo[q], lo[q + 4]),
+                                                  __builtin_amdgcn_fmed3f(md[q], z[q + 3], md[q + 4]),
+                                                  fminf(up[q], up[q + 4]));
+        } else if (W == 7) {
+            // a NaN in the tile (half mode: a z-score that overflowed): min / med3 / max drop it, the network, with the
+            // host routine's comparisons, moves it like any value
+#pragma unroll
+            for (int q = 0; q < 8; q++) {
                 float win[7];
 #pragma unroll
-                for (int q = 0; q < 7; q++) win[q] = zr[q];
-                acc[k] += median7(win);
-            } else {
+                for (int e = 0; e < 7; e++) win[e] = zr[q + e];
+                acc[q] += median7(win);
+            }
+        } else {
+#pragma unroll 1
+            for (int q = 0; q < 8; q++) {
                 float win[MZ_TS_MAX_WIDTH];
-                for (int q = 0; q < width; q++) {
-                    const float v = zr[q];
-                    int r = q - 1;
+                for (int e = 0; e < width; e++) {
+                    const float v = zr[q + e];
+                    int r = e - 1;
                     while (r >= 0 && win[r] > v) {
                         win[r + 1] = win[r];
                         r--;
                     }
                     win[r + 1] = v;
                 }
-                acc[k] += win[pad];
+                const float m = win[pad];
+#pragma unroll
+                for (int x = 0; x < 8; x++) acc[x] += x == q ? m : 0.f;
             }
         }
-        __syncthreads();  // zt is rewritten for the next head
+        lds_barrier();  // zt is rewritten for the next head
+        if (tid == 0) nan_seen[a & 1] = 0;  // (read again, after another barrier, two heads on)
     }
 #pragma unroll
-    for (int k = 0; k < COST_RT / 4; k++) {
-        float v = acc[k] / (float)p.heads;
+    for (int q = 0; q < 8; q++) {
+        float v = acc[q] / (float)p.heads;
         if (p.half) v = rh(v);
-        val[ib + 4 * k][jl] = v;
+        val[il][jl + q] = v;
     }
     __syncthreads();
     // DTW cell (i + 1, j + 1) lies on anti-diagonal i + j + 2: tile diagonal dl = il + jl holds rows il of one run
     float* dst = p.cost + c * p.diag_stride + (long)(i0 + j0 + 2) * p.ldd + (i0 + 1);
-    const int il = tid & 31;
+    const int dr = tid & 31;
     for (int dl = tid >> 5; dl < COST_RT + COST_CT - 1; dl += 8) {
-        const int cl = dl - il;
-        if (cl >= 0 && cl < COST_CT && i0 + il < R && j0 + cl < C) dst[(long)dl * p.ldd + il] = val[il][cl];
+        const int cl = dl - dr;
+        if (cl >= 0 && cl < COST_CT && i0 + dr < R && j0 + cl < C) dst[(long)dl * p.ldd + dr] = val[dr][cl];
     }
 }
 
