@@ -335,8 +335,10 @@ int mz_resample_16k(const float* y, size_t n, int sr, float* out, size_t cap, si
 int mz_mel_tables(int n_mels, float* filters, double* cosb, double* sinb);
 /* Mel::features (src/audio.rs:195-249) of n clips on the device: audio f32 [n][480000] at device address `audio`
  * (16 kHz; samples at or past n_samples[i] read as zero) -> normalised log-mel f32 [n][n_mels][3000] at `mel`;
- * frames[i] (may be null) = 10 ms frames that hold audio. The power spectra equal the reference's bit for bit
- * (double sums in sample order); log10 is the device library's. Synchronous; allocates and frees its scratch. */
+ * frames[i] (may be null) = 10 ms frames that hold audio.
+ * The power spectra are sums in double, rounded to float, as the reference's, but folded by the symmetries of the
+ * transform rather than in sample order; log10 is the device library's. Synchronous; allocates and frees its
+ * scratch. */
 int mz_log_mel(mz_ctx* c, uint64_t audio, const int32_t* n_samples, int n, int n_mels, uint64_t mel, int32_t* frames);
 
 /* ------------------------------------------------------------------ text (src/tok.rs, src/main.rs) */

@@ -176,24 +176,56 @@ extern "C" int mz_resample_16k(const float* y, size_t n, int sr, float* out, siz
     return MZ_OK;
 }
 
+namespace {
+
+// Slaney mel filters up to 8 kHz, as Mel::new (src/audio.rs:161-189) builds them
+struct MelBank {
+    std::vector<double> ff;  // band edges in Hz, n_mels + 2 of them
+    explicit MelBank(int n_mels) : ff(n_mels + 2) {
+        const double m0 = hz_to_mel(0.0), m1 = hz_to_mel(8000.0);
+        for (int i = 0; i < n_mels + 2; i++) ff[i] = mel_to_hz(m0 + (m1 - m0) * (double)i / (double)(n_mels + 1));
+    }
+    float weight(int k, int m) const {
+        const double fq = (double)k * (16000.0 / 2.0) / (double)(MZ_MEL_BINS - 1);
+        const double dn = (fq - ff[m]) / (ff[m + 1] - ff[m]);
+        const double upv = (ff[m + 2] - fq) / (ff[m + 2] - ff[m + 1]);
+        const double enorm = 2.0 / (ff[m + 2] - ff[m]);
+        return (float)(std::max(std::min(dn, upv), 0.0) * enorm);
+    }
+    // the non-zero weights of filter m: first bin | bins << 8 | index of the first weight << 16
+    bool compact(int n_mels, int32_t* meta, float* wts) const {
+        const double hz = (16000.0 / 2.0) / (double)(MZ_MEL_BINS - 1);
+        int n = 0;
+        for (int m = 0; m < n_mels; m++) {
+            // a bin more on either side of the band: its weight decides
+            const int k0 = std::max((int)(ff[m] / hz) - 1, 0), k1 = std::min((int)(ff[m + 2] / hz) + 1, MZ_MEL_BINS - 1);
+            int lo = 0, cnt = 0;
+            const int off = n;
+            for (int k = k0; k <= k1; k++) {
+                const float w = weight(k, m);
+                if (w == 0.f && cnt == 0) continue;
+                if (n >= MZ_MEL_WTS) return false;
+                if (cnt++ == 0) lo = k;
+                wts[n++] = w;
+            }
+            while (cnt > 0 && wts[n - 1] == 0.f) n--, cnt--;
+            meta[m] = lo | cnt << 8 | off << 16;
+        }
+        return true;
+    }
+};
+
+}  // namespace
+
 // Slaney mel filters [201][n_mels] up to 8 kHz and the periodic-Hann-windowed DFT basis [400][201] (cos, sin),
-// as Mel::new (src/audio.rs:161-189) builds them, the basis stored sample-major for the device.
+// as Mel::new (src/audio.rs:161-189) builds them, the basis stored sample-major.
 extern "C" int mz_mel_tables(int n_mels, float* filters, double* cosb, double* sinb) {
     if (n_mels <= 0 || n_mels > 256) return mz_fail(MZ_ERR_ARG, "mz_mel_tables: n_mels %d out of range", n_mels);
     const int NB = MZ_MEL_BINS, NF = MZ_MEL_NFFT;
     if (filters) {
-        const double m0 = hz_to_mel(0.0), m1 = hz_to_mel(8000.0);
-        std::vector<double> ff(n_mels + 2);
-        for (int i = 0; i < n_mels + 2; i++) ff[i] = mel_to_hz(m0 + (m1 - m0) * (double)i / (double)(n_mels + 1));
-        for (int k = 0; k < NB; k++) {
-            const double fq = (double)k * (16000.0 / 2.0) / (double)(NB - 1);
-            for (int m = 0; m < n_mels; m++) {
-                const double dn = (fq - ff[m]) / (ff[m + 1] - ff[m]);
-                const double upv = (ff[m + 2] - fq) / (ff[m + 2] - ff[m + 1]);
-                const double enorm = 2.0 / (ff[m + 2] - ff[m]);
-                filters[(size_t)k * n_mels + m] = (float)(std::max(std::min(dn, upv), 0.0) * enorm);
-            }
-        }
+        const MelBank bank(n_mels);
+        for (int k = 0; k < NB; k++)
+            for (int m = 0; m < n_mels; m++) filters[(size_t)k * n_mels + m] = bank.weight(k, m);
     }
     if (cosb || sinb) {
         for (int j = 0; j < NF; j++) {
@@ -212,43 +244,38 @@ extern "C" int mz_log_mel(mz_ctx* c, uint64_t audio, const int32_t* n_samples, i
                           int32_t* frames) {
     if (!c || !audio || !n_samples || !mel) return mz_fail(MZ_ERR_ARG, "mz_log_mel: null argument");
     if (n <= 0 || n_mels <= 0 || n_mels > 256) return mz_fail(MZ_ERR_ARG, "mz_log_mel: bad sizes");
-    const int NB = MZ_MEL_BINS, NF = MZ_MEL_NFFT, T = MZ_NFR_HOST;
-    std::vector<int32_t> ns(n);
+    std::vector<int32_t> ns(n), meta(n_mels);
+    long live = 0;
     for (int i = 0; i < n; i++) {
         if (n_samples[i] < 0) return mz_fail(MZ_ERR_ARG, "mz_log_mel: negative sample count");
         ns[i] = std::min(n_samples[i], (int32_t)MZ_MEL_NSAMPLES);
-        if (frames) frames[i] = std::min((ns[i] + MZ_MEL_HOP - 1) / MZ_MEL_HOP, T);
+        if (frames) frames[i] = std::min((ns[i] + MZ_MEL_HOP - 1) / MZ_MEL_HOP, MZ_NFR_HOST);
+        live += std::min((ns[i] + MZ_MEL_NFFT / 2 + MZ_MEL_HOP - 1) / MZ_MEL_HOP, MZ_NFR_HOST);
     }
-    std::vector<float> filt((size_t)NB * n_mels);
-    std::vector<double> cb((size_t)NF * NB), sb((size_t)NF * NB);
-    mz_mel_tables(n_mels, filt.data(), cb.data(), sb.data());
-    // scratch: tables, per-clip sample counts, power spectra [n][3000][201], per-clip maxima
-    const size_t bytes_f = filt.size() * 4, bytes_b = cb.size() * 8, bytes_p = (size_t)n * T * NB * 4;
-    char* base = nullptr;
-    const size_t total = bytes_f + 2 * bytes_b + (size_t)n * 4 + bytes_p + (size_t)n * 4 + 1024;
-    if (int r = mz_hip(hipMalloc((void**)&base, total), "hipMalloc")) return r;
+    std::vector<float> wts(MZ_MEL_WTS, 0.f);
+    if (!MelBank(n_mels).compact(n_mels, meta.data(), wts.data()))
+        return mz_fail(MZ_ERR_STATE, "mz_log_mel: more filter weights than %d", MZ_MEL_WTS);
+    // scratch: basis, filters, per-clip sample counts, the workgroups' maxima
     auto align = [](size_t v) { return (v + 255) & ~(size_t)255; };
+    const size_t bytes[5] = {MZ_MEL_BASIS * sizeof(double), wts.size() * 4, meta.size() * 4, (size_t)n * 4,
+                             (size_t)n * MZ_MEL_BLOCKS * 4};
+    size_t total = 0;
+    for (size_t b : bytes) total += align(b);
+    char* base = nullptr;
+    if (int r = mz_hip(hipMalloc((void**)&base, total), "hipMalloc")) return r;
+    char* at[5];
     size_t off = 0;
-    float* d_filt = (float*)(base + off);
-    off = align(off + bytes_f);
-    double* d_cos = (double*)(base + off);
-    off = align(off + bytes_b);
-    double* d_sin = (double*)(base + off);
-    off = align(off + bytes_b);
-    int* d_ns = (int*)(base + off);
-    off = align(off + (size_t)n * 4);
-    float* d_pow = (float*)(base + off);
-    off = align(off + bytes_p);
-    float* d_max = (float*)(base + off);
-    int r = MZ_OK;
-    if (off + (size_t)n * 4 > total) r = mz_fail(MZ_ERR_STATE, "mz_log_mel: scratch layout");
-    if (!r) r = mz_hip(hipMemcpyAsync(d_filt, filt.data(), bytes_f, hipMemcpyHostToDevice, c->stream), "hipMemcpy");
-    if (!r) r = mz_hip(hipMemcpyAsync(d_cos, cb.data(), bytes_b, hipMemcpyHostToDevice, c->stream), "hipMemcpy");
-    if (!r) r = mz_hip(hipMemcpyAsync(d_sin, sb.data(), bytes_b, hipMemcpyHostToDevice, c->stream), "hipMemcpy");
-    if (!r) r = mz_hip(hipMemcpyAsync(d_ns, ns.data(), (size_t)n * 4, hipMemcpyHostToDevice, c->stream), "hipMemcpy");
+    for (int i = 0; i < 5; i++) {
+        at[i] = base + off;
+        off += align(bytes[i]);
+    }
+    int r = mz_hip(hipMemcpyAsync(at[1], wts.data(), bytes[1], hipMemcpyHostToDevice, c->stream), "hipMemcpy");
+    if (!r) r = mz_hip(hipMemcpyAsync(at[2], meta.data(), bytes[2], hipMemcpyHostToDevice, c->stream), "hipMemcpy");
+    if (!r) r = mz_hip(hipMemcpyAsync(at[3], ns.data(), bytes[3], hipMemcpyHostToDevice, c->stream), "hipMemcpy");
     if (!r) {
-        MzMel p{(const float*)(uintptr_t)audio, d_ns, d_cos, d_sin, d_filt, d_pow, d_max, (float*)(uintptr_t)mel, n, n_mels};
-        r = mz_hip(mz_log_mel_launch(c->stream, p), "log-mel");
+        const MzMel p{(const float*)(uintptr_t)audio, (const int*)at[3], (const int*)at[2], (const float*)at[1],
+                      (double*)at[0], (float*)at[4], (float*)(uintptr_t)mel, n, n_mels};
+        r = mz_hip(mz_log_mel_launch(c->stream, p, live), "log-mel");
     }
     const int rs = mz_hip(hipStreamSynchronize(c->stream), "hipStreamSynchronize");
     hipFree(base);

@@ -197,18 +197,21 @@ int mz_ts_scratch_setup(int device);
 #define MZ_MEL_BINS 201          // MZ_MEL_NFFT / 2 + 1
 #define MZ_MEL_NSAMPLES 480000   // 30 s at 16 kHz
 #define MZ_NFR_HOST 3000         // log-mel frames of 30 s
-// audio [n][480000] f32 (samples at or past ns[c] read as zero), tables from mz_mel_tables (cosb / sinb
-// [400][201] windowed DFT basis, filt [201][n_mels]); pow [n][3000][201] and mx [n] are scratch;
+#define MZ_MEL_BASIS (4 * 7 * 26 * 64 + 256)  // doubles of the folded DFT basis and the window
+#define MZ_MEL_WTS 512           // filter weights: a bin lies in at most two filters
+#define MZ_MEL_BLOCKS 188        // workgroups of a clip (16 frames each)
+// audio [n][480000] f32 (samples at or past ns[c] read as zero); meta [n_mels] and wts the filters' non-zero weights
+// (first bin | bins << 8 | first weight << 16); basis [MZ_MEL_BASIS] and mx [n][MZ_MEL_BLOCKS] are scratch;
 // mel [n][n_mels][3000] the normalised log-mel
 struct MzMel {
     const float* audio;
     const int* ns;
-    const double* cosb;
-    const double* sinb;
-    const float* filt;
-    float* pow;
+    const int* meta;
+    const float* wts;
+    double* basis;
     float* mx;
     float* mel;
     int n, n_mels;
 };
-hipError_t mz_log_mel_launch(hipStream_t s, const MzMel& p);
+// frames: those of all clips that hold audio
+hipError_t mz_log_mel_launch(hipStream_t s, const MzMel& p, long frames);

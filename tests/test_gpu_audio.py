@@ -80,3 +80,40 @@ def test_log_mel_matches_transformers(ctx):
         got, frames = log_mel(ctx, [y], int(fx["n_mels"]))
         assert frames[0] == int(fx["frames"])
         assert np.abs(got[0][:, fx["cols"]] - fx["features"]).max() < 2e-5, name
+
+
+@pytest.mark.parametrize("n_mels,lengths", [(1, [400, 161]), (40, [16000 * 12 + 77, 2401, 2400]), (256, [NS, 16 * 160, 41 * 160]),
+                                            (80, [NS] * 6)])
+def test_log_mel_tiles_and_widths(ctx, n_mels, lengths):
+    """Frame counts at the borders of the 16- and 32-frame tiles (six full clips take the larger), the fewest and the
+    most filters the entry point takes."""
+    rng = np.random.default_rng(n_mels + len(lengths))
+    clips = [(0.2 * rng.standard_normal(k)).astype(np.float32) for k in lengths]
+    got, frames = log_mel(ctx, clips, n_mels)
+    tables = A.mel_tables(n_mels)
+    for i in sorted({0, len(clips) // 2, len(clips) - 1}):
+        ref, fr = A.features(clips[i], n_mels, tables)
+        assert frames[i] == fr
+        assert np.abs(got[i] - ref).max() <= 1e-6, (i, lengths[i])
+
+
+def test_log_mel_unaligned_output_and_a_nan_sample(ctx):
+    """An output address that is only 4-byte aligned; and a NaN sample, whose frames have no finite power: every filter's
+    sum is NaN there, which the floor turns into -10 (before the clamp), and no other frame changes."""
+    rng = np.random.default_rng(3)
+    y = (0.2 * rng.standard_normal(NS)).astype(np.float32)
+    ref, _ = log_mel(ctx, [y], 80)
+    z = y.copy()
+    z[100000] = np.nan
+    d_audio = ctx.upload_new(z[None])
+    d_mel = ctx.alloc(80 * 3000 * 4 + 16)
+    ns = np.array([NS], np.int32)
+    L.check(L.lib().mz_log_mel(ctx.h, d_audio, ns.ctypes.data_as(C.c_void_p), 1, 80, d_mel + 4, None))
+    got = ctx.download(d_mel + 4, (80, 3000), np.float32)
+    t = np.arange(3000)
+    hit = (160 * t - 200 < 100000) & (100000 < 160 * t + 200)  # (the first sample of a frame has weight 0)
+    assert np.ptp(got[:, hit]) == 0 and got[0, hit][0] <= ref[0].min()
+    edge = (160 * t - 200 <= 100000) & (100000 < 160 * t + 200)
+    np.testing.assert_array_equal(got[:, ~edge], ref[0][:, ~edge])
+    ctx.free(d_audio)
+    ctx.free(d_mel)
