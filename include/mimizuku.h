@@ -271,7 +271,9 @@ int mz_transcribe_collect(mz_engine* e, const int32_t* frames, int n, const int3
  * src/align.rs:8-63; the reference runs it on the host after downloading the weights, transcribe.rs:150-158).
  * Clip c's alignment-head weights are rows[c] rows of heads x cols_full floats at device address
  * w + c * clip_stride * 4, cropped to cols[c] frames; its times go to host out[c * out_stride + k], k < rows[c].
- * Odd width <= 15. Allocates and frees its own device scratch; synchronous on the context's stream. */
+ * Odd width <= 15. Synchronous on the context's stream. Its device and pinned host scratch is kept in the context from
+ * call to call, up to 192 MiB and 4 MiB, and freed by mz_ctx_free; a call that needs more, or that runs while another
+ * thread's uses it, allocates and frees its own. */
 int mz_jump_times_device(mz_ctx* c, uint64_t w, int64_t clip_stride, int n, const int32_t* rows, const int32_t* cols,
                          int heads, int cols_full, int width, int half, float* out, int64_t out_stride);
 
@@ -337,8 +339,8 @@ int mz_mel_tables(int n_mels, float* filters, double* cosb, double* sinb);
  * (16 kHz; samples at or past n_samples[i] read as zero) -> normalised log-mel f32 [n][n_mels][3000] at `mel`;
  * frames[i] (may be null) = 10 ms frames that hold audio.
  * The power spectra are sums in double, rounded to float, as the reference's, but folded by the symmetries of the
- * transform rather than in sample order; log10 is the device library's. Synchronous; allocates and frees its
- * scratch. */
+ * transform rather than in sample order; log10 is the device library's. Synchronous; its
+ * scratch is the context's (see mz_jump_times_device). */
 int mz_log_mel(mz_ctx* c, uint64_t audio, const int32_t* n_samples, int n, int n_mels, uint64_t mel, int32_t* frames);
 
 /* ------------------------------------------------------------------ text (src/tok.rs, src/main.rs) */

@@ -244,40 +244,34 @@ extern "C" int mz_log_mel(mz_ctx* c, uint64_t audio, const int32_t* n_samples, i
                           int32_t* frames) {
     if (!c || !audio || !n_samples || !mel) return mz_fail(MZ_ERR_ARG, "mz_log_mel: null argument");
     if (n <= 0 || n_mels <= 0 || n_mels > 256) return mz_fail(MZ_ERR_ARG, "mz_log_mel: bad sizes");
-    std::vector<int32_t> ns(n), meta(n_mels);
+    for (int i = 0; i < n; i++)
+        if (n_samples[i] < 0) return mz_fail(MZ_ERR_ARG, "mz_log_mel: negative sample count");
+    // uploaded in one piece: filter weights, filters, per-clip sample counts; then the kernels' scratch: the basis and the
+    // workgroups' maxima
+    auto align = [](size_t v) { return (v + 255) & ~(size_t)255; };
+    const size_t o_meta = MZ_MEL_WTS * 4, o_ns = o_meta + 256 * 4, bytes_up = align(o_ns + (size_t)n * 4);
+    const size_t o_max = bytes_up + align(MZ_MEL_BASIS * sizeof(double));
+    if (int r = mz_hip(hipSetDevice(c->device), "hipSetDevice")) return r;
+    MzScratch scratch(c, o_max + (size_t)n * MZ_MEL_BLOCKS * 4, bytes_up);
+    if (scratch.status()) return scratch.status();
+    float* wts = (float*)scratch.pin;
+    int32_t *meta = (int32_t*)(scratch.pin + o_meta), *ns = (int32_t*)(scratch.pin + o_ns);
+    memset(scratch.pin, 0, o_ns);
+    if (!MelBank(n_mels).compact(n_mels, meta, wts))
+        return mz_fail(MZ_ERR_STATE, "mz_log_mel: more filter weights than %d", MZ_MEL_WTS);
     long live = 0;
     for (int i = 0; i < n; i++) {
-        if (n_samples[i] < 0) return mz_fail(MZ_ERR_ARG, "mz_log_mel: negative sample count");
         ns[i] = std::min(n_samples[i], (int32_t)MZ_MEL_NSAMPLES);
         if (frames) frames[i] = std::min((ns[i] + MZ_MEL_HOP - 1) / MZ_MEL_HOP, MZ_NFR_HOST);
         live += std::min((ns[i] + MZ_MEL_NFFT / 2 + MZ_MEL_HOP - 1) / MZ_MEL_HOP, MZ_NFR_HOST);
     }
-    std::vector<float> wts(MZ_MEL_WTS, 0.f);
-    if (!MelBank(n_mels).compact(n_mels, meta.data(), wts.data()))
-        return mz_fail(MZ_ERR_STATE, "mz_log_mel: more filter weights than %d", MZ_MEL_WTS);
-    // scratch: basis, filters, per-clip sample counts, the workgroups' maxima
-    auto align = [](size_t v) { return (v + 255) & ~(size_t)255; };
-    const size_t bytes[5] = {MZ_MEL_BASIS * sizeof(double), wts.size() * 4, meta.size() * 4, (size_t)n * 4,
-                             (size_t)n * MZ_MEL_BLOCKS * 4};
-    size_t total = 0;
-    for (size_t b : bytes) total += align(b);
-    char* base = nullptr;
-    if (int r = mz_hip(hipMalloc((void**)&base, total), "hipMalloc")) return r;
-    char* at[5];
-    size_t off = 0;
-    for (int i = 0; i < 5; i++) {
-        at[i] = base + off;
-        off += align(bytes[i]);
-    }
-    int r = mz_hip(hipMemcpyAsync(at[1], wts.data(), bytes[1], hipMemcpyHostToDevice, c->stream), "hipMemcpy");
-    if (!r) r = mz_hip(hipMemcpyAsync(at[2], meta.data(), bytes[2], hipMemcpyHostToDevice, c->stream), "hipMemcpy");
-    if (!r) r = mz_hip(hipMemcpyAsync(at[3], ns.data(), bytes[3], hipMemcpyHostToDevice, c->stream), "hipMemcpy");
+    char* d = scratch.dev;
+    int r = mz_hip(hipMemcpyAsync(d, scratch.pin, bytes_up, hipMemcpyHostToDevice, c->stream), "hipMemcpy");
     if (!r) {
-        const MzMel p{(const float*)(uintptr_t)audio, (const int*)at[3], (const int*)at[2], (const float*)at[1],
-                      (double*)at[0], (float*)at[4], (float*)(uintptr_t)mel, n, n_mels};
+        const MzMel p{(const float*)(uintptr_t)audio, (const int*)(d + o_ns), (const int*)(d + o_meta), (const float*)d,
+                      (double*)(d + bytes_up), (float*)(d + o_max), (float*)(uintptr_t)mel, n, n_mels};
         r = mz_hip(mz_log_mel_launch(c->stream, p, live), "log-mel");
     }
     const int rs = mz_hip(hipStreamSynchronize(c->stream), "hipStreamSynchronize");
-    hipFree(base);
     return r ? r : rs;
 }

@@ -21,6 +21,7 @@
 
 #include <algorithm>
 #include <mutex>
+#include <vector>
 
 #include "../../include/mimizuku.h"
 #include "mz_common.h"
@@ -640,10 +641,11 @@ extern "C" int mz_jump_times_device_noalloc(mz_ctx* c, uint64_t w, int64_t clip_
     // scratch of k clips whose longest has rmax rows: (rows, columns), column statistics, DTW cost and trace, times
     auto need = [&](int k, int rmax) {
         return up256((size_t)k * sizeof(int2)) + 2 * up256((size_t)k * heads * cols_full * 4) +
-               up256((size_t)k * mz_ts_diag_stride(rmax, cols_full) * 5) + up256((size_t)k * out_stride * 4);
+               up256((size_t)k * mz_ts_diag_stride(rmax, cols_full) * 5) + up256((size_t)k * rmax * 4);
     };
     // the clips go through the array in chunks of at most MZ_TS_NOALLOC_CHUNK that fit in it, one after the other
     int2 rc[MZ_TS_NOALLOC_CHUNK];
+    std::vector<float> times;
     for (int c0 = 0; c0 < n;) {
         int k = 0, rmax = 0;
         while (c0 + k < n && k < MZ_TS_NOALLOC_CHUNK && need(k + 1, std::max(rmax, (int)rows[c0 + k])) <= MZ_TS_SCRATCH_BYTES) {
@@ -678,19 +680,21 @@ extern "C" int mz_jump_times_device_noalloc(mz_ctx* c, uint64_t w, int64_t clip_
         p.trace = (signed char*)(p.cost + (size_t)k * ds);
         p.diag_stride = ds;
         p.ldd = mz_ts_ldd(rmax);
-        p.out = (float*)carve((size_t)k * out_stride * 4);
-        p.out_stride = out_stride;
+        p.out = (float*)carve((size_t)k * rmax * 4);
+        p.out_stride = rmax;
         int r = mz_hip(hipMemcpyAsync((void*)p.rc, rc, (size_t)k * sizeof(int2), hipMemcpyHostToDevice, c->stream),
                        "upload");
         if (!r) r = mz_hip(mz_ts_launch(c->stream, p, k), "timestamp kernels");
-        for (int i = 0; i < k && !r; i++)
-            if (rows[c0 + i] > 0)
-                r = mz_hip(hipMemcpyAsync(out + (size_t)(c0 + i) * out_stride, p.out + (size_t)i * out_stride,
-                                          (size_t)rows[c0 + i] * 4, hipMemcpyDeviceToHost, c->stream),
-                           "download");
+        // the chunk's times in one copy (one per clip took longer than the kernels of a large chunk)
+        times.resize((size_t)k * rmax);
+        if (!r && rmax > 0)
+            r = mz_hip(hipMemcpyAsync(times.data(), p.out, times.size() * 4, hipMemcpyDeviceToHost, c->stream), "download");
         // the next chunk reuses the array (and rc): wait for this one
-        if (!r) r = mz_hip(hipStreamSynchronize(c->stream), "hipStreamSynchronize");
-        if (r) return r;
+        const int rs = mz_hip(hipStreamSynchronize(c->stream), "hipStreamSynchronize");
+        if (r || rs) return r ? r : rs;
+        for (int i = 0; i < k; i++)
+            std::copy(times.data() + (size_t)i * rmax, times.data() + (size_t)i * rmax + rows[c0 + i],
+                      out + (size_t)(c0 + i) * out_stride);
         c0 += k;
     }
     return MZ_OK;

@@ -64,6 +64,8 @@ extern "C" int mz_ctx_free(mz_ctx* c) {
     hipSetDevice(c->device);
     hipStreamSynchronize(c->stream);
     for (void* p : c->allocs) hipFree(p);
+    hipFree(c->scratch_dev);
+    hipHostFree(c->scratch_pin);
     hipStreamDestroy(c->stream);
     delete c;
     return MZ_OK;
@@ -77,6 +79,43 @@ int mz_ctx_alloc(mz_ctx* c, size_t bytes, void** p) {
     if (int r = mz_hip(hipStreamSynchronize(c->stream), "hipStreamSynchronize")) return r;
     c->allocs.insert(*p);
     return MZ_OK;
+}
+
+MzScratch::MzScratch(mz_ctx* c, size_t dev_bytes, size_t pin_bytes) : c_(c), lock_(c->scratch_mu, std::try_to_lock) {
+    auto get = [&](size_t bytes, size_t keep, void** kept, size_t* kept_bytes, bool* own, char** out, auto alloc, auto free) {
+        *own = !lock_.owns_lock() || bytes > keep;
+        void* p = nullptr;
+        if (*own) {
+            if ((status_ = alloc(&p, bytes))) return;
+        } else {
+            if (bytes > *kept_bytes) {
+                free(*kept);
+                *kept = nullptr;
+                *kept_bytes = 0;
+                // (in steps, so that slightly larger batches do not allocate each time)
+                const size_t step = (size_t)1 << 16, n = bytes < keep / 4 ? 2 * bytes : bytes;
+                const size_t want = (n + step - 1) / step * step;
+                if ((status_ = alloc(kept, want))) {
+                    *kept = nullptr;
+                    return;
+                }
+                *kept_bytes = want;
+            }
+            p = *kept;
+        }
+        *out = (char*)p;
+    };
+    get(dev_bytes, KEEP_DEV, &c->scratch_dev, &c->scratch_dev_bytes, &own_dev_, &dev,
+        [](void** p, size_t n) { return mz_hip(hipMalloc(p, n), "hipMalloc (scratch)"); }, [](void* p) { hipFree(p); });
+    if (!status_)
+        get(pin_bytes, KEEP_PIN, &c->scratch_pin, &c->scratch_pin_bytes, &own_pin_, &pin,
+            [](void** p, size_t n) { return mz_hip(hipHostMalloc(p, n, hipHostMallocDefault), "hipHostMalloc (scratch)"); },
+            [](void* p) { hipHostFree(p); });
+}
+
+MzScratch::~MzScratch() {
+    if (own_dev_ && dev) hipFree(dev);
+    if (own_pin_ && pin) hipHostFree(pin);
 }
 
 extern "C" int mz_alloc(mz_ctx* c, size_t bytes, uint64_t* dptr) {
@@ -312,18 +351,16 @@ extern "C" int mz_jump_times_device(mz_ctx* c, uint64_t w, int64_t clip_stride, 
     if (int r = mz_hip(hipSetDevice(c->device), "hipSetDevice")) return r;
     const long ds = mz_ts_diag_stride(rmax, cols_full);
     const size_t stat = (size_t)n * heads * cols_full;
-    const size_t bytes[5] = {(size_t)n * sizeof(int2), stat * 4, stat * 4, (size_t)n * ds * 5,
-                             (size_t)n * out_stride * 4};
-    void* buf[5] = {};
-    auto release = [&]() {
-        for (void* b : buf)
-            if (b) hipFree(b);
+    auto up = [](size_t v) { return (v + 255) & ~(size_t)255; };
+    const size_t bytes_rc = (size_t)n * sizeof(int2), bytes_out = (size_t)n * std::max(rmax, 1) * 4;
+    MzScratch scratch(c, up(bytes_rc) + 2 * up(stat * 4) + up((size_t)n * ds * 5) + up(bytes_out), up(bytes_rc) + bytes_out);
+    if (scratch.status()) return scratch.status();
+    char* q = scratch.dev;
+    auto carve = [&](size_t bytes) {
+        char* r = q;
+        q += up(bytes);
+        return r;
     };
-    for (int i = 0; i < 5; i++)
-        if (int r = mz_hip(hipMalloc(&buf[i], std::max<size_t>(bytes[i], 4)), "hipMalloc")) {
-            release();
-            return r;
-        }
     MzTs p{};
     p.w = (const float*)(uintptr_t)w;
     p.clip_stride = clip_stride;
@@ -332,23 +369,23 @@ extern "C" int mz_jump_times_device(mz_ctx* c, uint64_t w, int64_t clip_stride, 
     p.width = width;
     p.half = half;
     p.rmax = rmax;
-    p.rc = (const int2*)buf[0];
-    p.mean = (float*)buf[1];
-    p.sd = (float*)buf[2];
-    p.cost = (float*)buf[3];
-    p.trace = (signed char*)((float*)buf[3] + (size_t)n * ds);
+    p.rc = (const int2*)carve(bytes_rc);
+    p.mean = (float*)carve(stat * 4);
+    p.sd = (float*)carve(stat * 4);
+    p.cost = (float*)carve((size_t)n * ds * 5);
+    p.trace = (signed char*)(p.cost + (size_t)n * ds);
     p.diag_stride = ds;
     p.ldd = mz_ts_ldd(rmax);
-    p.out = (float*)buf[4];
-    p.out_stride = out_stride;
-    int r = mz_hip(hipMemcpyAsync(buf[0], rc.data(), bytes[0], hipMemcpyHostToDevice, c->stream), "upload");
+    // the times come back packed, in one copy, and go to the caller's rows from there
+    p.out = (float*)carve(bytes_out);
+    p.out_stride = rmax;
+    float* times = (float*)(scratch.pin + up(bytes_rc));
+    std::memcpy(scratch.pin, rc.data(), bytes_rc);
+    int r = mz_hip(hipMemcpyAsync((void*)p.rc, scratch.pin, bytes_rc, hipMemcpyHostToDevice, c->stream), "upload");
     if (!r) r = mz_hip(mz_ts_launch(c->stream, p, n), "timestamp kernels");
-    for (int i = 0; i < n && !r; i++)
-        if (rows[i] > 0)
-            r = mz_hip(hipMemcpyAsync(out + i * out_stride, (float*)buf[4] + i * out_stride, (size_t)rows[i] * 4,
-                                      hipMemcpyDeviceToHost, c->stream),
-                       "download");
-    if (!r) r = mz_hip(hipStreamSynchronize(c->stream), "hipStreamSynchronize");
-    release();
-    return r;
+    if (!r && rmax > 0) r = mz_hip(hipMemcpyAsync(times, p.out, bytes_out, hipMemcpyDeviceToHost, c->stream), "download");
+    const int rs = mz_hip(hipStreamSynchronize(c->stream), "hipStreamSynchronize");
+    if (r || rs) return r ? r : rs;
+    for (int i = 0; i < n; i++) std::copy(times + (size_t)i * rmax, times + (size_t)i * rmax + rows[i], out + i * out_stride);
+    return MZ_OK;
 }

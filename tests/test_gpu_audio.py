@@ -117,3 +117,62 @@ def test_log_mel_unaligned_output_and_a_nan_sample(ctx):
     np.testing.assert_array_equal(got[:, ~edge], ref[0][:, ~edge])
     ctx.free(d_audio)
     ctx.free(d_mel)
+
+
+def test_scratch_kept_between_calls():
+    """Features and timestamps take turns on one context's scratch, in sizes that grow and shrink it, and from two threads
+    at once: the same values as on a context of their own."""
+    import threading
+
+    from mimizuku_amd import transcribe
+    rng = np.random.default_rng(12)
+    own = model.Context(0)
+    jobs = []
+    for n, rows, seconds in ((1, 9, 0.5), (3, 130, 7.0), (2, 300, 2.0), (1, 40, 30.0)):
+        w = rng.random((n, rows, 4, 1500), dtype=np.float32)
+        clips = [(0.1 * rng.standard_normal(int(16000 * seconds))).astype(np.float32) for _ in range(n)]
+        jobs.append((w, clips))
+
+    def do(ctx, job):
+        w, clips = job
+        n, rows = w.shape[:2]
+        dw = ctx.upload_new(w)
+        t = transcribe.jump_times_device(ctx, dw, rows * 4 * 1500, [rows - i for i in range(n)], [1500] * n, 4, 1500)
+        ctx.free(dw)
+        return t, log_mel(ctx, clips, 80)[0]
+
+    ref = []
+    for job in jobs:
+        c = model.Context(0)
+        ref.append(do(c, job))
+        c.close()
+
+    def same(a, b):
+        for x, y in zip(a[0], b[0]):
+            np.testing.assert_array_equal(x, y)
+        np.testing.assert_array_equal(a[1], b[1])
+
+    for i in (0, 1, 2, 3, 1, 0):
+        same(do(own, jobs[i]), ref[i])
+    # two threads, each with a context's timestamps of its own weights at once on one shared context
+    dws = [own.upload_new(jobs[i][0]) for i in (1, 2)]
+    got = [[], []]
+
+    def times(k):
+        w = jobs[k + 1][0]
+        n, rows = w.shape[:2]
+        for _ in range(5):
+            got[k].append(transcribe.jump_times_device(own, dws[k], rows * 4 * 1500, [rows - i for i in range(n)],
+                                                       [1500] * n, 4, 1500))
+
+    threads = [threading.Thread(target=times, args=(k,)) for k in (0, 1)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for k in (0, 1):
+        assert len(got[k]) == 5
+        for g in got[k]:
+            for x, y in zip(g, ref[k + 1][0]):
+                np.testing.assert_array_equal(x, y)
+    own.close()
