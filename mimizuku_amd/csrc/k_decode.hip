@@ -95,63 +95,74 @@ __global__ void __launch_bounds__(512) dec_add_ln_kernel(const float* xin, float
     ln_row4(v, on, dim, wv, bv, y + (long)row * dim, eps, red);
 }
 
-// LayerNorm of one row held by one wave, NC float4 per lane (v[i] = x[4 (lane + 64 i) ..]), written to y as fp16:
-// two-pass statistics over the wave through DPP and lane reads (no LDS, no barrier)
-template <int NC>
-__device__ __forceinline__ void ln_wave(const f32x4 (&v)[NC], const f16x4 (&wv)[NC], const f16x4 (&bv)[NC],
-                                        f16* __restrict__ y, float eps) {
-    constexpr int dim = 256 * NC;
+// LayerNorm of one row held by one wave, NC groups of VW floats per lane (v[i] = x[VW (lane + 64 i) ..]), written to y as
+// fp16: two-pass statistics over the wave through DPP and lane reads (no LDS, no barrier)
+template <int VW>
+struct Vec {
+    typedef float f __attribute__((ext_vector_type(VW)));
+    typedef f16 h __attribute__((ext_vector_type(VW)));
+};
+template <int VW, int NC>
+__device__ __forceinline__ void ln_wave(const typename Vec<VW>::f (&v)[NC], const typename Vec<VW>::h (&wv)[NC],
+                                        const typename Vec<VW>::h (&bv)[NC], f16* __restrict__ y, float eps) {
+    constexpr int dim = 64 * VW * NC;
     const int lane = threadIdx.x & 63;
     float sum = 0.f;
 #pragma unroll
-    for (int i = 0; i < NC; i++) sum += (v[i][0] + v[i][1]) + (v[i][2] + v[i][3]);
+    for (int i = 0; i < NC; i++) {
+        if constexpr (VW == 4) sum += (v[i][0] + v[i][1]) + (v[i][2] + v[i][3]);
+        else sum += v[i][0] + v[i][1];
+    }
     const float mean = wave_sum(sum) / dim;
     float q = 0.f;
 #pragma unroll
     for (int i = 0; i < NC; i++)
 #pragma unroll
-        for (int e = 0; e < 4; e++) {
+        for (int e = 0; e < VW; e++) {
             const float d = v[i][e] - mean;
             q = fmaf(d, d, q);
         }
     const float rstd = rsqrtf(wave_sum(q) / dim + eps);
 #pragma unroll
     for (int i = 0; i < NC; i++) {
-        float o[4];
+        typename Vec<VW>::h o;
 #pragma unroll
-        for (int e = 0; e < 4; e++) o[e] = (v[i][e] - mean) * rstd * (float)wv[i][e] + (float)bv[i][e];
-        st4(y + (lane + 64 * i) * 4, o[0], o[1], o[2], o[3]);
+        for (int e = 0; e < VW; e++) o[e] = (f16)((v[i][e] - mean) * rstd * (float)wv[i][e] + (float)bv[i][e]);
+        *(typename Vec<VW>::h*)(y + (lane + 64 * i) * VW) = o;
     }
 }
 
-// dec_add_ln_kernel's work with one wave per row for NC float4 per lane (dim = 256 NC) and NP partials: every load of
-// the row (residual, partials, bias, gamma, beta: 6 NC + 3 NC requests per lane) is issued before the first use, the
-// residual is summed in dec_add_ln_kernel's order (the same x), and the LayerNorm statistics are two-pass sums over
-// the wave through DPP and lane reads, so no barrier and no LDS are needed.
-template <int NC, int NP>
+// dec_add_ln_kernel's work with one wave per row for NC groups of VW floats per lane (dim = 64 VW NC) and NP partials:
+// every load of the row (residual, partials, bias, gamma, beta) is issued before the first use, the residual is summed in
+// dec_add_ln_kernel's order (the same x), and the LayerNorm statistics are two-pass sums over the wave through DPP and
+// lane reads, so no barrier and no LDS are needed. Bound by the launch and one round trip.
+template <int VW, int NC, int NP>
 __global__ void __launch_bounds__(64) dec_add_ln_wave_kernel(const float* xin, float* x, const float* __restrict__ parts,
                                                               long part_stride, const f16* __restrict__ bias,
                                                               const f16* __restrict__ w, const f16* __restrict__ b,
                                                               f16* __restrict__ y, float eps) {
 #if defined(__HIP_DEVICE_COMPILE__)
-    constexpr int dim = 256 * NC;
+    typedef typename Vec<VW>::f vf;
+    typedef typename Vec<VW>::h vh;
+    constexpr int dim = 64 * VW * NC;
     const int row = blockIdx.x, lane = threadIdx.x;
     const long r0 = (long)row * dim;
-    f32x4 v[NC], pp[NP][NC];
-    f16x4 bb[NC], wv[NC], bv[NC];
+    vf v[NC], pp[NP][NC];
+    vh bb[NC], wv[NC], bv[NC];
 #pragma unroll
-    for (int i = 0; i < NC; i++) v[i] = *(const f32x4*)(xin + r0 + (lane + 64 * i) * 4);
+    for (int i = 0; i < NC; i++) v[i] = *(const vf*)(xin + r0 + (lane + 64 * i) * VW);
 #pragma unroll
     for (int s = 0; s < NP; s++)
 #pragma unroll
-        for (int i = 0; i < NC; i++) pp[s][i] = *(const f32x4*)(parts + s * part_stride + r0 + (lane + 64 * i) * 4);
+        for (int i = 0; i < NC; i++) pp[s][i] = *(const vf*)(parts + s * part_stride + r0 + (lane + 64 * i) * VW);
     const __amdgpu_buffer_rsrc_t rB = rsrc(bias, bias ? (unsigned)dim * 2u : 0u);
 #pragma unroll
     for (int i = 0; i < NC; i++) {
-        const unsigned o = (unsigned)(lane + 64 * i) * 8u;
-        bb[i] = __builtin_bit_cast(f16x4, __builtin_amdgcn_raw_buffer_load_b64(rB, o, 0, 0));
-        wv[i] = *(const f16x4*)(w + (lane + 64 * i) * 4);
-        bv[i] = *(const f16x4*)(b + (lane + 64 * i) * 4);
+        const unsigned o = (unsigned)(lane + 64 * i) * VW * 2u;
+        if constexpr (VW == 4) bb[i] = __builtin_bit_cast(vh, __builtin_amdgcn_raw_buffer_load_b64(rB, o, 0, 0));
+        else bb[i] = __builtin_bit_cast(vh, __builtin_amdgcn_raw_buffer_load_b32(rB, o, 0, 0));
+        wv[i] = *(const vh*)(w + (lane + 64 * i) * VW);
+        bv[i] = *(const vh*)(b + (lane + 64 * i) * VW);
     }
     __builtin_amdgcn_sched_barrier(0);  // every request above is issued before anything waits for data
 #pragma unroll
@@ -159,10 +170,10 @@ __global__ void __launch_bounds__(64) dec_add_ln_wave_kernel(const float* xin, f
 #pragma unroll
         for (int s = 0; s < NP; s++) v[i] += pp[s][i];
 #pragma unroll
-        for (int e = 0; e < 4; e++) v[i][e] += (float)bb[i][e];
-        *(f32x4*)(x + r0 + (lane + 64 * i) * 4) = v[i];
+        for (int e = 0; e < VW; e++) v[i][e] += (float)bb[i][e];
+        *(vf*)(x + r0 + (lane + 64 * i) * VW) = v[i];
     }
-    ln_wave<NC>(v, wv, bv, y + r0, eps);
+    ln_wave<VW, NC>(v, wv, bv, y + r0, eps);
 #endif
 }
 
@@ -1016,11 +1027,23 @@ hipError_t mz_dec_add_ln_launch(hipStream_t s, const float* xin, float* x, const
                                 long part_stride, const f16* bias, const f16* w, const f16* b, f16* y, int rows,
                                 int dim, float eps) {
     if (dim % 4 != 0 || dim > 2048 || rows <= 0 || nparts < 0 || nparts > MZ_MAX_PARTS) return hipErrorInvalidValue;
-    // one wave per row for the decoder width of large-v3 and large-v3-turbo with its five split-K partials
-    if (dim == 1280 && nparts == 5) {
-        hipLaunchKernelGGL((dec_add_ln_wave_kernel<5, 5>), dim3(rows), dim3(64), 0, s, xin, x, parts, part_stride, bias,
-                           w, b, y, eps);
+    // One wave per row at the models' widths with the split-K counts that the engine's products of those widths take
+    // (ksplit_for): in a replayed step a launch costs about 1 us less than the general kernel (one workgroup of up to
+    // five waves per row, their sums through LDS): 12 launches a step, width 384 at one row 196 -> 188 us, 1024 at six
+    // 244 -> 234, 1280 at 32 401.8 -> 390.4.
+    auto wave = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(rows), dim3(64), 0, s, xin, x, parts, part_stride, bias, w, b, y, eps);
         return hipGetLastError();
+    };
+    switch (dim * 100 + nparts) {
+        case 38406: return wave(dec_add_ln_wave_kernel<2, 3, 6>);
+        case 38412: return wave(dec_add_ln_wave_kernel<2, 3, 12>);
+        case 51208: return wave(dec_add_ln_wave_kernel<4, 2, 8>);
+        case 51216: return wave(dec_add_ln_wave_kernel<4, 2, 16>);
+        case 76808: return wave(dec_add_ln_wave_kernel<4, 3, 8>);
+        case 76812: return wave(dec_add_ln_wave_kernel<4, 3, 12>);
+        case 102408: return wave(dec_add_ln_wave_kernel<4, 4, 8>);
+        case 128005: return wave(dec_add_ln_wave_kernel<4, 5, 5>);
     }
     hipLaunchKernelGGL(dec_add_ln_kernel, dim3(rows), dim3(row_threads(dim)), 0, s, xin, x, parts, nparts, part_stride,
                        bias, w, b, y, dim, eps);
