@@ -153,6 +153,7 @@ struct mz_engine {
     f16 *h = nullptr, *datt = nullptr, *dff = nullptr, *kc = nullptr, *vc = nullptr;
     float* align = nullptr;  // alignment-head probabilities [bmax][max_t][na][1500], fp32
     f16* alignh = nullptr;   // the same rows rounded to fp16 (the reference's own buffer, src/model.rs:455)
+    float* xpart = nullptr;  // split cross-attention: four states per (row, head) of a small batch
     int2* amax = nullptr;  // LM head argmax partials [mz_lm_blocks(vocab)][bmax]
     int* aslot = nullptr;
     unsigned char *sup = nullptr, *sup_lang = nullptr;
@@ -226,6 +227,8 @@ size_t weight_elems(const mz_dims& d, int* k1pad) {
 // one set of cross keys/values: [bmax][dec layers][k|v][heads] tiles of 1536 x 64
 size_t xkv_elems(const mz_dims& d, int bmax) { return (size_t)bmax * d.dec_layers * 2 * d.nh * (size_t)TPAD * HD; }
 
+constexpr size_t XPART = (size_t)MZ_CROSS_SPLIT_PAIRS * 4 * MZ_CROSS_STATE;  // floats of the split cross-attention's states
+
 int ksplit_for(int N, int K) {
     // Split K over workgroups until the grid covers most of the 256 CUs, with at most 16 groups of 64 per workgroup
     // (a slice within MZ_DEC_KSLICE, both operands resident in LDS) and at most MZ_MAX_PARTS partials.
@@ -257,7 +260,7 @@ extern "C" size_t mz_scratch_bytes(const mz_dims* d, int n_align, int bmax, int 
                  G * TENC * D * 2 * 3 + G * 3 * nh * TPAD * HD * 2 + G * TENC * F * 2;
     size_t dec = B * nl * 2 * nh * TPAD * HD * 2 + B * mt * 4 + B * 4 + 16 + B * D * 4 + B * D * 2 * 2 + B * F * 2 +
                  2 * nl * B * nh * mt * HD * 2 + B * V * 4 + B * mt * n_align * TENC * (4 + 2) + (size_t)mz_lm_blocks((int)V) * B * 8 +
-                 nl * nh * 4 + 2 * V;
+                 nl * nh * 4 + 2 * V + XPART * 4;
     size_t part = part_elems((int)D, (int)F, (int)B) * 4;
     size_t ts = B * 8 + 2 * B * n_align * TENC * 4 + B * (size_t)mz_ts_diag_stride((int)mt - 1, TENC) * 5 + B * mt * 4;
     return MZ_ENC_LANES * enc + dec + part + ts;
@@ -422,7 +425,7 @@ extern "C" int mz_engine_new(mz_ctx* c, const mz_dims* d, const mz_gencfg* g, in
         (r = e->alloc(&e->vc, (size_t)nl * B * nh * mt * HD)) || (r = e->alloc(&e->logits, B * V)) ||
         (r = e->alloc(&e->align, B * mt * e->na * (size_t)TENC)) ||
         (r = e->alloc(&e->alignh, B * mt * e->na * (size_t)TENC)) ||
-        (r = e->alloc(&e->amax, (size_t)mz_lm_blocks(V) * B)) ||
+        (r = e->alloc(&e->xpart, XPART)) || (r = e->alloc(&e->amax, (size_t)mz_lm_blocks(V) * B)) ||
         (r = e->alloc(&e->aslot, (size_t)nl * nh)) || (r = e->alloc(&e->sup, V)) || (r = e->alloc(&e->sup_lang, V)))
         return fail(r);
     const size_t tsd = (size_t)mz_ts_diag_stride(mt - 1, TENC);
@@ -764,7 +767,7 @@ static int step_impl(mz_engine* e, int b, int lang, int prompt_len) {
     // the projection weights stay in the memory-side cache between steps when all layers' fit it with room to spare
     // (large-v3-turbo: 183 MB of 256) and the batch has two rows or more; otherwise they stream nontemporally
     const bool w_cached = (size_t)nl * (6 * (size_t)D * D + 2 * (size_t)D * F) * 2 <= ((size_t)200 << 20) && b >= 2;
-    auto gemm = [&](int epi, const f16* x, int ldx, const Lin& L, int N, int K, int ks, void* out, long ldo) {
+    auto gemm_args = [&](const f16* x, int ldx, const Lin& L, int N, int K, int ks, void* out, long ldo) {
         MzDec g{};
         g.w_nt = w_cached ? 0 : 1;
         g.x = x;
@@ -778,7 +781,10 @@ static int step_impl(mz_engine* e, int b, int lang, int prompt_len) {
         g.out = out;
         g.ldo = ldo;
         g.ctr = e->ctr;
-        return mz_dec_gemm_launch(s, epi, g);
+        return g;
+    };
+    auto gemm = [&](int epi, const f16* x, int ldx, const Lin& L, int N, int K, int ks, void* out, long ldo) {
+        return mz_dec_gemm_launch(s, epi, gemm_args(x, ldx, L, N, K, ks, out, ldo));
     };
     auto attn_args = [&](const float* q, int nq, const f16* wq, const f16* qbias, const f16* k, const f16* v, long kv_b,
                          int L, const int* aslot) {
@@ -808,6 +814,8 @@ static int step_impl(mz_engine* e, int b, int lang, int prompt_len) {
     };
     const int ks_dd = ksplit_for(D, D), ks_df = ksplit_for(D, F), ks_qkv = ksplit_for(3 * D, D);
     const f16* xkv = e->xkvbuf;
+    // the split needs K slices of whole heads within the out-projection's x block
+    const bool xsplit = mz_cross_split(b, nh) && D / ks_dd <= 256;
     for (int i = 0; i < nl; i++) {
         const DecLayer& L = e->decv[i];
         f16* kc = e->kc + (size_t)i * e->bmax * nh * mt * HD;
@@ -850,9 +858,21 @@ static int step_impl(mz_engine* e, int b, int lang, int prompt_len) {
             c.align = e->align;
             c.alignh = e->alignh;
             c.na = e->na;
+            c.part = xsplit ? e->xpart : nullptr;
             PROF(MZ_K_DEC_CROSS, mz_dec_cross_launch(s, c), "cross attention");
+            MzDec g = gemm_args(e->datt, D, L.xo, D, D, ks_dd, e->part, D);
+            if (xsplit) {
+                g.part = e->xpart;
+                g.nh = nh;
+                g.maxT = mt;
+                g.na = e->na;
+                g.done = e->done;
+                g.aslot = c.aslot;
+                g.align = e->align;
+                g.alignh = e->alignh;
+            }
+            PROF(MZ_K_DEC_XO, mz_dec_gemm_launch(s, DEPI_PARTIAL, g), "dec cross out-proj");
         }
-        PROF(MZ_K_DEC_XO, gemm(DEPI_PARTIAL, e->datt, D, L.xo, D, D, ks_dd, e->part, D), "dec cross out-proj");
         PROF(MZ_K_DEC_ADDLN,
              mz_dec_add_ln_launch(s, e->x, e->x, e->part, ks_dd, (long)b * D, L.xo.b, L.ln3.w, L.ln3.b, e->h, b, D,
                                   EPS),
@@ -1024,7 +1044,7 @@ extern "C" int mz_engine_free(mz_engine* e) {
     for (void* p : {(void*)e->arena, (void*)e->mel, (void*)e->melT, (void*)e->h1, (void*)e->ex, (void*)e->hb, (void*)e->dd,
                     (void*)e->qkvh, (void*)e->att, (void*)e->ff, (void*)e->trace, (void*)e->dtrace, (void*)e->xkvbuf, (void*)e->tok,
                     (void*)e->done, (void*)e->ctr, (void*)e->x, (void*)e->h, (void*)e->datt,
-                    (void*)e->dff, (void*)e->kc, (void*)e->vc, (void*)e->logits, (void*)e->align, (void*)e->alignh, (void*)e->amax,
+                    (void*)e->dff, (void*)e->kc, (void*)e->vc, (void*)e->logits, (void*)e->align, (void*)e->alignh, (void*)e->xpart, (void*)e->amax,
                     (void*)e->aslot, (void*)e->sup, (void*)e->sup_lang,
                     (void*)e->part})
         if (p) mz_free(e->c, (uint64_t)(uintptr_t)p);

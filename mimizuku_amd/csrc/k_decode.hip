@@ -20,6 +20,7 @@
 //                 step's key and value into the cache (kv_write + whisper.cu:319-353), and cross-attention over the
 //                 encoder keys/values, which projects its own query from the row's LayerNorm output and records the
 //                 alignment-head probabilities (whisper.cu:355-449)
+//                 Small batches: the cross-attention over four workgroups per (row, head), merged by the out-projection
 //   dec_add_ln    residual add of the split-K partials + bias, fused with the next LayerNorm (whisper.cu:71-82)
 //   dec_argmax    greedy choice from the per-workgroup argmax partials; advances the position (whisper.cu:451-495)
 #include "mz_common.h"
@@ -202,6 +203,36 @@ __global__ void __launch_bounds__(512) dec_embed_ln_kernel(const int* __restrict
     ln_row4(v, on, dim, wv, bv, y + (long)row * dim, eps, red);
 }
 
+// ---------------------------------------------------------------- merging softmax states
+
+// A query's groups of 8 lanes each hold an online softmax over their keys: maximum, sum, and 64 accumulators. They merge
+// in two levels, the same everywhere so that every form of the attention gives the same bits: the eight groups of a
+// wave in order, then the four waves' states in order. (A group or wave without keys: maximum -inf, no weight.)
+struct SoftmaxState {
+    float m, l, o;
+};
+template <class Get>
+__device__ __forceinline__ SoftmaxState merge_states(int n, Get get) {
+    float m = -3.402823466e38f;
+    for (int g = 0; g < n; g++) m = fmaxf(m, get(g).m);
+    SoftmaxState r{m, 0.f, 0.f};
+    for (int g = 0; g < n; g++) {
+        const SoftmaxState s = get(g);
+        const float w = __builtin_amdgcn_exp2f(s.m - m);
+        r.l = fmaf(s.l, w, r.l);
+        r.o = fmaf(s.o, w, r.o);
+    }
+    return r;
+}
+
+// An alignment probability from a score in log2 units. The product is kept from being fused with a conversion: the fp16
+// row is the fp32 row's value rounded, not the exact product rounded (the kernels differed there in one value in 1e5).
+__device__ __forceinline__ float prob(float s, float m, float inv) {
+    float p = __builtin_amdgcn_exp2f(s - m) * inv;
+    asm volatile("" : "+v"(p));
+    return p;
+}
+
 // ---------------------------------------------------------------- skinny GEMM
 
 typedef __attribute__((address_space(3))) void lds_void;
@@ -209,6 +240,8 @@ typedef __attribute__((address_space(3))) void lds_void;
 
 // s_waitcnt operand that waits until at most n vector memory operations of this wave are outstanding (n < 64)
 constexpr int vm_wait(int n) { return (n & 15) | ((n >> 4) << 14) | (7 << 4) | (15 << 8); }
+// ... and no LDS operation is
+constexpr int vm_lgkm0_wait(int n) { return (n & 15) | ((n >> 4) << 14) | (7 << 4); }
 
 
 // Cache policy of the decoder's streams. The cross keys / values (983 MB per 32-row turbo step) and the LM head's
@@ -229,7 +262,10 @@ constexpr int MZ_NT = 2;  // cache-policy bit of a buffer load: nontemporal
 // banks. The 4 waves split the K groups; their 32x32 products are summed in LDS. Every operand of the epilogue (bias,
 // mask, position) is requested at entry with the loads, so the kernel makes a single round trip to memory.
 // KS: the largest K slice of the launch (LDS sized to it: a workgroup asks for no more than it uses)
-template <int EPI, int KS>
+// MERGE: x is the cross-attention's output, still in the four states per (row, head) that dec_cross_split_kernel leaves
+// (p.part): each workgroup merges its K slice's heads into the x block while its W rows are on their way, and the
+// alignment heads' raw scores become probabilities here, where the merged maximum and sum are known.
+template <int EPI, int KS, bool MERGE = false>
 __global__ void __launch_bounds__(256) dec_gemm_kernel(const MzDec p) {
 #if defined(__HIP_DEVICE_COMPILE__)  // the buffer-resource type exists only in the device pass
     constexpr int NC = 4;  // output columns per epilogue thread
@@ -251,8 +287,9 @@ __global__ void __launch_bounds__(256) dec_gemm_kernel(const MzDec p) {
     for (int i = wave; i < 4 * G; i += 4) {
         const int g = i >> 2, rg = i & 3, c = q8 ^ r8 ^ (rg & 1);
         const unsigned col = (unsigned)(kb + g * 64 + c * 8) * 2;
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rX, LDSP(sx + i * 512), 16, (unsigned)(rg * 8 + r8) * ldx2 + col, 0, 0,
-                                                 0);
+        if (!MERGE)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rX, LDSP(sx + i * 512), 16, (unsigned)(rg * 8 + r8) * ldx2 + col, 0,
+                                                     0, 0);
         const unsigned ow = (unsigned)(n0 + rg * 8 + r8) * (unsigned)p.K * 2u + col;
         if (p.w_nt)  // (the policy is an immediate of the instruction: one load per branch, a uniform branch)
             __builtin_amdgcn_raw_ptr_buffer_load_lds(rW, LDSP(sw + i * 512), 16, ow, 0, 0, MZ_NT);
@@ -268,7 +305,39 @@ __global__ void __launch_bounds__(256) dec_gemm_kernel(const MzDec p) {
         bv[e] = (EPI != DEPI_PARTIAL && p.bias) ? (float)p.bias[n] : 0.f;
         msk[e] = EPI == DEPI_LOGITS ? p.sup[n] != 0 : false;
     }
-    const int pos = EPI == DEPI_LOGITS ? p.ctr[1] : 0;
+    const int pos = EPI == DEPI_LOGITS || MERGE ? p.ctr[1] : 0;
+    if (MERGE) {
+        auto state = [&](int ph, int i, int w) {
+            const float* q = p.part + (long)(ph * 4 + w) * MZ_CROSS_STATE;
+            return SoftmaxState{q[64], q[65], q[i]};
+        };
+        // (rows past M keep what is in LDS: their columns of the product are not stored)
+        for (int e = tid; e < p.M * ksl; e += 256) {
+            const int row = e / ksl, k = e - row * ksl, head = (kb + k) >> 6, i = (kb + k) & 63;
+            const SoftmaxState t = merge_states(4, [&](int w) { return state(row * p.nh + head, i, w); });
+            const int rg = row >> 3, r = row & 7, c = (k & 63) >> 3;
+            sx[((k >> 6) * 4 + rg) * 512 + r * 64 + ((c ^ r ^ (rg & 1)) << 3) + (k & 7)] = (f16)(t.o / t.l);
+        }
+        // the workgroups share the (row, head) pairs' alignment rows (usually one pair or none each)
+        for (int pair = blockIdx.y * gridDim.x + blockIdx.x; pair < p.M * p.nh; pair += gridDim.x * gridDim.y) {
+            const int row = pair / p.nh, slot = p.aslot[pair - row * p.nh];
+            if (slot < 0 || p.done[row] || pos >= p.maxT) continue;
+            constexpr int NSC = (MZ_TENC + 255) / 256;
+            float sc[NSC];
+            const long ao = (((long)row * p.maxT + pos) * p.na + slot) * MZ_TENC;
+#pragma unroll
+            for (int k = 0; k < NSC; k++) sc[k] = tid + 256 * k < MZ_TENC ? p.align[ao + tid + 256 * k] : 0.f;
+            const SoftmaxState t = merge_states(4, [&](int w) { return state(pair, 0, w); });
+            const float inv = 1.f / t.l;
+#pragma unroll
+            for (int k = 0; k < NSC; k++)
+                if (tid + 256 * k < MZ_TENC) {
+                    const float pj = prob(sc[k], t.m, inv);
+                    p.align[ao + tid + 256 * k] = pj;
+                    if (p.alignh) p.alignh[ao + tid + 256 * k] = (f16)pj;
+                }
+        }
+    }
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
 
@@ -500,6 +569,7 @@ __global__ void __launch_bounds__(AG * 8) dec_attn_kernel(const MzDecAttn a) {
     __shared__ float sc[MZ_TPAD];
     __shared__ float gm[AG], gl[AG];
     __shared__ float gacc[AG][MZ_HD + 1];
+    __shared__ float wm[AG / 8], wl[AG / 8], wo[AG / 8][MZ_HD];
     __shared__ float tot[2];
     __shared__ __attribute__((aligned(16))) f16 kvn[2][MZ_HD];  // the step's own key and value (self, kw set)
 
@@ -666,19 +736,22 @@ __global__ void __launch_bounds__(AG * 8) dec_attn_kernel(const MzDecAttn a) {
 #pragma unroll
     for (int e = 0; e < 8; e++) gacc[grp][sub * 8 + e] = acc[e];
     __syncthreads();
-    if (tid < MZ_HD) {
-        float M = gm[0];
-        for (int g = 1; g < AG; g++) M = fmaxf(M, gm[g]);
-        float lt = 0.f, o = 0.f;
-        for (int g = 0; g < AG; g++) {
-            const float w = __builtin_amdgcn_exp2f(gm[g] - M);
-            lt = fmaf(gl[g], w, lt);
-            o = fmaf(gacc[g][tid], w, o);
+    {  // wave w merges its eight groups (dim i in lane i), then the first wave the four
+        const int w = tid >> 6, i = tid & 63;
+        const SoftmaxState t = merge_states(8, [&](int g) { return SoftmaxState{gm[8 * w + g], gl[8 * w + g], gacc[8 * w + g][i]}; });
+        wo[w][i] = t.o;
+        if (i == 0) {
+            wm[w] = t.m;
+            wl[w] = t.l;
         }
-        a.out[(long)b * a.d + head * MZ_HD + tid] = (f16)(o / lt);
+    }
+    __syncthreads();
+    if (tid < MZ_HD) {
+        const SoftmaxState t = merge_states(4, [&](int w) { return SoftmaxState{wm[w], wl[w], wo[w][tid]}; });
+        a.out[(long)b * a.d + head * MZ_HD + tid] = (f16)(t.o / t.l);
         if (tid == 0) {
-            tot[0] = M;
-            tot[1] = lt;
+            tot[0] = t.m;
+            tot[1] = t.l;
         }
     }
     if (slot < 0 || pos >= a.maxT) return;
@@ -688,7 +761,7 @@ __global__ void __launch_bounds__(AG * 8) dec_attn_kernel(const MzDecAttn a) {
     float* al = a.align + ao;
     f16* alh = a.alignh ? a.alignh + ao : nullptr;
     for (int j = tid; j < L; j += blockDim.x) {
-        const float pj = __builtin_amdgcn_exp2f(sc[j] - M) * inv;
+        const float pj = prob(sc[j], M, inv);
         al[j] = pj;
         if (alh) alh[j] = (f16)pj;
     }
@@ -715,6 +788,7 @@ __global__ void __launch_bounds__(256, 1) dec_cross_wide_kernel(const MzDecCross
     __shared__ float sc[MZ_TPAD];
     __shared__ float gm[AG], gl[AG];
     __shared__ float gacc[AG][MZ_HD + 1];
+    __shared__ float wm[AG / 8], wl[AG / 8], wo[AG / 8][MZ_HD];
     __shared__ float tot[2];
 
     const int bh = blockIdx.x, b = bh / a.nh, head = bh - b * a.nh;
@@ -865,19 +939,22 @@ __global__ void __launch_bounds__(256, 1) dec_cross_wide_kernel(const MzDecCross
 #pragma unroll
     for (int e = 0; e < 8; e++) gacc[grp][sub * 8 + e] = acc[e];
     __syncthreads();
-    if (tid < MZ_HD) {
-        float M = gm[0];
-        for (int g = 1; g < AG; g++) M = fmaxf(M, gm[g]);
-        float lt = 0.f, o = 0.f;
-        for (int g = 0; g < AG; g++) {
-            const float w = __builtin_amdgcn_exp2f(gm[g] - M);
-            lt = fmaf(gl[g], w, lt);
-            o = fmaf(gacc[g][tid], w, o);
+    {  // wave w merges its eight groups (dim i in lane i), then the first wave the four
+        const int w = tid >> 6, i = tid & 63;
+        const SoftmaxState t = merge_states(8, [&](int g) { return SoftmaxState{gm[8 * w + g], gl[8 * w + g], gacc[8 * w + g][i]}; });
+        wo[w][i] = t.o;
+        if (i == 0) {
+            wm[w] = t.m;
+            wl[w] = t.l;
         }
-        a.out[(long)b * a.d + head * MZ_HD + tid] = (f16)(o / lt);
+    }
+    __syncthreads();
+    if (tid < MZ_HD) {
+        const SoftmaxState t = merge_states(4, [&](int w) { return SoftmaxState{wm[w], wl[w], wo[w][tid]}; });
+        a.out[(long)b * a.d + head * MZ_HD + tid] = (f16)(t.o / t.l);
         if (tid == 0) {
-            tot[0] = M;
-            tot[1] = lt;
+            tot[0] = t.m;
+            tot[1] = t.l;
         }
     }
     if (slot < 0 || pos >= a.maxT) return;
@@ -887,9 +964,160 @@ __global__ void __launch_bounds__(256, 1) dec_cross_wide_kernel(const MzDecCross
     float* al = a.align + ao;
     f16* alh = a.alignh ? a.alignh + ao : nullptr;
     for (int j = tid; j < L; j += 256) {
-        const float pj = __builtin_amdgcn_exp2f(sc[j] - M) * inv;
+        const float pj = prob(sc[j], M, inv);
         al[j] = pj;
         if (alh) alh[j] = (f16)pj;
+    }
+#endif
+}
+
+// ---------------------------------------------------------------- cross-attention for the smallest batches
+
+// The same arithmetic for at most 256 / (4 nh) rows: four workgroups per (row, head), each one wave's eight groups of
+// dec_attn_kernel (keys 8 s .. 8 s + 7 of every 32). What bounds a (row, head) on one CU is the CU's own rate for what
+// misses its caches (25 to 50 GB/s, whatever is in flight), so its 384 KB of keys and values go over four CUs. Each
+// projects the query for itself (its wq rows come from the L2 that the four share: they run on one XCD). The four
+// states (MZ_CROSS_STATE floats: 64 accumulators, maximum, sum) are merged by the out-projection that reads them, as
+// another launch for that would cost what the split gains. The four waves share the arithmetic that one would take 3 us
+// for: the scores by batches of keys, then the softmax by dims. One row: width 384 14.7 -> 9.1 us a layer, 1280 16.2 ->
+// 11.0, the out-projection 3.7 -> 4.0.
+__global__ void __launch_bounds__(256, 1) dec_cross_split_kernel(const MzDecCross a) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    constexpr int L = MZ_TENC, NI = (L + 31) / 32, AU = 8, NJ = MZ_DEC_KSLICE / 64;
+    __shared__ __attribute__((aligned(16))) f16x8 ks[NI][64], vs[NI][64];  // [key / 32][lane]: 8 keys x 64 dims, 1 KB
+    __shared__ __attribute__((aligned(16))) f16 xs[MZ_DEC_KSLICE];
+    __shared__ float qs[MZ_HD];
+    __shared__ __attribute__((aligned(16))) float ss[8][NI + 5];  // scores: group, key / 32
+    __shared__ float gm[8], gl[8], gacc[8][MZ_HD + 1];
+
+    const int xcd = blockIdx.x & 7, li = blockIdx.x >> 3, bh = (li >> 2) * 8 + xcd, split = li & 3;
+    if (bh >= a.B * a.nh) return;
+    const int b = bh / a.nh, head = bh - b * a.nh;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int r8 = lane >> 3, q8 = lane & 7, nj = a.d >> 6;
+    const int pos = a.ctr[1];
+    const int slot = a.aslot ? a.aslot[head] : -1;
+    const bool done = a.done[b] != 0;
+    const long kv = (long)b * a.kv_b + (long)head * a.kv_h;
+    const __amdgpu_buffer_rsrc_t rK = rsrc(a.k + kv, L * MZ_HD * 2), rV = rsrc(a.v + kv, L * MZ_HD * 2);
+
+    // in issue order: the row, this thread's chunks of wq (as dec_cross_wide_kernel), its two query biases, then this
+    // wave's share of the keys and values, straight into LDS (keys past the last read zeros)
+    const bool xl = tid < (a.d >> 3);
+    const f16x8 xv0 = xl ? *(const f16x8*)(a.xin + (long)b * a.d + tid * 8) : f16x8{};
+    const f16* wr = a.wq + (long)(head * MZ_HD + 8 * wave + r8) * a.d + q8 * 8;
+    f16x8 wv[2][NJ];
+#pragma unroll
+    for (int h = 0; h < 2; h++)
+#pragma unroll
+        for (int j = 0; j < NJ; j++) wv[h][j] = j < nj ? *(const f16x8*)(wr + 32L * h * a.d + j * 64) : f16x8{};
+    const __amdgpu_buffer_rsrc_t rQB = rsrc(a.qbias, a.qbias ? (unsigned)a.d * 2u : 0u);
+    const unsigned short qb[2] = {__builtin_amdgcn_raw_buffer_load_b16(rQB, (unsigned)(head * MZ_HD + 8 * wave + r8) * 2u, 0, 0),
+                                  __builtin_amdgcn_raw_buffer_load_b16(rQB, (unsigned)(head * MZ_HD + 32 + 8 * wave + r8) * 2u, 0, 0)};
+    __builtin_amdgcn_sched_barrier(0);
+    auto stage = [&](const __amdgpu_buffer_rsrc_t r, f16x8(*dst)[64]) {
+        for (int i = wave; i < NI; i += 4)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(r, LDSP(&dst[i][0]), 16,
+                                                     (unsigned)((32 * i + 8 * split) * MZ_HD * 2) + lane * 16u, 0, 0, MZ_NT);
+    };
+    stage(rK, ks);
+    __builtin_amdgcn_sched_barrier(0);
+    stage(rV, vs);
+    __builtin_amdgcn_sched_barrier(0);  // every request above is issued before anything waits for data
+    if (done) {  // a finished row: no attention (the staged loads land before the LDS is released)
+        __builtin_amdgcn_s_waitcnt(vm_wait(0));
+        return;
+    }
+    if (xl) *(f16x8*)&xs[tid * 8] = xv0;
+    lds_barrier();  // the row in LDS; the keys and values stay in flight
+    constexpr float QS = 0.125f * 1.4426950408889634f;  // 1/8 and log2(e)
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        float t = 0.f;
+#pragma unroll
+        for (int j = 0; j < NJ; j++) {
+            if (j < nj) {
+                const f16x8 xq = *(const f16x8*)&xs[(q8 + 8 * j) * 8];
+#pragma unroll
+                for (int e = 0; e < 8; e += 2)
+                    t = __builtin_amdgcn_fdot2(f16x2{wv[h][j][e], wv[h][j][e + 1]}, f16x2{xq[e], xq[e + 1]}, t, false);
+            }
+        }
+        t = group8_sum(t);
+        const int i = 32 * h + 8 * wave + r8;
+        if (q8 == 0) qs[i] = (t + (a.qbias ? (float)__builtin_bit_cast(f16, qb[h]) : 0.f)) * QS;
+    }
+    // this wave's keys have landed (its 11 or 12 loads of values, issued after them, may be in flight), then every wave's
+    __builtin_amdgcn_s_waitcnt(vm_lgkm0_wait(11));
+    asm volatile("s_barrier" ::: "memory");
+
+    // scores: group r8 has keys 8 split + r8 + 32 i; wave w takes dec_attn_kernel's batches w and w + 4 of eight i
+    float* al = slot >= 0 && pos < a.maxT ? a.align + (((long)b * a.maxT + pos) * a.na + slot) * MZ_TENC : nullptr;
+    {
+        float q8v[8];
+#pragma unroll
+        for (int e = 0; e < 8; e++) q8v[e] = qs[q8 * 8 + e];
+        for (int i0 = AU * wave; i0 < NI; i0 += 4 * AU) {
+            f16x8 K[AU];
+#pragma unroll
+            for (int u = 0; u < AU; u++) K[u] = ks[min(i0 + u, NI - 1)][lane];
+#pragma unroll
+            for (int u = 0; u < AU; u++) {
+                float t = 0.f;
+#pragma unroll
+                for (int e = 0; e < 8; e++) t = fmaf(q8v[e], (float)K[u][e], t);
+                t = group8_sum(t);
+                const int j = 8 * split + r8 + 32 * (i0 + u);
+                if (q8 == 0) {
+                    ss[r8][i0 + u] = j < L ? t : -INFINITY;
+                    if (al && j < L) al[j] = t;  // raw: the out-projection normalises it
+                }
+            }
+        }
+    }
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+    // the online softmax of dec_attn_kernel, wave w for dims 2 w and 2 w + 1 of each lane's eight
+    float m = -INFINITY, l = 0.f, acc[2] = {0.f, 0.f};
+    for (int i0 = 0; i0 < NI; i0 += AU) {
+        float s[AU];
+        f16x2 V[AU];
+#pragma unroll
+        for (int u = 0; u < AU; u++) {
+            s[u] = ss[r8][i0 + u];
+            V[u] = ((const f16x2*)&vs[min(i0 + u, NI - 1)][lane])[wave];
+        }
+        float mx = s[0];  // the batch's first key exists
+#pragma unroll
+        for (int u = 1; u < AU; u++) mx = fmaxf(mx, s[u]);
+        const float mn = fmaxf(m, mx);
+        const float cr = __builtin_amdgcn_exp2f(m - mn);
+        l *= cr;
+        acc[0] *= cr;
+        acc[1] *= cr;
+#pragma unroll
+        for (int u = 0; u < AU; u++) {
+            const float pe = __builtin_amdgcn_exp2f(s[u] - mn);
+            l += pe;
+            acc[0] = fmaf(pe, (float)V[u][0], acc[0]);
+            acc[1] = fmaf(pe, (float)V[u][1], acc[1]);
+        }
+        m = mn;
+    }
+    if (q8 == 0 && wave == 0) {
+        gm[r8] = m;
+        gl[r8] = l;
+    }
+    gacc[r8][q8 * 8 + 2 * wave] = acc[0];
+    gacc[r8][q8 * 8 + 2 * wave + 1] = acc[1];
+    __syncthreads();
+    if (wave) return;
+    const SoftmaxState t = merge_states(8, [&](int g) { return SoftmaxState{gm[g], gl[g], gacc[g][lane]}; });
+    float* part = a.part + (long)(bh * 4 + split) * MZ_CROSS_STATE;
+    part[lane] = t.o;
+    if (lane == 0) {
+        part[64] = t.m;
+        part[65] = t.l;
     }
 #endif
 }
@@ -955,6 +1183,12 @@ hipError_t mz_dec_gemm_launch(hipStream_t s, int epi, const MzDec& g) {
     const int ksl = g.K / g.ksplit;
     switch (epi) {
         case DEPI_PARTIAL:
+            if (g.part) {  // the cross-attention's states as x
+                if (g.M > 32 || !g.done || !g.ctr || !g.aslot || !g.align || g.K != g.nh * MZ_HD || ksl % 64) return hipErrorInvalidValue;
+                if (ksl > 256) return hipErrorInvalidValue;
+                hipLaunchKernelGGL((dec_gemm_kernel<DEPI_PARTIAL, 256, true>), grid, dim3(256), 0, s, g);
+                break;
+            }
             if (ksl <= 256) hipLaunchKernelGGL((dec_gemm_kernel<DEPI_PARTIAL, 256>), grid, dim3(256), 0, s, g);
             else if (ksl <= 512) hipLaunchKernelGGL((dec_gemm_kernel<DEPI_PARTIAL, 512>), grid, dim3(256), 0, s, g);
             else if (ksl <= 640) hipLaunchKernelGGL((dec_gemm_kernel<DEPI_PARTIAL, 640>), grid, dim3(256), 0, s, g);
@@ -994,6 +1228,11 @@ hipError_t mz_dec_cross_launch(hipStream_t s, const MzDecCross& a) {
         !a.wq)
         return hipErrorInvalidValue;
     if (a.aslot && (!a.align || a.na <= 0)) return hipErrorInvalidValue;
+    if (a.part) {  // four workgroups per (row, head), their states for the out-projection
+        if (!mz_cross_split(a.B, a.nh)) return hipErrorInvalidValue;
+        hipLaunchKernelGGL(dec_cross_split_kernel, dim3(8 * 4 * ((a.B * a.nh + 7) / 8)), dim3(256), 0, s, a);
+        return hipGetLastError();
+    }
     if (a.B * a.nh <= 256) {  // one workgroup per CU, all at once
         hipLaunchKernelGGL(dec_cross_wide_kernel, dim3(a.B * a.nh), dim3(256), 0, s, a);
         return hipGetLastError();

@@ -86,6 +86,14 @@ struct MzDec {
     int bs1, bs2, prompt_len;
     void* amax;  // int2 {float bits, id} [mz_lm_blocks(N)][M]
     int w_nt;    // projections: W read nontemporally (1) or with the default policy (0); the LM head always streams
+    // DEPI_PARTIAL with part set: x is the merged cross-attention states of dec_cross_split (K = nh * 64, K / ksplit <= 256,
+    // M <= 32), and the alignment rows' raw scores are normalised (fields as in MzDecCross)
+    const float* part;
+    int nh, maxT, na;
+    const int* done;
+    const int* aslot;
+    float* align;
+    f16* alignh;
 };
 hipError_t mz_dec_gemm_launch(hipStream_t s, int epi, const MzDec& g);
 // LM head workgroups (each with one argmax partial per row) and vocabulary tiles of 16 per workgroup
@@ -145,7 +153,14 @@ struct MzDecCross {
     float* align;      // [bmax][maxT][na][1500]
     f16* alignh;       // the same rows rounded to fp16 (may be null)
     int na;
+    // set (and mz_cross_split(B, nh)): the output goes here as four states of MZ_CROSS_STATE floats per (row, head), and the
+    // alignment rows hold raw scores, until the out-projection with the same part merges and normalises them
+    float* part;
 };
+#define MZ_CROSS_STATE 66
+#define MZ_CROSS_SPLIT_PAIRS 64
+// batches whose cross-attention is split: four workgroups per (row, head) still have a CU each
+inline bool mz_cross_split(int B, int nh) { return B * nh <= MZ_CROSS_SPLIT_PAIRS; }
 hipError_t mz_dec_cross_launch(hipStream_t s, const MzDecCross& a);
 
 // x[b] = xin[b] + sum_s parts[s][b] + bias; y[b] = LN(x[b])  (the residual add fused with the next layer norm;

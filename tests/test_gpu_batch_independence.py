@@ -83,3 +83,39 @@ def test_encoder_group_size_does_not_change_results(setup, parts):
             other.close()
         for c in range(N):
             same(got[c], ref[c], f"clip {c}, groups of {eg}")
+
+
+@pytest.mark.parametrize("d,nh,rows", [(128, 2, (33, 32, 5)), (384, 6, (11, 10, 1)), (1024, 16, (5, 4, 3))])
+def test_decoder_rows_alone_and_split(d, nh, rows):
+    """Batches on both sides of the border at which a row's cross-attention goes over four workgroups (64 rows x heads):
+    the same logits, residual and alignment rows (fp32 and fp16) bit for bit, for the rows they share, over a prompt and
+    some generated positions."""
+    from mimizuku_amd import _lib as L
+    g = synth.Geometry(d=d, ff=4 * d, nh=nh, enc_layers=1, dec_layers=2, n_mels=80, vocab=51865, max_t=32)
+    W = synth.random_weights(g, seed=nh, bias_std=0.02, ln_std=0.05)
+    heads = [[0, 1], [1, 0], [1, nh - 1]]
+    dims = model.Dims(g.d, g.ff, g.nh, g.enc_layers, g.dec_layers, g.n_mels, g.vocab, g.max_t)
+    gc = model.GenCfg.from_dict(synth.generation_config(g, align_heads=heads), dims)
+    ctx = model.Context(0)
+    e = model.Engine(ctx, dims, gc, max(rows), 1)
+    e.load(W)
+    mel = synth.synthetic_mel(max(rows), g.n_mels, seed=2)
+    for c in range(max(rows)):
+        e.encode(mel[c:c + 1], c)
+    steps, out = 9, []
+    for b in rows:
+        e.reset([[gc.sot, 50259 + i % 8, 50359, gc.no_timestamps] for i in range(b)])
+        for p in range(steps):
+            e.step(b, False, 4)
+        out.append((e.logits()[:b], e.dec_x()[:b], e.align()[:b, :steps], e.tokens()[:b, :steps + 1],
+                    e.read(L.BUF_ALIGN_H, np.float16, (max(rows), g.max_t, 3, 1500))[:b, :steps]))
+    assert np.isfinite(out[0][0]).all()
+    np.testing.assert_allclose(out[0][2].sum(-1), 1.0, atol=1e-4)
+    for o in out:
+        np.testing.assert_array_equal(o[4], o[2].astype(np.float16))
+    for b, o in zip(rows[1:], out[1:]):
+        k = min(b, rows[0])
+        for x, y in zip(o, out[0]):
+            np.testing.assert_array_equal(x[:k], y[:k], err_msg=f"{b} rows against {rows[0]}")
+    e.close()
+    ctx.close()
