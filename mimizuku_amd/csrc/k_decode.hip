@@ -240,8 +240,6 @@ typedef __attribute__((address_space(3))) void lds_void;
 
 // s_waitcnt operand that waits until at most n vector memory operations of this wave are outstanding (n < 64)
 constexpr int vm_wait(int n) { return (n & 15) | ((n >> 4) << 14) | (7 << 4) | (15 << 8); }
-// ... and no LDS operation is
-constexpr int vm_lgkm0_wait(int n) { return (n & 15) | ((n >> 4) << 14) | (7 << 4); }
 
 
 // Cache policy of the decoder's streams. The cross keys / values (983 MB per 32-row turbo step) and the LM head's
@@ -973,18 +971,18 @@ __global__ void __launch_bounds__(256, 1) dec_cross_wide_kernel(const MzDecCross
 
 // ---------------------------------------------------------------- cross-attention for the smallest batches
 
-// The same arithmetic for at most 256 / (4 nh) rows: four workgroups per (row, head), each one wave's eight groups of
+// The same arithmetic for at most 64 / nh rows: four workgroups per (row, head), each one wave's eight groups of
 // dec_attn_kernel (keys 8 s .. 8 s + 7 of every 32). What bounds a (row, head) on one CU is the CU's own rate for what
 // misses its caches (25 to 50 GB/s, whatever is in flight), so its 384 KB of keys and values go over four CUs. Each
 // projects the query for itself (its wq rows come from the L2 that the four share: they run on one XCD). The four
 // states (MZ_CROSS_STATE floats: 64 accumulators, maximum, sum) are merged by the out-projection that reads them, as
 // another launch for that would cost what the split gains. The four waves share the arithmetic that one would take 3 us
-// for: the scores by batches of keys, then the softmax by dims. One row: width 384 14.7 -> 9.1 us a layer, 1280 16.2 ->
-// 11.0, the out-projection 3.7 -> 4.0.
-__global__ void __launch_bounds__(256, 1) dec_cross_split_kernel(const MzDecCross a) {
+// for: the scores by batches of keys, then the softmax by dims. One row: width 384 14.7 -> 8.5 us a layer, 1280 16.2 ->
+// 9.9 (9.1 and 11.0 with the keys through LDS as well), the out-projection 3.7 -> 4.0.
+__global__ void __launch_bounds__(256, 2) dec_cross_split_kernel(const MzDecCross a) {
 #if defined(__HIP_DEVICE_COMPILE__)
     constexpr int L = MZ_TENC, NI = (L + 31) / 32, AU = 8, NJ = MZ_DEC_KSLICE / 64;
-    __shared__ __attribute__((aligned(16))) f16x8 ks[NI][64], vs[NI][64];  // [key / 32][lane]: 8 keys x 64 dims, 1 KB
+    __shared__ __attribute__((aligned(16))) f16x8 vs[NI][64];  // values: [key / 32][lane]: 8 keys x 64 dims, 1 KB
     __shared__ __attribute__((aligned(16))) f16 xs[MZ_DEC_KSLICE];
     __shared__ float qs[MZ_HD];
     __shared__ __attribute__((aligned(16))) float ss[8][NI + 5];  // scores: group, key / 32
@@ -1001,8 +999,9 @@ __global__ void __launch_bounds__(256, 1) dec_cross_split_kernel(const MzDecCros
     const long kv = (long)b * a.kv_b + (long)head * a.kv_h;
     const __amdgpu_buffer_rsrc_t rK = rsrc(a.k + kv, L * MZ_HD * 2), rV = rsrc(a.v + kv, L * MZ_HD * 2);
 
-    // in issue order: the row, this thread's chunks of wq (as dec_cross_wide_kernel), its two query biases, then this
-    // wave's share of the keys and values, straight into LDS (keys past the last read zeros)
+    // in issue order: the row, this thread's chunks of wq (as dec_cross_wide_kernel), its two query biases, the
+    // keys whose scores this wave takes, then its share of the values, straight into LDS (past the last key: zeros, no
+    // memory read)
     const bool xl = tid < (a.d >> 3);
     const f16x8 xv0 = xl ? *(const f16x8*)(a.xin + (long)b * a.d + tid * 8) : f16x8{};
     const f16* wr = a.wq + (long)(head * MZ_HD + 8 * wave + r8) * a.d + q8 * 8;
@@ -1015,14 +1014,18 @@ __global__ void __launch_bounds__(256, 1) dec_cross_split_kernel(const MzDecCros
     const unsigned short qb[2] = {__builtin_amdgcn_raw_buffer_load_b16(rQB, (unsigned)(head * MZ_HD + 8 * wave + r8) * 2u, 0, 0),
                                   __builtin_amdgcn_raw_buffer_load_b16(rQB, (unsigned)(head * MZ_HD + 32 + 8 * wave + r8) * 2u, 0, 0)};
     __builtin_amdgcn_sched_barrier(0);
-    auto stage = [&](const __amdgpu_buffer_rsrc_t r, f16x8(*dst)[64]) {
-        for (int i = wave; i < NI; i += 4)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(r, LDSP(&dst[i][0]), 16,
-                                                     (unsigned)((32 * i + 8 * split) * MZ_HD * 2) + lane * 16u, 0, 0, MZ_NT);
-    };
-    stage(rK, ks);
+    f16x8 K[2][AU];
+#pragma unroll
+    for (int h = 0; h < 2; h++)
+#pragma unroll
+        for (int u = 0; u < AU; u++)
+            K[h][u] = __builtin_bit_cast(
+                f16x8, __builtin_amdgcn_raw_buffer_load_b128(
+                           rK, (unsigned)((32 * (AU * (wave + 4 * h) + u) + 8 * split) * MZ_HD * 2) + lane * 16u, 0, MZ_NT));
     __builtin_amdgcn_sched_barrier(0);
-    stage(rV, vs);
+    for (int i = wave; i < NI; i += 4)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rV, LDSP(&vs[i][0]), 16,
+                                                 (unsigned)((32 * i + 8 * split) * MZ_HD * 2) + lane * 16u, 0, 0, MZ_NT);
     __builtin_amdgcn_sched_barrier(0);  // every request above is issued before anything waits for data
     if (done) {  // a finished row: no attention (the staged loads land before the LDS is released)
         __builtin_amdgcn_s_waitcnt(vm_wait(0));
@@ -1047,9 +1050,7 @@ __global__ void __launch_bounds__(256, 1) dec_cross_split_kernel(const MzDecCros
         const int i = 32 * h + 8 * wave + r8;
         if (q8 == 0) qs[i] = (t + (a.qbias ? (float)__builtin_bit_cast(f16, qb[h]) : 0.f)) * QS;
     }
-    // this wave's keys have landed (its 11 or 12 loads of values, issued after them, may be in flight), then every wave's
-    __builtin_amdgcn_s_waitcnt(vm_lgkm0_wait(11));
-    asm volatile("s_barrier" ::: "memory");
+    lds_barrier();  // the query
 
     // scores: group r8 has keys 8 split + r8 + 32 i; wave w takes dec_attn_kernel's batches w and w + 4 of eight i
     float* al = slot >= 0 && pos < a.maxT ? a.align + (((long)b * a.maxT + pos) * a.na + slot) * MZ_TENC : nullptr;
@@ -1057,15 +1058,15 @@ __global__ void __launch_bounds__(256, 1) dec_cross_split_kernel(const MzDecCros
         float q8v[8];
 #pragma unroll
         for (int e = 0; e < 8; e++) q8v[e] = qs[q8 * 8 + e];
-        for (int i0 = AU * wave; i0 < NI; i0 += 4 * AU) {
-            f16x8 K[AU];
 #pragma unroll
-            for (int u = 0; u < AU; u++) K[u] = ks[min(i0 + u, NI - 1)][lane];
+        for (int h = 0; h < 2; h++) {
+            const int i0 = AU * (wave + 4 * h);
+            if (i0 >= NI) break;
 #pragma unroll
             for (int u = 0; u < AU; u++) {
                 float t = 0.f;
 #pragma unroll
-                for (int e = 0; e < 8; e++) t = fmaf(q8v[e], (float)K[u][e], t);
+                for (int e = 0; e < 8; e++) t = fmaf(q8v[e], (float)K[h][u][e], t);
                 t = group8_sum(t);
                 const int j = 8 * split + r8 + 32 * (i0 + u);
                 if (q8 == 0) {

@@ -159,8 +159,11 @@ struct MzDecCross {
 };
 #define MZ_CROSS_STATE 66
 #define MZ_CROSS_SPLIT_PAIRS 64
-// batches whose cross-attention is split: four workgroups per (row, head) still have a CU each
-inline bool mz_cross_split(int B, int nh) { return B * nh <= MZ_CROSS_SPLIT_PAIRS; }
+// Batches whose cross-attention is split, four workgroups per (row, head): as long as those have a CU each. At two per CU
+// it is slower than one workgroup per (row, head) (steps of 2 layers, width 1280: 3 rows 140.9 -> 131.2 us, 4 rows 140.6 ->
+// 140.9, 6 rows 143.4 -> 144.4; width 384 at 21 rows 119.9, 22 rows unsplit 114.0). One block of 32 rows of the
+// out-projection merges them.
+inline bool mz_cross_split(int B, int nh) { return B <= 32 && B * nh <= MZ_CROSS_SPLIT_PAIRS; }
 hipError_t mz_dec_cross_launch(hipStream_t s, const MzDecCross& a);
 
 // x[b] = xin[b] + sum_s parts[s][b] + bias; y[b] = LN(x[b])  (the residual add fused with the next layer norm;
