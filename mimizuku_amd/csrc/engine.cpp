@@ -227,7 +227,7 @@ size_t weight_elems(const mz_dims& d, int* k1pad) {
 // one set of cross keys/values: [bmax][dec layers][k|v][heads] tiles of 1536 x 64
 size_t xkv_elems(const mz_dims& d, int bmax) { return (size_t)bmax * d.dec_layers * 2 * d.nh * (size_t)TPAD * HD; }
 
-constexpr size_t XPART = (size_t)MZ_CROSS_SPLIT_PAIRS * 4 * MZ_CROSS_STATE;  // floats of the split cross-attention's states
+constexpr size_t XPART = (size_t)MZ_CROSS_SPLIT_PAIRS * MZ_CROSS_STATE;  // floats of the split cross-attention's states
 
 int ksplit_for(int N, int K) {
     // Split K over workgroups until the grid covers most of the 256 CUs, with at most 16 groups of 64 per workgroup

@@ -205,24 +205,44 @@ __global__ void __launch_bounds__(512) dec_embed_ln_kernel(const int* __restrict
 
 // ---------------------------------------------------------------- merging softmax states
 
-// A query's groups of 8 lanes each hold an online softmax over their keys: maximum, sum, and 64 accumulators. They merge
-// in two levels, the same everywhere so that every form of the attention gives the same bits: the eight groups of a
-// wave in order, then the four waves' states in order. (A group or wave without keys: maximum -inf, no weight.)
-struct SoftmaxState {
-    float m, l, o;
+// A query's 32 groups of 8 lanes each hold an online softmax over their keys: maximum, sum, and 64 accumulators. One
+// wave merges them, a dim per lane, one group after the other in every form of the attention, so that all give the same
+// bits. (A group without keys: maximum -inf, no weight.) The serial part is two chains of 32 multiply-adds on values
+// that are all at hand: lane g works out group g's weight once (gm[g], gl[g] in lane g's m and l) and leaves it beside
+// the sum in this wave's 64 floats of LDS, from where they come back broadcast, four to a read. With the weights
+// worked out in the chain, an exp2 and three reads per group, a launch took 0.6 us longer (32 rows, width 1280).
+struct Merged {
+    float m, l;  // maximum and sum of the query
 };
-template <class Get>
-__device__ __forceinline__ SoftmaxState merge_states(int n, Get get) {
-    float m = -3.402823466e38f;
-    for (int g = 0; g < n; g++) m = fmaxf(m, get(g).m);
-    SoftmaxState r{m, 0.f, 0.f};
-    for (int g = 0; g < n; g++) {
-        const SoftmaxState s = get(g);
-        const float w = __builtin_amdgcn_exp2f(s.m - m);
-        r.l = fmaf(s.l, w, r.l);
-        r.o = fmaf(s.o, w, r.o);
+template <class Acc>
+__device__ __forceinline__ float merge_groups(float m, float l, float* ws, Merged& q, Acc acc) {
+    const int lane = threadIdx.x & 63;
+    q.m = wave_max(m);
+    ws[lane] = lane < 32 ? __builtin_amdgcn_exp2f(m - q.m) : l;
+    f32x4 w4[8], l4[8];
+#pragma unroll
+    for (int g = 0; g < 8; g++) {
+        w4[g] = *(const f32x4*)&ws[4 * g];
+        l4[g] = *(const f32x4*)&ws[32 + 4 * g];
     }
-    return r;
+    float o = 0.f;
+    q.l = 0.f;
+#pragma unroll
+    for (int g = 0; g < 32; g++) {
+        q.l = fmaf(l4[g >> 2][g & 3], w4[g >> 2][g & 3], q.l);
+        o = fmaf(acc(g), w4[g >> 2][g & 3], o);
+    }
+    return o;
+}
+// the same states in memory: accumulators [32][64], maxima, sums (MZ_CROSS_STATE floats)
+struct GroupStates {
+    float m, l, o[32];
+};
+__device__ __forceinline__ void load_states(const float* q, int lane, GroupStates& s) {
+    s.m = q[32 * MZ_HD + (lane & 31)];
+    s.l = q[32 * MZ_HD + 32 + (lane & 31)];
+#pragma unroll
+    for (int g = 0; g < 32; g++) s.o[g] = q[g * MZ_HD + lane];
 }
 
 // An alignment probability from a score in log2 units. The product is kept from being fused with a conversion: the fp16
@@ -260,8 +280,8 @@ constexpr int MZ_NT = 2;  // cache-policy bit of a buffer load: nontemporal
 // banks. The 4 waves split the K groups; their 32x32 products are summed in LDS. Every operand of the epilogue (bias,
 // mask, position) is requested at entry with the loads, so the kernel makes a single round trip to memory.
 // KS: the largest K slice of the launch (LDS sized to it: a workgroup asks for no more than it uses)
-// MERGE: x is the cross-attention's output, still in the four states per (row, head) that dec_cross_split_kernel leaves
-// (p.part): each workgroup merges its K slice's heads into the x block while its W rows are on their way, and the
+// MERGE: x is the cross-attention's output, still in the 32 group states per (row, head) that dec_cross_split_kernel
+// leaves (p.part): each workgroup merges its K slice's heads into the x block while its W rows are on their way, and the
 // alignment heads' raw scores become probabilities here, where the merged maximum and sum are known.
 template <int EPI, int KS, bool MERGE = false>
 __global__ void __launch_bounds__(256) dec_gemm_kernel(const MzDec p) {
@@ -282,6 +302,15 @@ __global__ void __launch_bounds__(256) dec_gemm_kernel(const MzDec p) {
     const unsigned ldx2 = (unsigned)p.ldx * 2u, mrows = (unsigned)min(p.M - m0, 32);
     const __amdgpu_buffer_rsrc_t rX = rsrc(p.x + (long)m0 * p.ldx, mrows * ldx2);
     const __amdgpu_buffer_rsrc_t rW = rsrc(p.W, (unsigned)p.N * (unsigned)p.K * 2u);
+    __shared__ __attribute__((aligned(16))) float ws[MERGE ? 4 : 1][64];
+    // the merge: wave w takes (row, head of the slice) pairs w, w + 4, ..., the first one's states requested ahead of W
+    const int nhs = ksl >> 6, npair = MERGE ? p.M * nhs : 0;
+    GroupStates st[2];
+    auto fetch = [&](int t, GroupStates& q) {
+        const int row = t / nhs, head = (kb >> 6) + t - row * nhs;
+        load_states(p.part + (long)(row * p.nh + head) * MZ_CROSS_STATE, lane, q);
+    };
+    if (MERGE && wave < npair) fetch(wave, st[0]);
     for (int i = wave; i < 4 * G; i += 4) {
         const int g = i >> 2, rg = i & 3, c = q8 ^ r8 ^ (rg & 1);
         const unsigned col = (unsigned)(kb + g * 64 + c * 8) * 2;
@@ -305,16 +334,18 @@ __global__ void __launch_bounds__(256) dec_gemm_kernel(const MzDec p) {
     }
     const int pos = EPI == DEPI_LOGITS || MERGE ? p.ctr[1] : 0;
     if (MERGE) {
-        auto state = [&](int ph, int i, int w) {
-            const float* q = p.part + (long)(ph * 4 + w) * MZ_CROSS_STATE;
-            return SoftmaxState{q[64], q[65], q[i]};
-        };
         // (rows past M keep what is in LDS: their columns of the product are not stored)
-        for (int e = tid; e < p.M * ksl; e += 256) {
-            const int row = e / ksl, k = e - row * ksl, head = (kb + k) >> 6, i = (kb + k) & 63;
-            const SoftmaxState t = merge_states(4, [&](int w) { return state(row * p.nh + head, i, w); });
-            const int rg = row >> 3, r = row & 7, c = (k & 63) >> 3;
-            sx[((k >> 6) * 4 + rg) * 512 + r * 64 + ((c ^ r ^ (rg & 1)) << 3) + (k & 7)] = (f16)(t.o / t.l);
+        auto put = [&](int t, const GroupStates& q) {
+            const int row = t / nhs, g = t - row * nhs, rg = row >> 3, r = row & 7, c = lane >> 3;
+            Merged t2;
+            const float o = merge_groups(q.m, q.l, ws[wave], t2, [&](int k) { return q.o[k]; });
+            sx[(g * 4 + rg) * 512 + r * 64 + ((c ^ r ^ (rg & 1)) << 3) + (lane & 7)] = (f16)(o / t2.l);
+        };
+        for (int t = wave; t < npair; t += 8) {
+            if (t + 4 < npair) fetch(t + 4, st[1]);
+            put(t, st[0]);
+            if (t + 8 < npair) fetch(t + 8, st[0]);
+            if (t + 4 < npair) put(t + 4, st[1]);
         }
         // the workgroups share the (row, head) pairs' alignment rows (usually one pair or none each)
         for (int pair = blockIdx.y * gridDim.x + blockIdx.x; pair < p.M * p.nh; pair += gridDim.x * gridDim.y) {
@@ -325,7 +356,9 @@ __global__ void __launch_bounds__(256) dec_gemm_kernel(const MzDec p) {
             const long ao = (((long)row * p.maxT + pos) * p.na + slot) * MZ_TENC;
 #pragma unroll
             for (int k = 0; k < NSC; k++) sc[k] = tid + 256 * k < MZ_TENC ? p.align[ao + tid + 256 * k] : 0.f;
-            const SoftmaxState t = merge_states(4, [&](int w) { return state(pair, 0, w); });
+            const float* q = p.part + (long)pair * MZ_CROSS_STATE + 32 * MZ_HD + (lane & 31);
+            Merged t;
+            merge_groups(q[0], q[32], ws[wave], t, [](int) { return 0.f; });
             const float inv = 1.f / t.l;
 #pragma unroll
             for (int k = 0; k < NSC; k++)
@@ -567,7 +600,8 @@ __global__ void __launch_bounds__(AG * 8) dec_attn_kernel(const MzDecAttn a) {
     __shared__ float sc[MZ_TPAD];
     __shared__ float gm[AG], gl[AG];
     __shared__ float gacc[AG][MZ_HD + 1];
-    __shared__ float wm[AG / 8], wl[AG / 8], wo[AG / 8][MZ_HD];
+    __shared__ __attribute__((aligned(16))) float ws[2 * AG];
+    static_assert(AG == 32, "merge_groups");
     __shared__ float tot[2];
     __shared__ __attribute__((aligned(16))) f16 kvn[2][MZ_HD];  // the step's own key and value (self, kw set)
 
@@ -734,22 +768,13 @@ __global__ void __launch_bounds__(AG * 8) dec_attn_kernel(const MzDecAttn a) {
 #pragma unroll
     for (int e = 0; e < 8; e++) gacc[grp][sub * 8 + e] = acc[e];
     __syncthreads();
-    {  // wave w merges its eight groups (dim i in lane i), then the first wave the four
-        const int w = tid >> 6, i = tid & 63;
-        const SoftmaxState t = merge_states(8, [&](int g) { return SoftmaxState{gm[8 * w + g], gl[8 * w + g], gacc[8 * w + g][i]}; });
-        wo[w][i] = t.o;
-        if (i == 0) {
-            wm[w] = t.m;
-            wl[w] = t.l;
-        }
-    }
-    __syncthreads();
     if (tid < MZ_HD) {
-        const SoftmaxState t = merge_states(4, [&](int w) { return SoftmaxState{wm[w], wl[w], wo[w][tid]}; });
-        a.out[(long)b * a.d + head * MZ_HD + tid] = (f16)(t.o / t.l);
+        Merged q;
+        const float o = merge_groups(gm[tid & 31], gl[tid & 31], ws, q, [&](int g) { return gacc[g][tid]; });
+        a.out[(long)b * a.d + head * MZ_HD + tid] = (f16)(o / q.l);
         if (tid == 0) {
-            tot[0] = t.m;
-            tot[1] = t.l;
+            tot[0] = q.m;
+            tot[1] = q.l;
         }
     }
     if (slot < 0 || pos >= a.maxT) return;
@@ -786,7 +811,8 @@ __global__ void __launch_bounds__(256, 1) dec_cross_wide_kernel(const MzDecCross
     __shared__ float sc[MZ_TPAD];
     __shared__ float gm[AG], gl[AG];
     __shared__ float gacc[AG][MZ_HD + 1];
-    __shared__ float wm[AG / 8], wl[AG / 8], wo[AG / 8][MZ_HD];
+    __shared__ __attribute__((aligned(16))) float ws[2 * AG];
+    static_assert(AG == 32, "merge_groups");
     __shared__ float tot[2];
 
     const int bh = blockIdx.x, b = bh / a.nh, head = bh - b * a.nh;
@@ -937,22 +963,13 @@ __global__ void __launch_bounds__(256, 1) dec_cross_wide_kernel(const MzDecCross
 #pragma unroll
     for (int e = 0; e < 8; e++) gacc[grp][sub * 8 + e] = acc[e];
     __syncthreads();
-    {  // wave w merges its eight groups (dim i in lane i), then the first wave the four
-        const int w = tid >> 6, i = tid & 63;
-        const SoftmaxState t = merge_states(8, [&](int g) { return SoftmaxState{gm[8 * w + g], gl[8 * w + g], gacc[8 * w + g][i]}; });
-        wo[w][i] = t.o;
-        if (i == 0) {
-            wm[w] = t.m;
-            wl[w] = t.l;
-        }
-    }
-    __syncthreads();
     if (tid < MZ_HD) {
-        const SoftmaxState t = merge_states(4, [&](int w) { return SoftmaxState{wm[w], wl[w], wo[w][tid]}; });
-        a.out[(long)b * a.d + head * MZ_HD + tid] = (f16)(t.o / t.l);
+        Merged q;
+        const float o = merge_groups(gm[tid & 31], gl[tid & 31], ws, q, [&](int g) { return gacc[g][tid]; });
+        a.out[(long)b * a.d + head * MZ_HD + tid] = (f16)(o / q.l);
         if (tid == 0) {
-            tot[0] = t.m;
-            tot[1] = t.l;
+            tot[0] = q.m;
+            tot[1] = q.l;
         }
     }
     if (slot < 0 || pos >= a.maxT) return;
@@ -974,9 +991,8 @@ __global__ void __launch_bounds__(256, 1) dec_cross_wide_kernel(const MzDecCross
 // The same arithmetic for at most 64 / nh rows: four workgroups per (row, head), each one wave's eight groups of
 // dec_attn_kernel (keys 8 s .. 8 s + 7 of every 32). What bounds a (row, head) on one CU is the CU's own rate for what
 // misses its caches (25 to 50 GB/s, whatever is in flight), so its 384 KB of keys and values go over four CUs. Each
-// projects the query for itself (its wq rows come from the L2 that the four share: they run on one XCD). The four
-// states (MZ_CROSS_STATE floats: 64 accumulators, maximum, sum) are merged by the out-projection that reads them, as
-// another launch for that would cost what the split gains. The four waves share the arithmetic that one would take 3 us
+// projects the query for itself (its wq rows come from the L2 that the four share: they run on one XCD). The groups'
+// states are merged by the out-projection that reads them, as another launch for that would cost what the split gains. The four waves share the arithmetic that one would take 3 us
 // for: the scores by batches of keys, then the softmax by dims. One row: width 384 14.7 -> 8.5 us a layer, 1280 16.2 ->
 // 9.9 (9.1 and 11.0 with the keys through LDS as well), the out-projection 3.7 -> 4.0.
 __global__ void __launch_bounds__(256, 2) dec_cross_split_kernel(const MzDecCross a) {
@@ -986,7 +1002,6 @@ __global__ void __launch_bounds__(256, 2) dec_cross_split_kernel(const MzDecCros
     __shared__ __attribute__((aligned(16))) f16 xs[MZ_DEC_KSLICE];
     __shared__ float qs[MZ_HD];
     __shared__ __attribute__((aligned(16))) float ss[8][NI + 5];  // scores: group, key / 32
-    __shared__ float gm[8], gl[8], gacc[8][MZ_HD + 1];
 
     const int xcd = blockIdx.x & 7, li = blockIdx.x >> 3, bh = (li >> 2) * 8 + xcd, split = li & 3;
     if (bh >= a.B * a.nh) return;
@@ -1105,20 +1120,13 @@ __global__ void __launch_bounds__(256, 2) dec_cross_split_kernel(const MzDecCros
         }
         m = mn;
     }
+    float* part = a.part + (long)bh * MZ_CROSS_STATE;
+    const int g = 8 * split + r8;
+    float* po = part + g * MZ_HD + q8 * 8 + 2 * wave;
+    *(float2*)po = make_float2(acc[0], acc[1]);
     if (q8 == 0 && wave == 0) {
-        gm[r8] = m;
-        gl[r8] = l;
-    }
-    gacc[r8][q8 * 8 + 2 * wave] = acc[0];
-    gacc[r8][q8 * 8 + 2 * wave + 1] = acc[1];
-    __syncthreads();
-    if (wave) return;
-    const SoftmaxState t = merge_states(8, [&](int g) { return SoftmaxState{gm[g], gl[g], gacc[g][lane]}; });
-    float* part = a.part + (long)(bh * 4 + split) * MZ_CROSS_STATE;
-    part[lane] = t.o;
-    if (lane == 0) {
-        part[64] = t.m;
-        part[65] = t.l;
+        part[32 * MZ_HD + g] = m;
+        part[32 * MZ_HD + 32 + g] = l;
     }
 #endif
 }

@@ -153,11 +153,12 @@ struct MzDecCross {
     float* align;      // [bmax][maxT][na][1500]
     f16* alignh;       // the same rows rounded to fp16 (may be null)
     int na;
-    // set (and mz_cross_split(B, nh)): the output goes here as four states of MZ_CROSS_STATE floats per (row, head), and the
-    // alignment rows hold raw scores, until the out-projection with the same part merges and normalises them
+    // set (and mz_cross_split(B, nh)): the output goes here as the 32 key groups' softmax states (MZ_CROSS_STATE floats
+    // per (row, head)), and the alignment rows hold raw scores, until the out-projection with the same part merges and
+    // normalises them
     float* part;
 };
-#define MZ_CROSS_STATE 66
+#define MZ_CROSS_STATE (32 * 66)
 #define MZ_CROSS_SPLIT_PAIRS 64
 // Batches whose cross-attention is split, four workgroups per (row, head): as long as those have a CU each. At two per CU
 // it is slower than one workgroup per (row, head) (steps of 2 layers, width 1280: 3 rows 140.9 -> 131.2 us, 4 rows 140.6 ->
