@@ -96,74 +96,90 @@ __global__ void __launch_bounds__(512) dec_add_ln_kernel(const float* xin, float
     ln_row4(v, on, dim, wv, bv, y + (long)row * dim, eps, red);
 }
 
-// LayerNorm of one row held by one wave, NC groups of VW floats per lane (v[i] = x[VW (lane + 64 i) ..]), written to y as
-// fp16: two-pass statistics over the wave through DPP and lane reads (no LDS, no barrier)
-template <int VW>
-struct Vec {
-    typedef float f __attribute__((ext_vector_type(VW)));
-    typedef f16 h __attribute__((ext_vector_type(VW)));
-};
-template <int VW, int NC>
-__device__ __forceinline__ void ln_wave(const typename Vec<VW>::f (&v)[NC], const typename Vec<VW>::h (&wv)[NC],
-                                        const typename Vec<VW>::h (&bv)[NC], f16* __restrict__ y, float eps) {
-    constexpr int dim = 64 * VW * NC;
+// LayerNorm of one row of DIM held by one wave (v[i] = x[4 (lane + 64 i) ..]; lanes with 4 (lane + 64 i) >= DIM hold
+// anything and store nothing), written to y as fp16: sums over the wave through DPP and lane reads, no LDS and no barrier.
+// DIM 1280: mean and squared deviations of the whole row, in two passes. The other widths: ln_row4's statistics, value by
+// value (each run of 256 columns, which is a wave there, has its own mean and squares, and they combine in order), so
+// that a row's bits do not depend on which kernel normalises it.
+template <int DIM>
+__device__ __forceinline__ void ln_wave(const f32x4 (&v)[(DIM + 255) / 256], const f16x4 (&wv)[(DIM + 255) / 256],
+                                        const f16x4 (&bv)[(DIM + 255) / 256], f16* __restrict__ y, float eps) {
+    constexpr int NC = (DIM + 255) / 256;
     const int lane = threadIdx.x & 63;
-    float sum = 0.f;
+    float mean = 0.f, var;
+    if constexpr (DIM == 1280) {
+        float sum = 0.f;
 #pragma unroll
-    for (int i = 0; i < NC; i++) {
-        if constexpr (VW == 4) sum += (v[i][0] + v[i][1]) + (v[i][2] + v[i][3]);
-        else sum += v[i][0] + v[i][1];
-    }
-    const float mean = wave_sum(sum) / dim;
-    float q = 0.f;
+        for (int i = 0; i < NC; i++) sum += (v[i][0] + v[i][1]) + (v[i][2] + v[i][3]);
+        mean = wave_sum(sum) / DIM;
+        float q = 0.f;
 #pragma unroll
-    for (int i = 0; i < NC; i++)
+        for (int i = 0; i < NC; i++)
 #pragma unroll
-        for (int e = 0; e < VW; e++) {
-            const float d = v[i][e] - mean;
-            q = fmaf(d, d, q);
+            for (int e = 0; e < 4; e++) {
+                const float d = v[i][e] - mean;
+                q = fmaf(d, d, q);
+            }
+        var = wave_sum(q) / DIM;
+    } else {
+        float mk[NC], qk[NC], m2 = 0.f;
+#pragma unroll
+        for (int i = 0; i < NC; i++) {
+            const bool on = 4 * (lane + 64 * i) < DIM;
+            mk[i] = wave_sum(on ? v[i][0] + v[i][1] + v[i][2] + v[i][3] : 0.f) / (float)min(256, DIM - 256 * i);
+            const float ex = v[i][0] - mk[i], ey = v[i][1] - mk[i], ez = v[i][2] - mk[i], ew = v[i][3] - mk[i];
+            qk[i] = wave_sum(on ? ex * ex + ey * ey + ez * ez + ew * ew : 0.f);
         }
-    const float rstd = rsqrtf(wave_sum(q) / dim + eps);
+#pragma unroll
+        for (int i = 0; i < NC; i++) mean += (float)min(256, DIM - 256 * i) * mk[i];
+        mean /= DIM;
+#pragma unroll
+        for (int i = 0; i < NC; i++) {
+            const float d = mk[i] - mean;
+            m2 += qk[i] + (float)min(256, DIM - 256 * i) * d * d;
+        }
+        var = m2 / DIM;
+    }
+    const float rstd = rsqrtf(var + eps);
 #pragma unroll
     for (int i = 0; i < NC; i++) {
-        typename Vec<VW>::h o;
+        float o[4];
 #pragma unroll
-        for (int e = 0; e < VW; e++) o[e] = (f16)((v[i][e] - mean) * rstd * (float)wv[i][e] + (float)bv[i][e]);
-        *(typename Vec<VW>::h*)(y + (lane + 64 * i) * VW) = o;
+        for (int e = 0; e < 4; e++) o[e] = (v[i][e] - mean) * rstd * (float)wv[i][e] + (float)bv[i][e];
+        if (4 * (lane + 64 * i) < DIM) st4(y + (lane + 64 * i) * 4, o[0], o[1], o[2], o[3]);
     }
 }
 
-// dec_add_ln_kernel's work with one wave per row for NC groups of VW floats per lane (dim = 64 VW NC) and NP partials:
-// every load of the row (residual, partials, bias, gamma, beta) is issued before the first use, the residual is summed in
-// dec_add_ln_kernel's order (the same x), and the LayerNorm statistics are two-pass sums over the wave through DPP and
-// lane reads, so no barrier and no LDS are needed. Bound by the launch and one round trip.
-template <int VW, int NC, int NP>
+// dec_add_ln_kernel's work with one wave per row of DIM and NP partials: every load of the row (residual, partials, bias,
+// gamma, beta) is issued before the first use, the residual is summed in dec_add_ln_kernel's order (the same x), and the
+// statistics are ln_wave's. Bound by the launch and one round trip.
+template <int DIM, int NP>
 __global__ void __launch_bounds__(64) dec_add_ln_wave_kernel(const float* xin, float* x, const float* __restrict__ parts,
                                                               long part_stride, const f16* __restrict__ bias,
                                                               const f16* __restrict__ w, const f16* __restrict__ b,
                                                               f16* __restrict__ y, float eps) {
 #if defined(__HIP_DEVICE_COMPILE__)
-    typedef typename Vec<VW>::f vf;
-    typedef typename Vec<VW>::h vh;
-    constexpr int dim = 64 * VW * NC;
+    constexpr int NC = (DIM + 255) / 256;
     const int row = blockIdx.x, lane = threadIdx.x;
-    const long r0 = (long)row * dim;
-    vf v[NC], pp[NP][NC];
-    vh bb[NC], wv[NC], bv[NC];
+    const long r0 = (long)row * DIM;
+    // (a last run of fewer than 256 columns: the lanes past it read the row's last four)
+    int c[NC];
 #pragma unroll
-    for (int i = 0; i < NC; i++) v[i] = *(const vf*)(xin + r0 + (lane + 64 * i) * VW);
+    for (int i = 0; i < NC; i++) c[i] = min(4 * (lane + 64 * i), DIM - 4);
+    f32x4 v[NC], pp[NP][NC];
+    f16x4 bb[NC], wv[NC], bv[NC];
+#pragma unroll
+    for (int i = 0; i < NC; i++) v[i] = *(const f32x4*)(xin + r0 + c[i]);
 #pragma unroll
     for (int s = 0; s < NP; s++)
 #pragma unroll
-        for (int i = 0; i < NC; i++) pp[s][i] = *(const vf*)(parts + s * part_stride + r0 + (lane + 64 * i) * VW);
-    const __amdgpu_buffer_rsrc_t rB = rsrc(bias, bias ? (unsigned)dim * 2u : 0u);
+        for (int i = 0; i < NC; i++) pp[s][i] = *(const f32x4*)(parts + s * part_stride + r0 + c[i]);
+    const __amdgpu_buffer_rsrc_t rB = rsrc(bias, bias ? (unsigned)DIM * 2u : 0u);
 #pragma unroll
     for (int i = 0; i < NC; i++) {
-        const unsigned o = (unsigned)(lane + 64 * i) * VW * 2u;
-        if constexpr (VW == 4) bb[i] = __builtin_bit_cast(vh, __builtin_amdgcn_raw_buffer_load_b64(rB, o, 0, 0));
-        else bb[i] = __builtin_bit_cast(vh, __builtin_amdgcn_raw_buffer_load_b32(rB, o, 0, 0));
-        wv[i] = *(const vh*)(w + (lane + 64 * i) * VW);
-        bv[i] = *(const vh*)(b + (lane + 64 * i) * VW);
+        bb[i] = __builtin_bit_cast(f16x4, __builtin_amdgcn_raw_buffer_load_b64(rB, (unsigned)c[i] * 2u, 0, 0));
+        wv[i] = *(const f16x4*)(w + c[i]);
+        bv[i] = *(const f16x4*)(b + c[i]);
     }
     __builtin_amdgcn_sched_barrier(0);  // every request above is issued before anything waits for data
 #pragma unroll
@@ -171,10 +187,10 @@ __global__ void __launch_bounds__(64) dec_add_ln_wave_kernel(const float* xin, f
 #pragma unroll
         for (int s = 0; s < NP; s++) v[i] += pp[s][i];
 #pragma unroll
-        for (int e = 0; e < VW; e++) v[i][e] += (float)bb[i][e];
-        *(vf*)(x + r0 + (lane + 64 * i) * VW) = v[i];
+        for (int e = 0; e < 4; e++) v[i][e] += (float)bb[i][e];
+        if (4 * (lane + 64 * i) < DIM) *(f32x4*)(x + r0 + c[i]) = v[i];
     }
-    ln_wave<VW, NC>(v, wv, bv, y + r0, eps);
+    ln_wave<DIM>(v, wv, bv, y + r0, eps);
 #endif
 }
 
@@ -1284,14 +1300,14 @@ hipError_t mz_dec_add_ln_launch(hipStream_t s, const float* xin, float* x, const
         return hipGetLastError();
     };
     switch (dim * 100 + nparts) {
-        case 38406: return wave(dec_add_ln_wave_kernel<2, 3, 6>);
-        case 38412: return wave(dec_add_ln_wave_kernel<2, 3, 12>);
-        case 51208: return wave(dec_add_ln_wave_kernel<4, 2, 8>);
-        case 51216: return wave(dec_add_ln_wave_kernel<4, 2, 16>);
-        case 76808: return wave(dec_add_ln_wave_kernel<4, 3, 8>);
-        case 76812: return wave(dec_add_ln_wave_kernel<4, 3, 12>);
-        case 102408: return wave(dec_add_ln_wave_kernel<4, 4, 8>);
-        case 128005: return wave(dec_add_ln_wave_kernel<4, 5, 5>);
+        case 38406: return wave(dec_add_ln_wave_kernel<384, 6>);
+        case 38412: return wave(dec_add_ln_wave_kernel<384, 12>);
+        case 51208: return wave(dec_add_ln_wave_kernel<512, 8>);
+        case 51216: return wave(dec_add_ln_wave_kernel<512, 16>);
+        case 76808: return wave(dec_add_ln_wave_kernel<768, 8>);
+        case 76812: return wave(dec_add_ln_wave_kernel<768, 12>);
+        case 102408: return wave(dec_add_ln_wave_kernel<1024, 8>);
+        case 128005: return wave(dec_add_ln_wave_kernel<1280, 5>);
     }
     hipLaunchKernelGGL(dec_add_ln_kernel, dim3(rows), dim3(row_threads(dim)), 0, s, xin, x, parts, nparts, part_stride,
                        bias, w, b, y, dim, eps);

@@ -127,3 +127,33 @@ def test_self_attention_merges_groups_in_order(ctx):
                 other = np.concatenate([merged_by_waves(v[b, h, :pos + 1]) for h in range(2)])
                 assert (want != other).mean() > 0.3
     e.close()
+
+
+# ---------------------------------------------------------------- layer norms: one row, whichever kernel takes it
+
+@pytest.mark.parametrize("d", [384, 512, 768, 1024])
+def test_layer_norms_of_one_row_agree(ctx, d):
+    """The first layer norm of a step (in the embedding's kernel, one workgroup per row) and the last one (after the
+    residual add, one wave per row at these widths) of the same row with the same weights are the same bits: the first
+    comes back through an identity k_proj as the position's key, the last through the identity part of the tied embedding
+    as logits. The weights cancel most of each result, so that fp16 shows the statistics' last places."""
+    rng = np.random.default_rng(d)
+    emb = np.zeros((1536, d), np.float16)
+    emb[:d] = np.eye(d)
+    rows = emb[d:d + 32]  # alike to 2^-10, so that one set of weights cancels all of them
+    rows[:] = (rng.standard_normal(d) * 1.5 + 0.3 + rng.standard_normal((32, d)) * 2.0 ** -10).astype(np.float16)
+    gamma = np.full(d, 4096.0, np.float16)
+    x = rows[0].astype(np.float64)
+    beta = (-4096.0 * (x - x.mean()) / np.sqrt(x.var() + 1e-5)).astype(np.float16)
+    ln = {DEC + "self_attn_layer_norm.", "model.decoder.layer_norm."}
+    w = {p + "weight": gamma for p in ln} | {p + "bias": beta for p in ln}
+    w |= {DEC + "self_attn.k_proj.weight": np.eye(d, dtype=np.float16), "model.decoder.embed_tokens.weight": emb}
+    e = engine(ctx, d, 32, w, max_t=16)
+    e.reset([[d + b, d] for b in range(32)])
+    e.step(32, False, 2)
+    np.testing.assert_array_equal(e.dec_x(), rows.astype(f32))
+    keys = e.self_kv()[0][0, :, :, 0].reshape(32, d)
+    got = e.logits()[:, :d]
+    assert np.abs(got).max() <= 64 and np.ptp(got[0]) > 1
+    np.testing.assert_array_equal(got, keys.astype(f32))
+    e.close()
