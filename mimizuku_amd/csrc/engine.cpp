@@ -863,6 +863,7 @@ static int step_impl(mz_engine* e, int b, int lang, int prompt_len) {
             MzDec g = gemm_args(e->datt, D, L.xo, D, D, ks_dd, e->part, D);
             if (xsplit) {
                 g.part = e->xpart;
+                g.xout = e->datt;
                 g.nh = nh;
                 g.maxT = mt;
                 g.na = e->na;

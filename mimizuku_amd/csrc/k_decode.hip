@@ -253,6 +253,7 @@ __device__ __forceinline__ float merge_groups(float m, float l, float* ws, Merge
 // the same states in memory: accumulators [32][64], maxima, sums (MZ_CROSS_STATE floats)
 struct GroupStates {
     float m, l, o[32];
+    bool done;  // a finished row: no states
 };
 __device__ __forceinline__ void load_states(const float* q, int lane, GroupStates& s) {
     s.m = q[32 * MZ_HD + (lane & 31)];
@@ -298,7 +299,9 @@ constexpr int MZ_NT = 2;  // cache-policy bit of a buffer load: nontemporal
 // KS: the largest K slice of the launch (LDS sized to it: a workgroup asks for no more than it uses)
 // MERGE: x is the cross-attention's output, still in the 32 group states per (row, head) that dec_cross_split_kernel
 // leaves (p.part): each workgroup merges its K slice's heads into the x block while its W rows are on their way, and the
-// alignment heads' raw scores become probabilities here, where the merged maximum and sum are known.
+// alignment heads' raw scores become probabilities here, where the merged maximum and sum are known. A finished row has no
+// states: as in the other forms of the attention its x is what its last step left in p.xout, where the first workgroup
+// of each K slice puts the merged rows for that.
 template <int EPI, int KS, bool MERGE = false>
 __global__ void __launch_bounds__(256) dec_gemm_kernel(const MzDec p) {
 #if defined(__HIP_DEVICE_COMPILE__)  // the buffer-resource type exists only in the device pass
@@ -325,6 +328,7 @@ __global__ void __launch_bounds__(256) dec_gemm_kernel(const MzDec p) {
     auto fetch = [&](int t, GroupStates& q) {
         const int row = t / nhs, head = (kb >> 6) + t - row * nhs;
         load_states(p.part + (long)(row * p.nh + head) * MZ_CROSS_STATE, lane, q);
+        q.done = p.done[row] != 0;
     };
     if (MERGE && wave < npair) fetch(wave, st[0]);
     for (int i = wave; i < 4 * G; i += 4) {
@@ -355,7 +359,11 @@ __global__ void __launch_bounds__(256) dec_gemm_kernel(const MzDec p) {
             const int row = t / nhs, g = t - row * nhs, rg = row >> 3, r = row & 7, c = lane >> 3;
             Merged t2;
             const float o = merge_groups(q.m, q.l, ws[wave], t2, [&](int k) { return q.o[k]; });
-            sx[(g * 4 + rg) * 512 + r * 64 + ((c ^ r ^ (rg & 1)) << 3) + (lane & 7)] = (f16)(o / t2.l);
+            f16* xo = p.xout + (long)row * p.ldx + kb + g * MZ_HD + lane;
+            f16 x = (f16)(o / t2.l);
+            if (q.done) x = *xo;
+            else if (blockIdx.x == 0) *xo = x;  // (a row is only read or only written)
+            sx[(g * 4 + rg) * 512 + r * 64 + ((c ^ r ^ (rg & 1)) << 3) + (lane & 7)] = x;
         };
         for (int t = wave; t < npair; t += 8) {
             if (t + 4 < npair) fetch(t + 4, st[1]);
@@ -1209,7 +1217,7 @@ hipError_t mz_dec_gemm_launch(hipStream_t s, int epi, const MzDec& g) {
     switch (epi) {
         case DEPI_PARTIAL:
             if (g.part) {  // the cross-attention's states as x
-                if (g.M > 32 || !g.done || !g.ctr || !g.aslot || !g.align || g.K != g.nh * MZ_HD || ksl % 64) return hipErrorInvalidValue;
+                if (g.M > 32 || !g.xout || !g.done || !g.ctr || !g.aslot || !g.align || g.K != g.nh * MZ_HD || ksl % 64) return hipErrorInvalidValue;
                 if (ksl > 256) return hipErrorInvalidValue;
                 hipLaunchKernelGGL((dec_gemm_kernel<DEPI_PARTIAL, 256, true>), grid, dim3(256), 0, s, g);
                 break;

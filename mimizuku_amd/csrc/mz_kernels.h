@@ -87,8 +87,10 @@ struct MzDec {
     void* amax;  // int2 {float bits, id} [mz_lm_blocks(N)][M]
     int w_nt;    // projections: W read nontemporally (1) or with the default policy (0); the LM head always streams
     // DEPI_PARTIAL with part set: x is the merged cross-attention states of dec_cross_split (K = nh * 64, K / ksplit <= 256,
-    // M <= 32), and the alignment rows' raw scores are normalised (fields as in MzDecCross)
+    // M <= 32), and the alignment rows' raw scores are normalised (fields as in MzDecCross). The merged rows go to xout
+    // too (row stride ldx), from where a finished row keeps its last ones, as if the attention had written there.
     const float* part;
+    f16* xout;
     int nh, maxT, na;
     const int* done;
     const int* aslot;

@@ -119,3 +119,36 @@ def test_decoder_rows_alone_and_split(d, nh, rows):
             np.testing.assert_array_equal(x[:k], y[:k], err_msg=f"{b} rows against {rows[0]}")
     e.close()
     ctx.close()
+
+
+@pytest.mark.parametrize("d,nh,rows", [(128, 2, (32, 33)), (384, 6, (10, 11)), (1280, 20, (3, 4))])
+def test_finished_rows_alone_and_split(d, nh, rows):
+    """Rows that are finished, one before an engine's first step and one between steps, on both sides of that border: every
+    value stays finite and the rows that both batches have, the finished ones among them, are the same bits."""
+    from mimizuku_amd import _lib as L
+    g = synth.Geometry(d=d, ff=4 * d, nh=nh, enc_layers=1, dec_layers=2, n_mels=80, vocab=51865, max_t=32)
+    W = synth.random_weights(g, seed=nh, bias_std=0.02, ln_std=0.05)
+    dims = model.Dims(g.d, g.ff, g.nh, g.enc_layers, g.dec_layers, g.n_mels, g.vocab, g.max_t)
+    gc = model.GenCfg.from_dict(synth.generation_config(g, align_heads=[[0, 1], [1, 0], [1, nh - 1]]), dims)
+    mel = synth.synthetic_mel(1, g.n_mels, seed=2)
+    ctx, out = model.Context(0), []
+    for b in rows:
+        e = model.Engine(ctx, dims, gc, b, 1)
+        e.load(W)
+        for c in range(b):
+            e.encode(mel, c)
+        e.reset([[gc.sot, 50259 + i % 8, 50359, gc.no_timestamps] for i in range(b)])
+        for p in range(6):
+            for step, row in ((0, 0), (3, 2)):
+                if p == step:
+                    ctx.upload(e.buffer(L.BUF_DONE)[0] + 4 * row, np.ones(1, np.int32))
+            e.step(b, False, 4)
+            k = min(rows)
+            out.append([a[:k] for a in (e.logits(), e.dec_x(), e.align(), e.tokens(), e.done())])
+        e.close()
+    ctx.close()
+    assert out[5][4][0] == 1 and out[5][4][2] == 1
+    for p in range(6):
+        for x, y in zip(out[p], out[6 + p]):
+            assert np.isfinite(x).all() and np.isfinite(y).all(), f"step {p}"
+            np.testing.assert_array_equal(x, y, err_msg=f"step {p}")
