@@ -93,6 +93,9 @@ __device__ __forceinline__ void gemm_epilogue(const MzGemm& p, const f32x16 (&ac
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lr = lane & 31, lh = lane >> 5;
     if (EPI == EPI_HEADS) {
         if (p.kind == 3) lds_barrier();  // every wave is done reading operands: LDS is free for the v transposes
+        // a partial last column tile: this wave has no head block (64 | N, so a wave's columns all exist or none does), and
+        // what lies a clip's blocks further is the next clip's
+        if (n0 >= p.N) return;
         const int blk = n0 >> 6;           // a wave's columns lie in one 64-wide head block (WN <= 64)
         const bool vt = p.kind == 3 && blk / p.nh == 2;
         if (vt) {

@@ -85,6 +85,28 @@ def test_encoder_group_size_does_not_change_results(setup, parts):
             same(got[c], ref[c], f"clip {c}, groups of {eg}")
 
 
+@pytest.mark.parametrize("d,clips", [(384, 5), (384, 8), (640, 3), (640, 6)])
+def test_encoder_of_odd_widths_in_one_group(d, clips):
+    """Widths whose QKV product ends in a partial column tile: a group of clips encodes to the bits of each clip alone."""
+    g = synth.Geometry(d=d, ff=4 * d, nh=d // 64, enc_layers=1, dec_layers=1, n_mels=80, vocab=51865, max_t=16)
+    dims = model.Dims(g.d, g.ff, g.nh, g.enc_layers, g.dec_layers, g.n_mels, g.vocab, g.max_t)
+    gc = model.GenCfg(sot=3, eos=2, no_timestamps=6, langs=[("en", 4)], tasks=[("transcribe", 5)], suppress=[],
+                      begin_suppress=[], align_heads=[(0, 1)])
+    ctx = model.Context(0)
+    e = model.Engine(ctx, dims, gc, clips, clips)
+    e.load(synth.random_weights(g, seed=d, bias_std=0.02, ln_std=0.05))
+    mel = synth.synthetic_mel(clips, g.n_mels, seed=4)
+    e.encode(mel, 0)
+    group = e.enc_out(clips).copy(), e.xkv()
+    assert np.isfinite(group[0]).all()
+    for c in range(clips):
+        e.encode(mel[c:c + 1], c)
+        np.testing.assert_array_equal(e.enc_out(1)[0], group[0][c], err_msg=f"clip {c}")
+    np.testing.assert_array_equal(e.xkv(), group[1])
+    e.close()
+    ctx.close()
+
+
 @pytest.mark.parametrize("d,nh,rows", [(128, 2, (33, 32, 5)), (384, 6, (11, 10, 1)), (1024, 16, (5, 4, 3))])
 def test_decoder_rows_alone_and_split(d, nh, rows):
     """Batches on both sides of the border at which a row's cross-attention goes over four workgroups (64 rows x heads):

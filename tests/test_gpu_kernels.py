@@ -304,6 +304,33 @@ def test_gemm_head_scatter(ctx, kind):
         ctx.free(p)
 
 
+@pytest.mark.parametrize("kind,nh,clips,blocks", [(3, 6, 5, 18), (2, 1, 6, 7), (3, 1, 6, 3)])
+def test_gemm_head_scatter_partial_columns(ctx, kind, nh, clips, blocks):
+    """Head counts that leave the last column tile partial (1152 columns in 256 x 256 tiles, 448 in 256 x 128, 192 in
+    128 x 128): the columns past the last head write nothing. Each clip has two more tiles than the product has heads, which
+    must stay as they were, as must every tile's padding."""
+    rng = np.random.default_rng(blocks)
+    n, k, m, bpc = blocks * 64, 128, clips * 1500, blocks + 2
+    x, w, b = f16(rng, (m, k)), f16(rng, (n, k), 0.1), f16(rng, (n,), 0.1)
+    dx, dw, db = (ctx.upload_new(a) for a in (x, w, b))
+    dh = ctx.upload_new(np.full((clips, bpc, TPAD * 64), 7, np.float16))
+    L.check(L.lib().mz_linear(ctx.h, linear_args(epilogue=L.EPI_HEADS, a=dx, lda=k, w=dw, bias=db, m=m, n=n, k=k,
+                                                 heads=dh, blocks_per_clip=bpc, nh=nh, kind=kind, slot0=0)))
+    got = ctx.download(dh, (clips, bpc, TPAD * 64), np.float16)
+    assert (got[:, blocks:] == 7).all(), "a tile past the last head was written"
+    ref = (x.astype(np.float64) @ w.astype(np.float64).T + b).reshape(clips, 1500, blocks, 64)
+    if kind == 3:
+        ref[:, :, :nh] *= QSCALE
+    for c in range(clips):
+        for blk in range(blocks):
+            v = kind == 3 and blk // nh == 2
+            tile = got[c, blk].reshape(64, TPAD).T if v else got[c, blk].reshape(TPAD, 64)
+            assert (tile[1500:] == 7).all()
+            assert_f16(tile[:1500], ref[c, :, blk])
+    for p in (dx, dw, db, dh):
+        ctx.free(p)
+
+
 def test_gemm_large_qkv_shape(ctx):
     """The encoder group's fused QKV product, M = 12000, N = 3840, K = 1280, 256 rows checked."""
     rng = np.random.default_rng(5)
