@@ -125,7 +125,7 @@ __device__ __forceinline__ void ln_wave(const f32x4 (&v)[(DIM + 255) / 256], con
         float mk[NC], qk[NC], m2 = 0.f;
 #pragma unroll
         for (int i = 0; i < NC; i++) {
-            const bool on = 4 * (lane + 64 * i) < DIM;
+            const bool on = 256 * (i + 1) <= DIM || 4 * lane + 256 * i < DIM;
             mk[i] = wave_sum(on ? v[i][0] + v[i][1] + v[i][2] + v[i][3] : 0.f) / (float)min(256, DIM - 256 * i);
             const float ex = v[i][0] - mk[i], ey = v[i][1] - mk[i], ez = v[i][2] - mk[i], ew = v[i][3] - mk[i];
             qk[i] = wave_sum(on ? ex * ex + ey * ey + ez * ez + ew * ew : 0.f);
@@ -146,7 +146,7 @@ __device__ __forceinline__ void ln_wave(const f32x4 (&v)[(DIM + 255) / 256], con
         float o[4];
 #pragma unroll
         for (int e = 0; e < 4; e++) o[e] = (v[i][e] - mean) * rstd * (float)wv[i][e] + (float)bv[i][e];
-        if (4 * (lane + 64 * i) < DIM) st4(y + (lane + 64 * i) * 4, o[0], o[1], o[2], o[3]);
+        if (256 * (i + 1) <= DIM || 4 * lane + 256 * i < DIM) st4(y + (lane + 64 * i) * 4, o[0], o[1], o[2], o[3]);
     }
 }
 
@@ -162,10 +162,11 @@ __global__ void __launch_bounds__(64) dec_add_ln_wave_kernel(const float* xin, f
     constexpr int NC = (DIM + 255) / 256;
     const int row = blockIdx.x, lane = threadIdx.x;
     const long r0 = (long)row * DIM;
-    // (a last run of fewer than 256 columns: the lanes past it read the row's last four)
+    // (a last run of fewer than 256 columns: the lanes past it read the row's last four. The whole runs keep a constant
+    // distance, which goes into the loads' immediate offsets: with the bound on all of them a launch took 0.3 us longer)
     int c[NC];
 #pragma unroll
-    for (int i = 0; i < NC; i++) c[i] = min(4 * (lane + 64 * i), DIM - 4);
+    for (int i = 0; i < NC; i++) c[i] = 256 * (i + 1) <= DIM ? 4 * lane + 256 * i : min(4 * lane + 256 * i, DIM - 4);
     f32x4 v[NC], pp[NP][NC];
     f16x4 bb[NC], wv[NC], bv[NC];
 #pragma unroll
@@ -188,7 +189,7 @@ __global__ void __launch_bounds__(64) dec_add_ln_wave_kernel(const float* xin, f
         for (int s = 0; s < NP; s++) v[i] += pp[s][i];
 #pragma unroll
         for (int e = 0; e < 4; e++) v[i][e] += (float)bb[i][e];
-        if (4 * (lane + 64 * i) < DIM) *(f32x4*)(x + r0 + c[i]) = v[i];
+        if (256 * (i + 1) <= DIM || 4 * lane + 256 * i < DIM) *(f32x4*)(x + r0 + c[i]) = v[i];
     }
     ln_wave<DIM>(v, wv, bv, y + r0, eps);
 #endif
