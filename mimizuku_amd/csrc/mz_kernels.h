@@ -162,11 +162,16 @@ struct MzDecCross {
 };
 #define MZ_CROSS_STATE (32 * 66)
 #define MZ_CROSS_SPLIT_PAIRS 64
-// Batches whose cross-attention is split, four workgroups per (row, head): as long as those have a CU each. At two per CU
-// it is slower than one workgroup per (row, head) (steps of 2 layers, width 1280: 3 rows 140.9 -> 131.2 us, 4 rows 140.6 ->
-// 140.9, 6 rows 143.4 -> 144.4; width 384 at 21 rows 119.9, 22 rows unsplit 114.0). One block of 32 rows of the
-// out-projection merges them.
-inline bool mz_cross_split(int B, int nh) { return B <= 32 && B * nh <= MZ_CROSS_SPLIT_PAIRS; }
+#define MZ_CROSS_SPLIT_ROWS 12
+// Batches whose cross-attention is split, four workgroups per (row, head): as long as those have a CU each (a quarter of
+// the CUs, and at most MZ_CROSS_SPLIT_PAIRS pairs, which the states' buffer holds). At two per CU it is slower than one
+// workgroup per (row, head) (steps of 2 layers, width 1280: 4 rows 140.6 -> 140.9 us, 6 rows 143.4 -> 144.4). And as long
+// as the rows are few: each workgroup of the out-projection merges every row of its K slice, four at a time (steps of 4
+// layers, split against not: 2 heads at 12 rows 171.5 / 175.0, 16 rows 178.8 / 176.4, 32 rows 216.2 / 182.9; 6 heads at
+// 10 rows 192.6 / 197.2, 20 heads at 3 rows 232.1 / 242.4).
+inline bool mz_cross_split(int B, int nh) {
+    return B <= MZ_CROSS_SPLIT_ROWS && B * nh <= MZ_CROSS_SPLIT_PAIRS && 4 * B * nh <= mz_cu_count();
+}
 hipError_t mz_dec_cross_launch(hipStream_t s, const MzDecCross& a);
 
 // x[b] = xin[b] + sum_s parts[s][b] + bias; y[b] = LN(x[b])  (the residual add fused with the next layer norm;

@@ -107,9 +107,10 @@ def test_encoder_of_odd_widths_in_one_group(d, clips):
     ctx.close()
 
 
-@pytest.mark.parametrize("d,nh,rows", [(128, 2, (33, 32, 5)), (384, 6, (11, 10, 1)), (1024, 16, (5, 4, 3))])
+@pytest.mark.parametrize("d,nh,rows", [(128, 2, (33, 32, 5)), (128, 2, (13, 12, 5)), (384, 6, (11, 10, 1)), (1024, 16, (5, 4, 3))])
 def test_decoder_rows_alone_and_split(d, nh, rows):
-    """Batches on both sides of the border at which a row's cross-attention goes over four workgroups (64 rows x heads):
+    """Batches on both sides of the borders at which a row's cross-attention goes over four workgroups (64 (row, head)
+    pairs, 12 rows):
     the same logits, residual and alignment rows (fp32 and fp16) bit for bit, for the rows they share, over a prompt and
     some generated positions."""
     from mimizuku_amd import _lib as L
@@ -143,7 +144,7 @@ def test_decoder_rows_alone_and_split(d, nh, rows):
     ctx.close()
 
 
-@pytest.mark.parametrize("d,nh,rows", [(128, 2, (32, 33)), (384, 6, (10, 11)), (1280, 20, (3, 4))])
+@pytest.mark.parametrize("d,nh,rows", [(128, 2, (12, 13)), (384, 6, (10, 11)), (1280, 20, (3, 4))])
 def test_finished_rows_alone_and_split(d, nh, rows):
     """Rows that are finished, one before an engine's first step and one between steps, on both sides of that border: every
     value stays finite and the rows that both batches have, the finished ones among them, are the same bits."""

@@ -74,9 +74,9 @@ def merged_by_waves(v):
     return (chain(np.stack([chain(a) for a in group_sums(v).reshape(4, 8, 64)])) / f32(len(v))).astype(np.float16)
 
 
-@pytest.mark.parametrize("rows", [1, 32, 40, 130])
+@pytest.mark.parametrize("rows", [1, 12, 32, 40, 130])
 def test_cross_attention_merges_groups_in_order(ctx, rows):
-    """The forms of the cross-attention (four workgroups per (row, head) up to 64 of those, one per CU up to 256, the
+    """The forms of the cross-attention (four workgroups per (row, head) up to 12 rows, one per CU up to 256, the
     general kernel above) give the 32 groups' states merged one after the other."""
     rng = np.random.default_rng(rows)
     e = engine(ctx, 128, rows, {DEC + "encoder_attn.out_proj.weight": np.eye(128, dtype=np.float16)})
