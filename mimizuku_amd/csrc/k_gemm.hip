@@ -93,9 +93,6 @@ __device__ __forceinline__ void gemm_epilogue(const MzGemm& p, const f32x16 (&ac
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lr = lane & 31, lh = lane >> 5;
     if (EPI == EPI_HEADS) {
         if (p.kind == 3) lds_barrier();  // every wave is done reading operands: LDS is free for the v transposes
-        // a partial last column tile: this wave has no head block (64 | N, so a wave's columns all exist or none does), and
-        // what lies a clip's blocks further is the next clip's
-        if (n0 >= p.N) return;
         const int blk = n0 >> 6;           // a wave's columns lie in one 64-wide head block (WN <= 64)
         const bool vt = p.kind == 3 && blk / p.nh == 2;
         if (vt) {
@@ -137,10 +134,12 @@ __device__ __forceinline__ void gemm_epilogue(const MzGemm& p, const f32x16 (&ac
         // wave's 128 rows span at most two of them (128 < 1500): the store descriptor starts at the first one's
         // tiles and ends after the second one, or after the last clip of the call, so the range check drops the
         // rows of a partial last tile. Rows of the second clip add one clip's worth of tiles; every offset stays
-        // below 2^31 bytes (two clips of at most 4096 tiles).
+        // below 2^31 bytes (two clips of at most 4096 tiles). A wave past the last head (a partial last column tile; 64
+        // divides N, so a wave's columns all exist or none does) has an empty descriptor: what lies a clip's heads further
+        // is the next clip's. (A branch round the stores made the QKV product 1 to 1.5 us slower.)
         const int g0 = m0 / MZ_TENC;
         const long clip = (long)p.blocks_per_clip * (MZ_TPAD * MZ_HD);
-        const int ncl = min(p.M / MZ_TENC - g0, 2);
+        const int ncl = n0 < p.N ? min(p.M / MZ_TENC - g0, 2) : 0;
         const __amdgpu_buffer_rsrc_t rH =
             rsrc(p.heads + (p.slot0 + g0) * clip, ncl > 0 ? (unsigned)(ncl * clip * 2) : 0u);
         const int blk = n0 >> 6, c0 = (n0 & 63) + lr;
