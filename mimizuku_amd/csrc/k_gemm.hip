@@ -3,7 +3,7 @@
 // implicit GEMM (no im2col buffer), and the cross-attention K/V of every decoder layer. Replaces the reference's
 // cuBLAS calls with a bias prefill (src/gpu.rs:208-236, 254-286; kernels/whisper.cu:92-104, 106-139).
 //
-// Two kernels, chosen by how many tiles a product has (pick): gemm_ring_kernel for few, described there, and for the rest
+// Two kernels, chosen by how many tiles a product has (pick_plain, pick_conv): gemm_ring_kernel for few, described there, for the rest
 // gemm_kernel: block tile BM x BN x 64 with 8 waves in a 2 x 4 grid (two waves per SIMD, so one wave's LDS reads overlap the
 // other's products); each wave owns a (BM/2) x (BN/4) tile of 32x32x16 MFMA products. Both operands are
 // K-contiguous and go from global memory straight into LDS (buffer_load ... lds, 16 bytes per lane, no register
@@ -17,6 +17,8 @@
 // The activation tile is the MFMA A operand and the W tile the B operand, so lane l of a 32x32 product holds output
 // column l % 32 of eight rows: every store instruction writes two 32-column row segments. The transposed tiles of
 // the encoder's v are staged through LDS to be written as runs of token positions.
+#include <algorithm>
+
 #include "mz_common.h"
 #include "mz_kernels.h"
 
@@ -589,20 +591,48 @@ hipError_t launch_ring(hipStream_t s, const MzGemm& g) {
     return hipGetLastError();
 }
 
-template <int ALOAD, int EPI>
-hipError_t pick(hipStream_t s, const MzGemm& g) {
-    // The largest tile that still gives half of the CUs one each: below that, more CUs at work gain more than the
-    // larger tile's fewer operand bytes per product. Over M = 1500 c (c = 1 .. 8) and the N, K of widths 384 to 1280 the
-    // choice is within 4% of the fastest of the five shapes (11% at one: M 4500, N 5120, K 1280). M = 1500, K = 1280 / 5120,
-    // N = 1280: 128 x 64 ring 9.4 / 28.4 us, 64 x 64 ring 10.2 / 34.9, 128 x 128 ring 11.0 / 34.0, a 128 x 128 tile with
-    // two buffers (the rule before) 13.5 / 52.9. N = 384, K = 1536: 64 x 64 ring 6.5 us, before 11.9.
-    auto tiles = [&](int bm, int bn) { return (long)((g.M + bm - 1) / bm) * ((g.N + bn - 1) / bn); };
-    const long half = mz_cu_count() / 2 + 2;
-    if (tiles(256, 256) >= half) return launch<256, 256, ALOAD, EPI>(s, g);
-    if (tiles(256, 128) >= half) return launch<256, 128, ALOAD, EPI>(s, g);
-    if (tiles(128, 128) >= half) return launch_ring<128, 128, 2, 4, ALOAD, EPI>(s, g);
-    if (tiles(128, 64) >= half) return launch_ring<128, 64, 2, 2, ALOAD, EPI>(s, g);
-    return launch_ring<64, 64, 2, 2, ALOAD, EPI>(s, g);
+// workgroups over the CUs, in whole rounds
+long tile_count(const MzGemm& g, int bm, int bn) { return (long)((g.M + bm - 1) / bm) * ((g.N + bn - 1) / bn); }
+long rounds(const MzGemm& g, int bm, int bn) { return (tile_count(g, bm, bn) + mz_cu_count() - 1) / mz_cu_count(); }
+
+// Plain products: the largest tile that still gives more than half of the CUs one each: below that, more CUs at work gain
+// more than the larger tile's fewer operand bytes per product. Kernel times in the encoder's own sequence (operands as the
+// kernels before leave them), this rule / the one before it (256-row tiles from 200 on, two buffers): one clip, width
+// 1280, qkv 35 / 38 us, out-projection 12 / 18, fc1 36 / 54, fc2 30 / 55; 4 clips, width 512, 24 / 25, 9.5 / 10, 26 / 28,
+// 20 / 25; 5 to 8 clips, width 1280, within 1.5% but for fc2 at 5 (115 / 170). The largest is not always the fastest: launched
+// back to back, the choice is 1.5% from the fastest of six shapes on average over M = 1500 c (c = 1 .. 8) and the N, K of
+// widths 128 to 1280 (4% or more at 88 of 480, the worst 19%: M 10500, N 1152, K 384, 256 x 256 20.4 us, 256 x 128 17.4);
+// fitted to those times it was 0.7%, but slower in the encoder (fc2 at 4 clips, width 1280, 92 -> 103).
+// Where a last column tile is partial, 256 x 128 may take no more rounds than 256 x 256 and has less to do in each: M 12000,
+// N 640, K 640 16.6 -> 12.9, M 6000, N 2688, K 896 46.6 -> 33.1.
+template <int EPI>
+hipError_t pick_plain(hipStream_t s, const MzGemm& g) {
+    const long half = mz_cu_count() / 2;
+    if (tile_count(g, 256, 256) > half && rounds(g, 256, 256) < rounds(g, 256, 128)) return launch<256, 256, ALOAD_PLAIN, EPI>(s, g);
+    if (tile_count(g, 256, 128) > half) return launch<256, 128, ALOAD_PLAIN, EPI>(s, g);
+    if (tile_count(g, 128, 128) > half) return launch_ring<128, 128, 2, 4, ALOAD_PLAIN, EPI>(s, g);
+    if (tile_count(g, 128, 64) > half) return launch_ring<128, 64, 2, 2, ALOAD_PLAIN, EPI>(s, g);
+    return launch_ring<64, 64, 2, 2, ALOAD_PLAIN, EPI>(s, g);
+}
+
+// The convolutions, whose A rows cost more to address and whose grid is not persistent (two 128 x 128 workgroups of two
+// buffers share a CU), go by an estimate of the time: rounds x (K tiles x k + per) + base in us, the constants fitted to the
+// measured times of both convolutions for 1 to 8 clips of widths 128 to 1280. 0.1% from the fastest of six shapes on
+// average; the rule above was 12% (up to 64%: M 21000, N 384, K 256, 256 x 256 17.0 us, 128 x 128 10.4). In the encoder,
+// conv1 / conv2 of 8 clips at width 1024 39.0 / 100.1 -> 31.0 / 97.9, of 3 at 1280 20.4 / 77.6 -> 20.3 / 66.0.
+template <int EPI>
+hipError_t pick_conv(hipStream_t s, const MzGemm& g) {
+    const int kt = g.K / 64;
+    const float est[5] = {rounds(g, 256, 256) * (kt * 1.27f + 11.50f) + 0.02f, rounds(g, 128, 128) * (kt * 0.55f + 0.99f) + 3.77f,
+                          rounds(g, 128, 128) * (kt * 0.53f + 3.81f) + 1.26f, rounds(g, 128, 64) * (kt * 0.43f + 3.20f) + 2.20f,
+                          rounds(g, 64, 64) * (kt * 0.23f + 0.66f) + 2.77f};
+    switch (std::min_element(est, est + 5) - est) {
+        case 0: return launch<256, 256, ALOAD_CONV, EPI>(s, g);
+        case 1: return launch<128, 128, ALOAD_CONV, EPI>(s, g);
+        case 2: return launch_ring<128, 128, 2, 4, ALOAD_CONV, EPI>(s, g);
+        case 3: return launch_ring<128, 64, 2, 2, ALOAD_CONV, EPI>(s, g);
+    }
+    return launch_ring<64, 64, 2, 2, ALOAD_CONV, EPI>(s, g);
 }
 
 }  // namespace
@@ -632,15 +662,15 @@ hipError_t mz_gemm_launch(hipStream_t s, int aload, int epi, const MzGemm& g) {
         return hipErrorInvalidValue;
     if (aload == ALOAD_CONV) {
         if (g.conv_cin % 8 != 0 || g.conv_tout <= 0) return hipErrorInvalidValue;
-        if (epi == EPI_GELU_F16) return pick<ALOAD_CONV, EPI_GELU_F16>(s, g);
-        if (epi == EPI_GELU_POS) return pick<ALOAD_CONV, EPI_GELU_POS>(s, g);
+        if (epi == EPI_GELU_F16) return pick_conv<EPI_GELU_F16>(s, g);
+        if (epi == EPI_GELU_POS) return pick_conv<EPI_GELU_POS>(s, g);
         return hipErrorInvalidValue;
     }
     switch (epi) {
-        case EPI_F16: return pick<ALOAD_PLAIN, EPI_F16>(s, g);
-        case EPI_GELU_F16: return pick<ALOAD_PLAIN, EPI_GELU_F16>(s, g);
-        case EPI_RESID_F32: return pick<ALOAD_PLAIN, EPI_RESID_F32>(s, g);
-        case EPI_HEADS: return pick<ALOAD_PLAIN, EPI_HEADS>(s, g);
+        case EPI_F16: return pick_plain<EPI_F16>(s, g);
+        case EPI_GELU_F16: return pick_plain<EPI_GELU_F16>(s, g);
+        case EPI_RESID_F32: return pick_plain<EPI_RESID_F32>(s, g);
+        case EPI_HEADS: return pick_plain<EPI_HEADS>(s, g);
     }
     return hipErrorInvalidValue;
 }

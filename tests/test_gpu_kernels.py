@@ -304,7 +304,7 @@ def test_gemm_head_scatter(ctx, kind):
         ctx.free(p)
 
 
-@pytest.mark.parametrize("kind,nh,clips,blocks", [(3, 6, 5, 18), (2, 1, 6, 7), (3, 1, 6, 3)])
+@pytest.mark.parametrize("kind,nh,clips,blocks", [(3, 6, 5, 18), (2, 1, 6, 7), (3, 1, 7, 3)])
 def test_gemm_head_scatter_partial_columns(ctx, kind, nh, clips, blocks):
     """Head counts that leave the last column tile partial (1152 columns in 256 x 256 tiles, 448 in 256 x 128, 192 in
     128 x 128): the columns past the last head write nothing. Each clip has two more tiles than the product has heads, which
@@ -331,6 +331,30 @@ def test_gemm_head_scatter_partial_columns(ctx, kind, nh, clips, blocks):
         ctx.free(p)
 
 
+@pytest.mark.parametrize("kind,nh,clips,blocks", [(3, 16, 7, 48), (2, 24, 3, 96)])
+def test_gemm_head_scatter_several_tiles_per_workgroup(ctx, kind, nh, clips, blocks):
+    """10500 x 3072 and 4500 x 6144: 504 and 432 tiles of 256 x 256 in equal shares of 63 and 54 per XCD, so that each
+    workgroup scatters a tile while the next one's operands come in. Bit for bit what each clip alone (one tile per
+    workgroup) gives; test_gemm_head_scatter compares that with float64."""
+    rng = np.random.default_rng(blocks)
+    n, k, m = blocks * 64, 192, clips * 1500
+    x, w, b = f16(rng, (m, k)), f16(rng, (n, k), 0.1), f16(rng, (n,), 0.1)
+    dx, dw, db = (ctx.upload_new(a) for a in (x, w, b))
+    out = []
+    for step in (clips, 1):
+        dh = ctx.upload_new(np.full((clips, blocks, TPAD * 64), 7, np.float16))
+        for c in range(0, clips, step):
+            L.check(L.lib().mz_linear(ctx.h, linear_args(epilogue=L.EPI_HEADS, a=dx + c * 1500 * k * 2, lda=k, w=dw, bias=db,
+                                                         m=step * 1500, n=n, k=k, heads=dh, blocks_per_clip=blocks, nh=nh,
+                                                         kind=kind, slot0=c)))
+        out.append(ctx.download(dh, (clips, blocks, TPAD * 64), np.float16))
+        ctx.free(dh)
+    np.testing.assert_array_equal(out[0], out[1])
+    assert (out[0][0, 0].reshape(TPAD, 64)[:1500] != 7).any()
+    for p in (dx, dw, db):
+        ctx.free(p)
+
+
 def test_gemm_large_qkv_shape(ctx):
     """The encoder group's fused QKV product, M = 12000, N = 3840, K = 1280, 256 rows checked."""
     rng = np.random.default_rng(5)
@@ -347,13 +371,20 @@ def test_gemm_large_qkv_shape(ctx):
         ctx.free(p)
 
 
-@pytest.mark.parametrize("m,n,k", [(9000, 2304, 320), (12000, 768, 448), (6000, 1000, 192)])
+@pytest.mark.parametrize("m,n,k", [(9000, 2304, 320), (12000, 768, 448), (6000, 1000, 192), (10500, 3072, 320),
+                                   (9000, 5116, 192), (6000, 2688, 192), (24988, 640, 128)])
 def test_gemm_persistent_shapes(ctx, m, n, k):
-    """Products with more tiles than CUs, so each workgroup of the persistent grid walks several tiles (requesting the
-    next tile's first K tile before each epilogue): 256 x 256 tiles with a partial last block row and an odd count
-    of 64-wide K tiles (9000 x 2304 x 320), 256 x 128 tiles (12000 x 768 x 448), 128 x 128 tiles with partial block
-    rows and columns (6000 x 1000 x 192); fp16 output against float64 on sampled rows, and on the first shape also
-    the GELU and fp32 residual epilogues."""
+    """Products of 256 x 256 and 256 x 128 tiles, whose workgroups walk several tiles where there are more than CUs
+    (requesting the next tile's first K tile before each epilogue):
+      9000 x 2304   256 x 256, 324 tiles, whole bands per XCD; partial last block row, odd count of 64-wide K tiles
+      10500 x 3072  256 x 256, 504 tiles, equal shares of 63 per XCD
+      9000 x 5116   256 x 256, 720 tiles, equal shares of 90, a last band of one block row and a partial last column
+      6000 x 2688   256 x 128, 504 tiles, whole bands (256 x 256 would take as many rounds)
+      24988 x 640   256 x 128, 490 tiles, equal shares of 62
+      12000 x 768   256 x 256, 141 tiles: one per workgroup
+      6000 x 1000   256 x 128, 192 tiles: one per workgroup, partial last row and column
+    fp16 output against float64 on sampled rows and bit for bit against the last 1500 rows alone (other tiles); the
+    GELU and fp32 residual epilogues too where a workgroup has several tiles."""
     rng = np.random.default_rng(m + n + k)
     x, w, b = f16(rng, (m, k)), f16(rng, (n, k), 0.05), f16(rng, (n,), 0.1)
     dx, dw, db = (ctx.upload_new(a) for a in (x, w, b))
@@ -361,8 +392,11 @@ def test_gemm_persistent_shapes(ctx, m, n, k):
     acc = x[rows].astype(np.float64) @ w.astype(np.float64).T + b
     dy = ctx.alloc(m * n * 2)
     L.check(L.lib().mz_gemm(ctx.h, dx, k, dw, dy, n, m, n, k, db))
-    assert_f16(ctx.download(dy, (m, n), np.float16)[rows], acc)
-    if m == 9000:
+    y = ctx.download(dy, (m, n), np.float16)
+    assert_f16(y[rows], acc)
+    L.check(L.lib().mz_gemm(ctx.h, dx + (m - 1500) * k * 2, k, dw, dy, n, 1500, n, k, db))
+    np.testing.assert_array_equal(ctx.download(dy, (1500, n), np.float16), y[-1500:])
+    if m * n >= 6000 * 2304:
         L.check(L.lib().mz_linear(ctx.h, linear_args(epilogue=L.EPI_GELU_F16, a=dx, lda=k, w=dw, bias=db, m=m, n=n,
                                                      k=k, out=dy, ldo=n)))
         assert_f16(ctx.download(dy, (m, n), np.float16)[rows], R.gelu(acc.astype(np.float32)))
@@ -382,7 +416,7 @@ def test_gemm_persistent_shapes(ctx, m, n, k):
 def test_gemm_small_grids(ctx, m, n, k):
     """Products of few tiles: 64 x 64, 128 x 64 and 128 x 128 tiles with partial last rows and columns, and K tile counts
     on both sides of the ring's four slots (1, 2, 3, 4, 5, 7 and whole rounds). The same bits as the same rows within a
-    product large enough for 256 x 256 tiles, and the float64 product."""
+    product large enough for tiles of 256 rows, and the float64 product."""
     rng = np.random.default_rng(m + 3 * n + k)
     big = 256 * (132 // ((n + 255) // 256) + 1)
     x, w, b = f16(rng, (max(m, big), k)), f16(rng, (n, k), 0.05), f16(rng, (n,), 0.1)
@@ -398,10 +432,12 @@ def test_gemm_small_grids(ctx, m, n, k):
         ctx.free(p)
 
 
-@pytest.mark.parametrize("clips,cin,n,stride", [(1, 80, 384, 1), (1, 384, 384, 2), (3, 128, 512, 1), (1, 512, 1280, 2)])
+@pytest.mark.parametrize("clips,cin,n,stride", [(1, 80, 384, 1), (1, 384, 384, 2), (3, 128, 512, 1), (1, 512, 1280, 2),
+                                                (1, 1280, 1280, 2), (2, 1024, 1024, 2), (8, 896, 896, 2)])
 def test_conv_small_grids(ctx, clips, cin, n, stride):
-    """The convolution's padding (both ends of each clip, K past the taps) in the tiles of few clips: the same bits as
-    the plain product of the unrolled rows."""
+    """The convolution's padding (both ends of each clip, K past the taps) in each of its tile shapes (64 x 64 for the
+    first two and the fourth, two buffers of 128 x 128 for the third, then 128 x 64, the ring of 128 x 128, and 256 x 256):
+    the same bits as the plain product of the unrolled rows."""
     rng = np.random.default_rng(clips + cin + n)
     src, b = f16(rng, (clips, 3000, cin)), f16(rng, (n,), 0.1)
     k, t = (3 * cin + 63) // 64 * 64, 3000 // stride
