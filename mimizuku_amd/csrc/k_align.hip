@@ -283,8 +283,12 @@ __global__ void __launch_bounds__(256) ts_cost_kernel(const MzTs p) {
         }
     };
     auto zscore = [&](float x, float m, float s) { return s > 0.f ? (p.half ? rh(rh(x - m) / s) : (x - m) / s) : 0.f; };
-    // the median phase: columns 8 jl .. 8 jl + 7 of row il
-    const int il = tid >> 3, jl = (tid & 7) * 8;
+    // the median phase, eight cells per thread: at width 7 columns jl .. jl + 7 of row il, otherwise column jl of rows
+    // il + 4 q (a wave's cells of one q lie in one row, and the rows past R are left out: 5 rows, width 15, 287 us for the
+    // whole call; with eight columns per thread, so that one wave had all the rows there are, 855)
+    const int il = W ? tid >> 3 : tid >> 6, jl = W ? (tid & 7) * 8 : tid & 63;
+    auto row = [&](int q) { return W ? il : il + 4 * q; };
+    auto col = [&](int q) { return W ? jl + q : jl; };
     float acc[8];
 #pragma unroll
     for (int q = 0; q < 8; q++) acc[q] = 0.f;
@@ -311,7 +315,7 @@ __global__ void __launch_bounds__(256) ts_cost_kernel(const MzTs p) {
         const float* zr = &zt[il][jl];
         if (C <= pad) {
 #pragma unroll
-            for (int q = 0; q < 8; q++) acc[q] += zr[q + pad];  // fewer columns than the half width: no filter
+            for (int q = 0; q < 8; q++) acc[q] += zt[row(q)][col(q) + pad];  // fewer columns than the half width: no filter
         } else if (W == 7 && !slow) {
             float z[14], lo[12], md[12], up[12];
 #pragma unroll
@@ -338,11 +342,12 @@ __global__ void __launch_bounds__(256) ts_cost_kernel(const MzTs p) {
                 acc[q] += median7(win);
             }
         } else {
-#pragma unroll 1
+#pragma unroll
             for (int q = 0; q < 8; q++) {
+                if (i0 + row(q) >= R) continue;
                 float win[MZ_TS_MAX_WIDTH];
                 for (int e = 0; e < width; e++) {
-                    const float v = zr[q + e];
+                    const float v = zt[row(q)][col(q) + e];
                     int r = e - 1;
                     while (r >= 0 && win[r] > v) {
                         win[r + 1] = win[r];
@@ -350,9 +355,7 @@ __global__ void __launch_bounds__(256) ts_cost_kernel(const MzTs p) {
                     }
                     win[r + 1] = v;
                 }
-                const float m = win[pad];
-#pragma unroll
-                for (int x = 0; x < 8; x++) acc[x] += x == q ? m : 0.f;
+                acc[q] += win[pad];
             }
         }
         lds_barrier();  // zt is rewritten for the next head
@@ -362,7 +365,7 @@ __global__ void __launch_bounds__(256) ts_cost_kernel(const MzTs p) {
     for (int q = 0; q < 8; q++) {
         float v = acc[q] / (float)p.heads;
         if (p.half) v = rh(v);
-        val[il][jl + q] = v;
+        val[row(q)][col(q)] = v;
     }
     __syncthreads();
     // DTW cell (i + 1, j + 1) lies on anti-diagonal i + j + 2: tile diagonal dl = il + jl holds rows il of one run
