@@ -20,8 +20,9 @@
 #include <math.h>
 
 #include <algorithm>
+#include <memory>
 #include <mutex>
-#include <vector>
+#include <new>
 
 #include "../../include/mimizuku.h"
 #include "mz_common.h"
@@ -715,7 +716,10 @@ extern "C" int mz_jump_times_device_noalloc(mz_ctx* c, uint64_t w, int64_t clip_
     };
     // the clips go through the array in chunks of at most MZ_TS_NOALLOC_CHUNK that fit in it, one after the other
     int2 rc[MZ_TS_NOALLOC_CHUNK];
-    std::vector<float> times;
+    // a chunk's times on the host: requested before anything is in flight, and without an exception past the C entry
+    const int longest = *std::max_element(rows, rows + n);
+    const std::unique_ptr<float[]> times(new (std::nothrow) float[(size_t)std::min(n, (int)MZ_TS_NOALLOC_CHUNK) * std::max(longest, 1)]);
+    if (!times) return mz_fail(MZ_ERR_STATE, "mz_jump_times_device_noalloc: out of host memory");
     for (int c0 = 0; c0 < n;) {
         int k = 0, rmax = 0;
         while (c0 + k < n && k < MZ_TS_NOALLOC_CHUNK && need(k + 1, std::max(rmax, (int)rows[c0 + k])) <= MZ_TS_SCRATCH_BYTES) {
@@ -756,14 +760,13 @@ extern "C" int mz_jump_times_device_noalloc(mz_ctx* c, uint64_t w, int64_t clip_
                        "upload");
         if (!r) r = mz_hip(mz_ts_launch(c->stream, p, k), "timestamp kernels");
         // the chunk's times in one copy (one per clip took longer than the kernels of a large chunk)
-        times.resize((size_t)k * rmax);
         if (!r && rmax > 0)
-            r = mz_hip(hipMemcpyAsync(times.data(), p.out, times.size() * 4, hipMemcpyDeviceToHost, c->stream), "download");
+            r = mz_hip(hipMemcpyAsync(times.get(), p.out, (size_t)k * rmax * 4, hipMemcpyDeviceToHost, c->stream), "download");
         // the next chunk reuses the array (and rc): wait for this one
         const int rs = mz_hip(hipStreamSynchronize(c->stream), "hipStreamSynchronize");
         if (r || rs) return r ? r : rs;
         for (int i = 0; i < k; i++)
-            std::copy(times.data() + (size_t)i * rmax, times.data() + (size_t)i * rmax + rows[c0 + i],
+            std::copy(times.get() + (size_t)i * rmax, times.get() + (size_t)i * rmax + rows[c0 + i],
                       out + (size_t)(c0 + i) * out_stride);
         c0 += k;
     }
