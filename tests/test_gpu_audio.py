@@ -176,3 +176,59 @@ def test_scratch_kept_between_calls():
             for x, y in zip(g, ref[k + 1][0]):
                 np.testing.assert_array_equal(x, y)
     own.close()
+
+
+def test_scratch_beyond_what_is_kept():
+    """Calls whose device scratch alone (120 clips: 220 MiB), or whose device and pinned scratch (60000 short clips: 200 MiB
+    and 5 MiB), are beyond what a context keeps, with small calls in between: the values of the entry point whose scratch
+    is static."""
+    from mimizuku_amd import transcribe
+    rng = np.random.default_rng(13)
+    ctx = model.Context(0)
+    for n, rows, full in ((3, 40, 1500), (120, 220, 1500), (3, 40, 1500), (60000, 20, 8), (3, 40, 1500)):
+        dw = ctx.upload_new(rng.random((n + rows, full), dtype=np.float32))  # clip c: rows c .. c + rows - 1
+        args = (ctx, dw, full, [rows - i % 7 for i in range(n)], [full] * n, 1, full)
+        got, ref = transcribe.jump_times_device(*args), transcribe.jump_times_device_noalloc(*args)
+        np.testing.assert_array_equal(np.concatenate(got), np.concatenate(ref))
+        ctx.free(dw)
+    ctx.close()
+
+
+def test_scratch_of_a_call_within_another():
+    """A call that runs while another thread's (8000 clips, about 20 ms) holds the context's scratch: it began
+    after that one and before its end, and both give the values they give alone."""
+    import threading
+    import time
+
+    from mimizuku_amd import transcribe
+    rng = np.random.default_rng(14)
+    ctx = model.Context(0)
+    big, small, full = 8000, 4, 1500
+    dw = ctx.upload_new(rng.random((big + 220, full), dtype=np.float32))
+    long_args = (ctx, dw, full, [220] * big, [full] * big, 1, full)
+    short_args = (ctx, dw, full, [50 + i for i in range(small)], [full] * small, 1, full)
+    want = [np.concatenate(transcribe.jump_times_device_noalloc(*a)) for a in (long_args, short_args)]
+    within = 0
+    for _ in range(5):
+        span, got = {}, {}
+        gate = threading.Barrier(2)
+
+        def call(name, args, wait):
+            gate.wait()
+            time.sleep(wait)
+            t0 = time.perf_counter()
+            got[name] = np.concatenate(transcribe.jump_times_device(*args))
+            span[name] = t0, time.perf_counter()
+
+        threads = [threading.Thread(target=call, args=a) for a in (("long", long_args, 0.0), ("short", short_args, 0.008))]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+        np.testing.assert_array_equal(got["long"], want[0])
+        np.testing.assert_array_equal(got["short"], want[1])
+        within += span["long"][0] + 0.004 < span["short"][0] < span["long"][1] - 0.004
+        print("long %.1f ms, the short one began %.1f ms into it" % (1e3 * (span["long"][1] - span["long"][0]),
+                                                                     1e3 * (span["short"][0] - span["long"][0])))
+    assert within > 0
+    ctx.close()
