@@ -229,24 +229,11 @@ size_t xkv_elems(const mz_dims& d, int bmax) { return (size_t)bmax * d.dec_layer
 
 constexpr size_t XPART = (size_t)MZ_CROSS_SPLIT_PAIRS * MZ_CROSS_STATE;  // floats of the split cross-attention's states
 
-int ksplit_for(int N, int K) {
-    // Split K over workgroups until the grid covers most of the 256 CUs, with at most 16 groups of 64 per workgroup
-    // (a slice within MZ_DEC_KSLICE, both operands resident in LDS) and at most MZ_MAX_PARTS partials.
-    const int tiles = (N + 31) / 32, groups = K / 64;
-    int best = 1;
-    for (int ks = 1; ks <= std::min(groups, MZ_MAX_PARTS); ks++) {
-        if (groups % ks) continue;
-        best = ks;
-        if (groups / ks <= 16 && (long)tiles * ks >= 192) break;
-    }
-    return best;
-}
-
 // elements of the decoder's split-K partials buffer: the largest ks * rows * n over the decoder products
 size_t part_elems(int D, int F, int B) {
     size_t pe = 0;
     for (auto nk : {std::pair<int, int>{D, D}, {D, F}, {3 * D, D}})
-        pe = std::max(pe, (size_t)ksplit_for(nk.first, nk.second) * B * nk.first);
+        pe = std::max(pe, (size_t)mz_dec_ksplit(nk.first, nk.second) * B * nk.first);
     return pe;
 }
 
@@ -812,7 +799,7 @@ static int step_impl(mz_engine* e, int b, int lang, int prompt_len) {
         a.na = e->na;
         return a;
     };
-    const int ks_dd = ksplit_for(D, D), ks_df = ksplit_for(D, F), ks_qkv = ksplit_for(3 * D, D);
+    const int ks_dd = mz_dec_ksplit(D, D), ks_df = mz_dec_ksplit(D, F), ks_qkv = mz_dec_ksplit(3 * D, D);
     const f16* xkv = e->xkvbuf;
     // the split needs K slices of whole heads within the out-projection's x block
     const bool xsplit = mz_cross_split(b, nh) && D / ks_dd <= 256;

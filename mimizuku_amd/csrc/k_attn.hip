@@ -3,20 +3,20 @@
 // fp16 for the P.V product, O / l rounded to fp16 (the SDPA arithmetic the reference follows, whisper.cu:3-4).
 //
 // Work: one block per (256 queries, head, clip) = 4 waves x 2 sets of 32 queries, or per 128 queries with one set per
-// wave where that spreads few (clip, head) pairs better over the CUs (mz_enc_attention_launch). K and V^T tiles of 64 keys are
-// staged in LDS (double buffered, register prefetch) and shared by the 4 waves. Scores are computed transposed,
-// S^T = K Q^T (32x32x16 MFMA), so each lane owns one query column: the running max and the rescale of O are per
-// lane, and the only cross-lane step is one swap with lane l ^ 32. K rows are stored in LDS with bits 2 and 3 of the
-// key index swapped, which makes each lane's 16 scores two runs of 8 consecutive keys: the probabilities, rounded to
-// fp16, are directly the B operand of O^T = V^T P^T, and V^T (written transposed by the QKV GEMM) is read with
+// wave where that spreads few (clip, head) pairs better over the CUs (mz_enc_attention_launch). K and V^T tiles of 64
+// keys are staged in LDS (double buffered, register prefetch) and shared by the 4 waves. Scores are computed
+// transposed, S^T = K Q^T (32x32x16 MFMA), so each lane owns one query column: the running max and the rescale of O are
+// per lane, and the only cross-lane step is one swap with lane l ^ 32. K rows are stored in LDS with bits 2 and 3 of
+// the key index swapped, which makes each lane's 16 scores two runs of 8 consecutive keys: the probabilities, rounded
+// to fp16, are directly the B operand of O^T = V^T P^T, and V^T (written transposed by the QKV GEMM) is read with
 // 16-byte LDS loads.
 //
 // Vector work hides only in part under the matrix cores (a wave's own vector instructions overlap about two thirds
 // of their time with its independent products, the other wave of the SIMD covers more), so every vector instruction
-// per score counts: the running max is set by the first block and later blocks compute no max at all; a block is recomputed against its own max (and O
-// rescaled) only when the sum of its probabilities reaches 2^12, i.e. some p = exp2(s - m) could leave the range
-// where fp16 holds it exactly enough; the probabilities are rounded two per packed conversion and summed two per
-// dot2 instruction, and the key mask of the padded last tile is applied in that tile only.
+// per score counts: the running max is set by the first block and later blocks compute no max at all; a block is
+// recomputed against its own max (and O rescaled) only when the sum of its probabilities reaches 2^12, i.e. some
+// p = exp2(s - m) could leave the range where fp16 holds it exactly enough; the probabilities are rounded two per packed
+// conversion and summed two per dot2 instruction, and the key mask of the padded last tile is applied in that tile only.
 #include <type_traits>
 
 #include "mz_common.h"
@@ -54,8 +54,9 @@ __device__ __forceinline__ float probs(const f32x16& sc, unsigned (&pw)[2][4]) {
     return lb;
 }
 
-// NS query sets of 32 per wave, NW waves: 32 NS NW queries per block
-template <int NS, int NW>
+// NS query sets of 32 per wave: 128 NS queries per block
+constexpr int NW = 4;  // waves per block
+template <int NS>
 __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
 enc_attn_kernel(const f16* __restrict__ qkvh, f16* __restrict__ out, int nh, int G) {
     __shared__ __attribute__((aligned(16))) f16 sK[2][64 * KP];
@@ -215,11 +216,11 @@ enc_attn_kernel(const f16* __restrict__ qkvh, f16* __restrict__ out, int nh, int
     }
 }
 
-template <int NS, int NW>
+template <int NS>
 hipError_t launch(hipStream_t s, const f16* qkvh, f16* out, int G, int nh) {
     // 1-D grid: 8 XCDs x an eighth of the query blocks, rounded up
     constexpr int QB = 32 * NS * NW, npq = (MZ_TENC + QB - 1) / QB;
-    hipLaunchKernelGGL((enc_attn_kernel<NS, NW>), dim3(8 * ((G * nh * npq + 7) / 8)), dim3(64 * NW), 0, s, qkvh, out, nh, G);
+    hipLaunchKernelGGL((enc_attn_kernel<NS>), dim3(8 * ((G * nh * npq + 7) / 8)), dim3(64 * NW), 0, s, qkvh, out, nh, G);
     return hipGetLastError();
 }
 
@@ -233,6 +234,6 @@ hipError_t mz_enc_attention_launch(hipStream_t s, const f16* qkvh, f16* out, int
     // the large ones would round up (1 x 20 heads 31.6 -> 20.4 us, 3 x 20 56.4 -> 50.4), and for two per CU (35.6 ->
     // 33.4); beyond 7 the large ones win either way (16 x 20 220 vs 231). Both give the same bits.
     const int k = (G * nh * ((MZ_TENC + 127) / 128) + mz_cu_count() - 1) / mz_cu_count();
-    if (k == 2 || (k <= 7 && k % 2 == 1)) return launch<1, 4>(s, qkvh, out, G, nh);
-    return launch<2, 4>(s, qkvh, out, G, nh);
+    if (k == 2 || (k <= 7 && k % 2 == 1)) return launch<1>(s, qkvh, out, G, nh);
+    return launch<2>(s, qkvh, out, G, nh);
 }

@@ -23,6 +23,8 @@
 //                 Small batches: the cross-attention over four workgroups per (row, head), merged by the out-projection
 //   dec_add_ln    residual add of the split-K partials + bias, fused with the next LayerNorm (whisper.cu:71-82)
 //   dec_argmax    greedy choice from the per-workgroup argmax partials; advances the position (whisper.cu:451-495)
+#include <type_traits>
+
 #include "mz_common.h"
 #include "mz_kernels.h"
 
@@ -1017,9 +1019,9 @@ __global__ void __launch_bounds__(256, 1) dec_cross_wide_kernel(const MzDecCross
 // dec_attn_kernel (keys 8 s .. 8 s + 7 of every 32). What bounds a (row, head) on one CU is the CU's own rate for what
 // misses its caches (25 to 50 GB/s, whatever is in flight), so its 384 KB of keys and values go over four CUs. Each
 // projects the query for itself (its wq rows come from the L2 that the four share: they run on one XCD). The groups'
-// states are merged by the out-projection that reads them, as another launch for that would cost what the split gains. The four waves share the arithmetic that one would take 3 us
-// for: the scores by batches of keys, then the softmax by dims. One row: width 384 14.7 -> 8.5 us a layer, 1280 16.2 ->
-// 9.9 (9.1 and 11.0 with the keys through LDS as well), the out-projection 3.7 -> 4.0.
+// states are merged by the out-projection that reads them, as another launch for that would cost what the split gains. The
+// four waves share the arithmetic that one would take 3 us for: the scores by batches of keys, then the softmax by dims.
+// One row: width 384 14.7 -> 8.5 us a layer, 1280 16.2 -> 9.9 (9.1 and 11.0 with the keys through LDS as well).
 __global__ void __launch_bounds__(256, 2) dec_cross_split_kernel(const MzDecCross a) {
 #if defined(__HIP_DEVICE_COMPILE__)
     constexpr int L = MZ_TENC, NI = (L + 31) / 32, AU = 8, NJ = MZ_DEC_KSLICE / 64;
@@ -1300,24 +1302,25 @@ hipError_t mz_dec_add_ln_launch(hipStream_t s, const float* xin, float* x, const
                                 long part_stride, const f16* bias, const f16* w, const f16* b, f16* y, int rows,
                                 int dim, float eps) {
     if (dim % 4 != 0 || dim > 2048 || rows <= 0 || nparts < 0 || nparts > MZ_MAX_PARTS) return hipErrorInvalidValue;
-    // One wave per row at the models' widths with the split-K counts that the engine's products of those widths take
-    // (ksplit_for): in a replayed step a launch costs about 1 us less than the general kernel (one workgroup of up to
+    // One wave per row at the models' widths with the partials that the out-projections (width x width) and fc2 (width x 4
+    // width) leave: in a replayed step a launch costs about 1 us less than the general kernel (one workgroup of up to
     // five waves per row, their sums through LDS): 12 launches a step, width 384 at one row 196 -> 188 us, 1024 at six
     // 244 -> 234, 1280 at 32 401.8 -> 390.4.
     auto wave = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, dim3(rows), dim3(64), 0, s, xin, x, parts, part_stride, bias, w, b, y, eps);
-        return hipGetLastError();
+        return true;
     };
-    switch (dim * 100 + nparts) {
-        case 38406: return wave(dec_add_ln_wave_kernel<384, 6>);
-        case 38412: return wave(dec_add_ln_wave_kernel<384, 12>);
-        case 51208: return wave(dec_add_ln_wave_kernel<512, 8>);
-        case 51216: return wave(dec_add_ln_wave_kernel<512, 16>);
-        case 76808: return wave(dec_add_ln_wave_kernel<768, 8>);
-        case 76812: return wave(dec_add_ln_wave_kernel<768, 12>);
-        case 102408: return wave(dec_add_ln_wave_kernel<1024, 8>);
-        case 128005: return wave(dec_add_ln_wave_kernel<1280, 5>);
-    }
+    auto at = [&](auto width) {
+        constexpr int D = decltype(width)::value, P1 = mz_dec_ksplit(D, D), P2 = mz_dec_ksplit(D, 4 * D);
+        if (dim != D) return false;
+        if (nparts == P1) return wave(dec_add_ln_wave_kernel<D, P1>);
+        if (nparts == P2) return wave(dec_add_ln_wave_kernel<D, P2>);
+        return false;
+    };
+    if (at(std::integral_constant<int, 384>{}) || at(std::integral_constant<int, 512>{}) ||
+        at(std::integral_constant<int, 768>{}) || at(std::integral_constant<int, 1024>{}) ||
+        at(std::integral_constant<int, 1280>{}))
+        return hipGetLastError();
     hipLaunchKernelGGL(dec_add_ln_kernel, dim3(rows), dim3(row_threads(dim)), 0, s, xin, x, parts, nparts, part_stride,
                        bias, w, b, y, dim, eps);
     return hipGetLastError();

@@ -3,12 +3,13 @@
 // implicit GEMM (no im2col buffer), and the cross-attention K/V of every decoder layer. Replaces the reference's
 // cuBLAS calls with a bias prefill (src/gpu.rs:208-236, 254-286; kernels/whisper.cu:92-104, 106-139).
 //
-// Two kernels, chosen by how many tiles a product has (pick_plain, pick_conv): gemm_ring_kernel for few, described there, for the rest
-// gemm_kernel: block tile BM x BN x 64 with 8 waves in a 2 x 4 grid (two waves per SIMD, so one wave's LDS reads overlap the
-// other's products); each wave owns a (BM/2) x (BN/4) tile of 32x32x16 MFMA products. Both operands are
-// K-contiguous and go from global memory straight into LDS (buffer_load ... lds, 16 bytes per lane, no register
-// staging), double buffered: the loads of K tile k + 1 are in flight while tile k is multiplied, with one barrier per
-// K tile; the operand fragments are software pipelined a 16-wide K step ahead of the products. In LDS a tile row is 64 halves (128 bytes) whose 16-byte chunks are XOR-swizzled by the row index (chunk c
+// Two kernels, chosen by how many tiles a product has (pick_plain, pick_conv): gemm_ring_kernel for few, described
+// there, and for the rest gemm_kernel: block tile BM x BN x 64 with 8 waves in a 2 x 4 grid (two waves per SIMD, so one
+// wave's LDS reads overlap the other's products); each wave owns a (BM/2) x (BN/4) tile of 32x32x16 MFMA products. Both
+// operands are K-contiguous and go from global memory straight into LDS (buffer_load ... lds, 16 bytes per lane, no
+// register staging), double buffered: the loads of K tile k + 1 are in flight while tile k is multiplied, with one
+// barrier per K tile; the operand fragments are software pipelined a 16-wide K step ahead of the products. In LDS a
+// tile row is 64 halves (128 bytes) whose 16-byte chunks are XOR-swizzled by the row index (chunk c
 // of row r sits at position c ^ (r % 8) ^ (r / 8 % 2)): the 16 lanes that one ds_read_b128 cycle serves read 16
 // consecutive rows at one chunk, and these land in 16 distinct 16-byte bank groups of the 256-byte bank row; a
 // direct load writes lane i's 16 bytes at base + 16 i, so each lane fetches the global chunk that belongs at its
@@ -556,9 +557,9 @@ __global__ void __launch_bounds__(NWM * NWN * 64) gemm_ring_kernel(const MzGemm 
     if (kt < nk) tile(kt, s0, s1, f0, f1);
     if (kt + 1 < nk) tile(kt + 1, s1, s2, f1, f0);
     if (kt + 2 < nk) tile(kt + 2, s2, s3, f0, f1);
-    // no load may still be on its way into LDS when the workgroup ends, or when the v transposes are staged there
+    // no load may still be on its way into LDS when the workgroup ends, or when the v transposes are staged there (past
+    // the epilogue's barrier, so after this wait in every wave)
     __builtin_amdgcn_s_waitcnt(vm_lgkm_wait(0));
-    if (EPI == EPI_HEADS) asm volatile("s_barrier" ::: "memory");
     gemm_epilogue<BM, BN, NWM, NWN, EPI>(p, acc, bias_h, s0, m0, n0);
 #endif
 }

@@ -63,6 +63,19 @@ hipError_t mz_mel_transpose_launch(hipStream_t s, const float* mel, f16* melT, i
 #define MZ_MAX_PARTS 16  // split-K partials summed by dec_add_ln
 #define MZ_DEC_KSLICE 1280  // largest K slice of one skinny-GEMM workgroup (both operands resident in 160 KB of LDS)
 
+// K slices of the step's split-K products: until the grid covers most of the 256 CUs, with at most 16 groups of 64 per
+// workgroup (a slice within MZ_DEC_KSLICE, both operands resident in LDS) and at most MZ_MAX_PARTS partials
+constexpr int mz_dec_ksplit(int N, int K) {
+    const int tiles = (N + 31) / 32, groups = K / 64;
+    int best = 1;
+    for (int ks = 1; ks <= groups && ks <= MZ_MAX_PARTS; ks++) {
+        if (groups % ks) continue;
+        best = ks;
+        if (groups / ks <= 16 && (long)tiles * ks >= 192) break;
+    }
+    return best;
+}
+
 // skinny GEMM for decode batches: rows m < M of x (f16, row stride ldx % 8 == 0, M <= 32 per m-tile) times W[N][K];
 // K / ksplit <= MZ_DEC_KSLICE
 enum MzDecEpi {
