@@ -159,9 +159,10 @@ __global__ void __launch_bounds__(256) ts_stats4_kernel(const MzTs p) {
 // The same statistics for at most ST_R rows from LDS, one workgroup per (clip, head, 64 columns): the block's rows go
 // straight into LDS once (whole 256-byte row segments, every load in flight together), and the first wave takes both
 // passes from there, a column per lane, each column's sums in row order as above. Bound by reading the rows: the two
-// passes over memory of ts_stats4_kernel read a large batch's rows (275 MB for 32 clips x 220 rows x 10 heads, more than
-// stays in the memory-side cache) twice: 110 -> 86 us, one clip of 41 rows x 6 heads 6.8 -> 3.6. Two workgroups per CU, so
-// that one's sums run under the other's loads.
+// passes over memory of ts_stats4_kernel read a large batch's rows twice, and these are more than stays in the
+// memory-side cache (275 MB for 32 clips of up to 220 rows and 1500 columns, 6.88 million cells of 10 heads: 110 -> 86 us;
+// 32 of 220 x 1500, 422 MB, 113; one clip of 41 rows x 6 heads 6.8 -> 3.5). Two workgroups per CU, so that one's sums run
+// under the other's loads.
 constexpr int ST_R = 256;
 
 __global__ void __launch_bounds__(256) ts_stats_lds_kernel(const MzTs p) {
@@ -226,8 +227,9 @@ __global__ void __launch_bounds__(256) ts_stats_lds_kernel(const MzTs p) {
 // W = 7: median of the two outer triples and the middle value. With both triples sorted, it is the middle one of the larger
 // low, the middle of the three middles and the smaller high (the 3 x 3 rule for the median of nine, the third triple being
 // -inf, the middle value, +inf), and a triple serves two windows: 8.5 min / med3 / max per cell where a sorting network
-// took 48 compares and selects. W = 0: any odd width up to MZ_TS_MAX_WIDTH (insertion sort). 32 clips x 220 rows x 1500
-// columns x 10 heads: 285 -> 109 us, one clip of 41 rows x 6 heads 40 -> 13.
+// took 48 compares and selects. W = 0: any odd width up to MZ_TS_MAX_WIDTH (insertion sort). 32 clips of up to 220 rows
+// and 1500 columns, 6.88 million cells of 10 heads: 285 -> 109 us (32 of 220 x 1500: 145), one clip of 41 rows x 6 heads
+// 40 -> 13.
 constexpr int COST_RT = 32, COST_CT = 64, COST_HALO = MZ_TS_MAX_WIDTH - 1;
 
 template <int W>
@@ -488,8 +490,9 @@ __global__ void __launch_bounds__(1024) ts_dtw_kernel(const MzTs p) {
 // wave before) reaches wave w in chunks of 64 diagonals through LDS: wave w works one chunk behind wave w - 1, with one
 // barrier per chunk, and takes the chunk's values out of a register that shifts by a lane per step. The moves (a bit per
 // lane and kind) collect in two registers per 32 diagonals and go to LDS, where the path is walked back a run of equal
-// moves at a time. The time is the serial chain of about 20 instructions per diagonal: 32 clips of 220 rows and 1500
-// columns 466 -> 147 us, one of 41 rows 415 -> 93 (four rows per lane in one wave and a walk of one cell at a time before).
+// moves at a time. The time is the serial chain of about 20 instructions per diagonal, the longest clip's: 32 clips of up
+// to 220 rows and 1500 columns 466 -> 145 us (all of 220 x 1500: 149), one of 41 rows 415 -> 91 (four rows per lane in one
+// wave and a walk of one cell at a time before).
 // Same comparisons and results as ts_dtw_kernel, so the same bits.
 constexpr int DTW_CH = 64;   // diagonals per chunk
 constexpr int DTW_NCH = 28;  // chunks of a table: its diagonals 2 .. R + C are at most 1792 (256 rows x 1500 columns: 1755)

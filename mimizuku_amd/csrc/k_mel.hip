@@ -60,9 +60,10 @@ __global__ void __launch_bounds__(256) mel_basis_kernel(double* __restrict__ bas
 // Bound by the fp64 matrix cores: 104 products of 16 x 16 x 4 per wave and 16 frames (a wave holds one 16-bin tile of all
 // four parts, so a bin's real and imaginary sums meet in one lane), 64 cycles each. The left operands are made from
 // the samples by every wave for itself (12 fp64 instructions per 4 products), so LDS holds the samples only. M = 2
-// halves the basis' reads per frame (373 KB per workgroup, from L2); M = 1 is for few frames. 32 clips of 30 s: 254 us
-// (45% of the matrix cores' fp64 rate) for the transform, filters and logarithm that took 1386 + 381 us (one bin per
-// thread, multiply and add apart; one workgroup per frame with 12 KB strided stores); one of 7 s 154 + 30 -> 19 us.
+// halves the basis' reads per frame (373 KB per workgroup, from L2); M = 1 is for few frames. 32 clips of 18 to 30 s
+// (76,536 frames): 257 us, 35% of the matrix cores' fp64 rate (91 us of products), for the transform, filters and
+// logarithm that took 1386 + 381 us (one bin per thread, multiply and add apart; one workgroup per frame with 12 KB strided
+// stores); 32 of 30 s (96,000 frames) 297 us, 38%; one of 7 s 154 + 30 -> 19.
 template <int M>
 __global__ void __launch_bounds__(64 * NT) mel_spec_kernel(const MzMel p) {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -169,7 +170,7 @@ __global__ void __launch_bounds__(64 * NT) mel_spec_kernel(const MzMel p) {
 #endif
 }
 
-// Bound by its one read and write of the mel (98 MB for 32 clips of 128 mels: 16 us; one workgroup per clip took 237).
+// Bound by its one read and write of the mel (98 MB in all for 32 clips of 128 mels: 17 us; one workgroup per clip took 237).
 // V frames per thread (4: 16-byte accesses, for a 16-byte aligned mel; a row is 3000 frames)
 template <int V>
 __global__ void __launch_bounds__(256) mel_norm_kernel(const MzMel p, int fb) {
