@@ -601,9 +601,9 @@ long rounds(const MzGemm& g, int bm, int bn) { return (tile_count(g, bm, bn) + m
 // kernels before leave them), this rule / the one before it (256-row tiles from 200 on, two buffers): one clip, width
 // 1280, qkv 35 / 38 us, out-projection 12 / 18, fc1 36 / 54, fc2 30 / 55; 4 clips, width 512, 24 / 25, 9.5 / 10, 26 / 28,
 // 20 / 25; 5 to 8 clips, width 1280, within 1.5% but for fc2 at 5 (115 / 170). The largest is not always the fastest: launched
-// back to back, the choice is 1.5% from the fastest of six shapes on average over M = 1500 c (c = 1 .. 8) and the N, K of
-// widths 128 to 1280 (4% or more at 88 of 480, the worst 19%: M 10500, N 1152, K 384, 256 x 256 20.4 us, 256 x 128 17.4);
-// fitted to those times it was 0.7%, but slower in the encoder (fc2 at 4 clips, width 1280, 92 -> 103).
+// back to back, the choice is 1.8% from the fastest of six shapes on average over M = 1500 c (c = 1 .. 8) and the N, K of
+// widths 128 to 1280 (4% or more at 95 of 480, the worst 20%: M 12000, N 768, K 256, 256 x 256 15.4 us, 128 x 128 12.9);
+// fitted to those times it was 0.5%, but slower in the encoder (fc2 at 4 clips, width 1280, 92 -> 103).
 // Where a last column tile is partial, 256 x 128 may take no more rounds than 256 x 256 and has less to do in each: M 12000,
 // N 640, K 640 16.6 -> 12.9, M 6000, N 2688, K 896 46.6 -> 33.1.
 template <int EPI>
