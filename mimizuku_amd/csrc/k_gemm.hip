@@ -19,6 +19,7 @@
 // column l % 32 of eight rows: every store instruction writes two 32-column row segments. The transposed tiles of
 // the encoder's v are staged through LDS to be written as runs of token positions.
 #include <algorithm>
+#include <atomic>
 
 #include "mz_common.h"
 #include "mz_kernels.h"
@@ -640,15 +641,16 @@ hipError_t pick_conv(hipStream_t s, const MzGemm& g) {
 
 // compute units of the current device rounded down to a multiple of 8 (workgroups of a persistent grid: one per CU)
 int mz_cu_count() {
-    static int cached[64] = {};
+    static std::atomic<int> cached[64];  // (contexts of several threads ask)
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-    if (!cached[dev]) {
-        int n = 0;
+    int n = cached[dev].load(std::memory_order_relaxed);
+    if (!n) {
         if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n < 8) n = 256;
-        cached[dev] = n / 8 * 8;
+        n = n / 8 * 8;
+        cached[dev].store(n, std::memory_order_relaxed);
     }
-    return cached[dev];
+    return n;
 }
 
 hipError_t mz_gemm_launch(hipStream_t s, int aload, int epi, const MzGemm& g) {
